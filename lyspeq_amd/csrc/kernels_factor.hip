@@ -2,11 +2,11 @@
 // Li = L^-1 of every chunk of a batch (gfx950, FP64).
 //
 // Right-looking with 64x64 blocks (Np is a multiple of 64).  The L slot of
-// the matrix arena starts as a copy of A and is factorised in place.  Block
+// the matrix arena starts as a copy of A's lower blocks and is factorised in
+// place.  Block
 // column p takes three launches over the whole batch:
-//   diag   : one workgroup per chunk factors the updated block (p,p) in LDS,
-//            inverts it (Li[p,p] = L[p,p]^-1) and zeroes block row p right of
-//            the diagonal in L and Li;
+//   diag   : one workgroup per chunk factors the updated block (p,p) and
+//            inverts it (Li[p,p] = L[p,p]^-1);
 //   panel  : TRSM tiles L[i,p] = A[i,p] Li[p,p]^T for i > p, and the tiles of
 //            block row p of the inverse, Li[p,j] = -Li[p,p] sum_{k=j}^{p-1}
 //            L[p,k] Li[k,j] for j < p (rows k < p of Li are final by then);
@@ -163,14 +163,64 @@ __device__ __forceinline__ void block_nt(double *sa, double *sb, const double *M
     }
 }
 
+// The L slot starts as the lower block triangle of A (its blocks above the
+// diagonal are never read) and the Li slot with zeros above its diagonal
+// blocks, which the split products' conversion reads.
 __global__ __launch_bounds__(256) void k_chol_init(const ChunkDev *cs, double *mat) {
     const ChunkDev c = cs[blockIdx.y];
-    const size_t n = (size_t)c.Np * c.Np;
-    const double *A = mat + c.mat_off;
-    double *L = mat + c.mat_off + n;
-    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) L[e] = A[e];
+    const int Np = c.Np, h = Np / 2;
+    const size_t n = (size_t)Np * Np;
+    const dvec2 *A = (const dvec2 *)(mat + c.mat_off);
+    dvec2 *L = (dvec2 *)(mat + c.mat_off + n), *Li = (dvec2 *)(mat + c.mat_off + 2 * n);
+    const size_t total = n / 2, step = (size_t)gridDim.x * 256;
+    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < total; e += step) {
+        const int r = (int)(e / h), q = 2 * (int)(e % h);
+        if (q / FB <= r / FB) L[e] = A[e];
+        else Li[e] = dvec2{0.0, 0.0};
+    }
 }
 
+__device__ __forceinline__ double lane_of(double x, int lane) {
+    const long long u = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_readlane((int)u, lane), hi = __builtin_amdgcn_readlane((int)(u >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// x / s with rs ~ 1 / s: the quotient's residual folded back in once
+__device__ __forceinline__ double quotient(double x, double s, double rs) {
+    const double q = x * rs;
+    return fma(fma(-q, s, x), rs, q);
+}
+
+// s = sqrt(d) and rs = 1 / s for d > 0: the hardware's reciprocal root and
+// two Newton steps on it, then one on the root; out of the range where those
+// neither overflow nor lose bits, sqrt and a division.
+__device__ __forceinline__ void root_pair(double d, double &s, double &rs) {
+    if (d > 1e-280 && d < 1e280) {
+        double y = __builtin_amdgcn_rsq(d);
+        y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
+        y = fma(0.5 * y, fma(-d * y, y, 1.0), y);
+        s = d * y;
+        s = fma(0.5 * y, fma(-s, s, d), s);
+        rs = fma(y, fma(-s, y, 1.0), y);
+    } else {
+        s = sqrt(d);
+        rs = 1.0 / s;
+    }
+}
+
+// Factors the updated diagonal block, L[p,p], and inverts it, Li[p,p], in
+// 16-column panels.  The 64 pivots are one dependent chain, so the kernel's
+// time is that chain's latency: a panel is factored by one wave with a row
+// per lane and the panel's 16 columns in registers, where a column costs a
+// reciprocal root and register broadcasts instead of three barriers and two
+// trips through LDS; the trailing 16 x 16 blocks are updated on the matrix
+// cores, one block a wave.  The inverse takes the four 16 x 16 diagonal
+// blocks by forward substitution, a wave each, then
+// Li[i,j] = -Li[i,i] sum_k L[i,k] Li[k,j] by block subdiagonals.
+// LDS: strictly below the diagonal L, from the diagonal up Li^T (33 KB).
+// 25 us a launch at 1 to 128 chunks; column by column in LDS it took 141.
+constexpr int PB = 16;   // panel width
 __global__ __launch_bounds__(256) void k_chol_diag(const ChunkDev *cs, double *mat, int *status, int p) {
     const ChunkDev c = cs[blockIdx.x];
     const int Np = c.Np, tid = threadIdx.x, p0 = p * FB;
@@ -178,50 +228,104 @@ __global__ __launch_bounds__(256) void k_chol_diag(const ChunkDev *cs, double *m
     double *L = mat + c.mat_off + (size_t)Np * Np;
     double *Li = mat + c.mat_off + 2 * (size_t)Np * Np;
     __shared__ double a[FB * FLD];
-    __shared__ double v[FB * FLD];
-    __shared__ int fail;
-    if (tid == 0) fail = 0;
+    __shared__ double sd[FB], sr[FB];   // L's diagonal and its reciprocals
+    const int w = tid / 64, l = tid % 64, lr = l % 16, lq = l / 16;
     load_block(a, L, Np, p0, p0, false);
-    for (int e = tid; e < FB * FB; e += 256) v[(e / FB) * FLD + e % FB] = (e / FB == e % FB) ? 1.0 : 0.0;
     __syncthreads();
-    // unblocked right-looking factorisation of the 64x64 block; alongside it,
-    // V = L^-1 by forward elimination of the identity: at step k row k of V
-    // (complete by then) is divided by L_kk, and every row i > k takes off
-    // L_ik times it
-    for (int k = 0; k < FB; ++k) {
-        if (tid == 0) {
-            const double d = a[k * FLD + k];
-            if (!(d > 0.0)) fail = 1;
-            a[k * FLD + k] = (d > 0.0) ? sqrt(d) : 1.0;
+    int fail = 0;
+#pragma unroll 1
+    for (int kb = 0; kb < FB; kb += PB) {
+        if (w == 0) {
+            const int row = kb + l;
+            double x[PB];
+#pragma unroll
+            for (int j = 0; j < PB; ++j) x[j] = (row < FB) ? a[row * FLD + kb + j] : 0.0;
+#pragma unroll
+            for (int k = 0; k < PB; ++k) {
+                const double d = lane_of(x[k], k);
+                double s = 1.0, rs = 1.0;
+                if (d > 0.0) root_pair(d, s, rs);
+                else fail = 1;
+                const double q = quotient(x[k], s, rs);
+                if (l == k) { sd[row] = s; sr[row] = rs; }
+                x[k] = (l > k) ? q : 0.0;
+#pragma unroll
+                for (int j = k + 1; j < PB; ++j) x[j] = fma(-x[k], lane_of(x[k], j), x[j]);
+            }
+            if (row < FB) {
+#pragma unroll
+                for (int j = 0; j < PB; ++j)
+                    if (l > j) a[row * FLD + kb + j] = x[j];
+            }
         }
         __syncthreads();
-        const double dkk = a[k * FLD + k];
-        if (tid > k && tid < FB) a[tid * FLD + k] /= dkk;
-        if (tid >= FB && tid - FB <= k) v[k * FLD + tid - FB] /= dkk;
-        __syncthreads();
-        for (int e = tid; e < FB * FB; e += 256) {
-            const int i = e / FB, j = e % FB;
-            if (i > k) {
-                if (j > k && j <= i) a[i * FLD + j] -= a[i * FLD + k] * a[j * FLD + k];
-                else if (j <= k) v[i * FLD + j] -= a[i * FLD + k] * v[k * FLD + j];
+        // trailing blocks (i, j), kb/16 < j <= i < 4: A -= L[i,kb] L[j,kb]^T
+        const int b0 = kb / PB + 1;
+        int t = 0;
+        for (int i = b0; i < FB / PB; ++i)
+            for (int j = b0; j <= i; ++j, ++t) {
+                if ((t & 3) != w) continue;
+                fd4 acc;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc[u] = a[(PB * i + 4 * u + lq) * FLD + PB * j + lr];
+#pragma unroll
+                for (int k = 0; k < PB; k += 4)
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[(PB * i + lr) * FLD + kb + k + lq],
+                                                               a[(PB * j + lr) * FLD + kb + k + lq], acc, 0, 0, 0);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) a[(PB * i + 4 * u + lq) * FLD + PB * j + lr] = acc[u];
             }
+        __syncthreads();
+    }
+    for (int e = tid; e < FB * FB; e += 256) {
+        const int i = e / FB, j = e % FB;
+        L[(size_t)(p0 + i) * Np + p0 + j] = (j < i) ? a[i * FLD + j] : (j == i) ? sd[i] : 0.0;
+    }
+    __syncthreads();   // the upper part now takes Li^T
+    // diagonal block w: lane lr solves column lr of its inverse
+    if (l < PB) {
+        double x[PB];
+#pragma unroll
+        for (int i = 0; i < PB; ++i) {
+            double s = (i == lr) ? 1.0 : 0.0;
+#pragma unroll
+            for (int k = 0; k < i; ++k) s = fma(-a[(PB * w + i) * FLD + PB * w + k], x[k], s);
+            x[i] = (i >= lr) ? quotient(s, sd[PB * w + i], sr[PB * w + i]) : 0.0;
+        }
+#pragma unroll
+        for (int i = 0; i < PB; ++i)
+            if (i >= lr) a[(PB * w + lr) * FLD + PB * w + i] = x[i];
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int t = 1; t < FB / PB; ++t) {   // block subdiagonal t, block (i, i - t) by wave i - t
+        const int j = w, i = w + t;
+        if (i < FB / PB) {
+            fd4 s = {0.0, 0.0, 0.0, 0.0}, x = {0.0, 0.0, 0.0, 0.0};
+            for (int k = j; k < i; ++k)
+#pragma unroll
+                for (int q = 0; q < PB; q += 4) {
+                    const int r = q + lq;   // Li[k,j](r, lr), zero above its diagonal
+                    const double b = (k > j || r >= lr) ? a[(PB * j + lr) * FLD + PB * k + r] : 0.0;
+                    s = __builtin_amdgcn_mfma_f64_16x16x4f64(a[(PB * i + lr) * FLD + PB * k + r], b, s, 0, 0, 0);
+                }
+            // element u of s holds row 4 u + lane / 16: the B operand of step u
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int r = 4 * q + lq;
+                const double v = (lr >= r) ? -a[(PB * i + r) * FLD + PB * i + lr] : 0.0;
+                x = __builtin_amdgcn_mfma_f64_16x16x4f64(v, s[q], x, 0, 0, 0);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a[(PB * j + lr) * FLD + PB * i + 4 * u + lq] = x[u];
         }
         __syncthreads();
     }
     for (int e = tid; e < FB * FB; e += 256) {
         const int i = e / FB, j = e % FB;
-        const size_t o = (size_t)(p0 + i) * Np + p0 + j;
-        L[o] = (j <= i) ? a[i * FLD + j] : 0.0;
-        Li[o] = v[i * FLD + j];
+        Li[(size_t)(p0 + i) * Np + p0 + j] = (j <= i) ? a[j * FLD + i] : 0.0;
     }
-    // block row p right of the diagonal is zero in L and Li
-    const int wr = Np - p0 - FB;
-    for (size_t e = tid; e < (size_t)FB * wr; e += 256) {
-        const size_t o = (size_t)(p0 + e / wr) * Np + p0 + FB + e % wr;
-        L[o] = 0.0;
-        Li[o] = 0.0;
-    }
-    if (tid == 0) {
+    if (tid == 0) {   // wave 0 saw every pivot
         if (p == 0) status[c.gidx] = fail;
         else if (fail) status[c.gidx] = 1;
     }
