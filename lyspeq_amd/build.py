@@ -13,7 +13,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libqmlhip.so")
 
-SOURCES = ["kernels_chunk.hip", "kernels_factor.hip", "kernels_gemm.hip", "kernels_rmat.hip", "kernels_tables.hip",
+SOURCES = ["kernels_chunk.hip", "kernels_factor.hip", "kernels_gemm.hip", "kernels_gemm64.hip", "kernels_rmat.hip", "kernels_tables.hip",
            "kernels_boot.hip", "qml_api.cpp",
            "rmat_prep.cpp"]
 

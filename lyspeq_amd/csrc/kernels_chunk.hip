@@ -530,9 +530,10 @@ __global__ __launch_bounds__(256) void k_small(const ChunkDev *cs, const double 
 template <class OutT> struct XStore4;
 template <> struct XStore4<double> {
     static __device__ __forceinline__ void put(double *X, size_t msz, int j, size_t off, const double *v) {
+        // streaming stores, as for the split form below
         double *p = X + j * msz + off;
-        *(double2 *)p = double2{v[0], v[1]};
-        *(double2 *)(p + 2) = double2{v[2], v[3]};
+        __builtin_nontemporal_store(dvec2{v[0], v[1]}, (dvec2 *)p);
+        __builtin_nontemporal_store(dvec2{v[2], v[3]}, (dvec2 *)(p + 2));
     }
 };
 template <> struct XStore4<float> {
@@ -559,10 +560,11 @@ template <> struct XStore4<__bf16> {
 
 // X_j = D (Q_j - U At_j^T - At_j U^T) D for every member, in the compute
 // type, with arithmetic in CT (FP64 for the FP64 path, FP32 otherwise).
-// The split form stores T = M^T instead, M the lower triangle of X_j with
-// its diagonal halved (X_j = M + M^T): element (i, b) is X_j[i,b] above the
-// diagonal, half of it on the diagonal and zero below; 128-blocks strictly
-// below the diagonal are not written at all (the products never read them).
+// FP64 and the split form store T = M^T instead, M the lower triangle of X_j
+// with its diagonal halved (X_j = M + M^T): element (i, b) is X_j[i,b] above
+// the diagonal, half of it on the diagonal and zero below; the products'
+// tiles (64 wide in FP64, 128 in the split form) strictly below the diagonal
+// are not written at all (the products never read them).
 //
 // A workgroup covers 16 EPT rows x 64 columns (EPT = 2 in FP32, 1 in
 // FP64); thread t owns the four consecutive columns 4(t%16).. and rows
@@ -585,11 +587,13 @@ __global__ __launch_bounds__(256, OCC) void k_xgen(const ChunkDev *cs, const dou
     constexpr int TR = 16 * EPT, TC = 64;
     constexpr int SL = (sizeof(CT) == 4) ? 2048 : 1024;        // slice buffer
     constexpr int NSL = 4, NAT = 4;   // prefetch registers: slice values, At values
-    constexpr bool UPPER = std::is_same<OutT, __bf16>::value;   // the T form
+    constexpr bool BLK = std::is_same<OutT, __bf16>::value;    // blocked layout
+    constexpr bool UPPER = !std::is_same<OutT, float>::value;   // the T form
+    constexpr int TSH = BLK ? 7 : 6;                            // log2 of the products' tile
     const ChunkDev c = cs[blockIdx.z];
     const int i0 = blockIdx.y * TR, b0 = blockIdx.x * TC;
     if (i0 >= c.Np || b0 >= c.Np) return;
-    if (UPPER && (b0 >> 7) < (i0 >> 7)) return;
+    if (UPPER && (b0 >> TSH) < (i0 >> TSH)) return;
     const int Np = c.Np, N = c.N, nu = c.nu, tid = threadIdx.x, nzq = c.nzq, kbu = c.kbu;
     const int cg = tid % 16, rl = tid / 16;
     const int bb = b0 + 4 * cg;            // first of the thread's columns
@@ -611,7 +615,7 @@ __global__ __launch_bounds__(256, OCC) void k_xgen(const ChunkDev *cs, const dou
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
         const int i = i0 + rl + 16 * e;
-        xoff[e] = UPPER ? (size_t)bf3_tiled(i, bb, Np) : (size_t)i * Np + bb;
+        xoff[e] = BLK ? (size_t)bf3_tiled(i, bb, Np) : (size_t)i * Np + bb;
     }
 
     // pair geometry

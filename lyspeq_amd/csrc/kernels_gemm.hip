@@ -1,4 +1,5 @@
-// Dense MFMA products of the QML engine (gfx950).
+// Dense MFMA products of the QML engine in FP32 and split BF16 (gfx950); the
+// FP64 ones are in kernels_gemm64.hip.
 //
 //   whiten_left :  Y_j = Li X_j              (Li lower triangular: K-range of
 //                                             tile row I is [0, 64 (I+1)); X_j is
@@ -13,11 +14,9 @@
 //   gram        :  E_s = sum_{k in G tile s} G_j[k] G_j'[k]   (split-K partials,
 //                                             x2 for off-diagonal G tiles)
 //
-// FP64 and FP32 (k_gemm): one 256-thread workgroup computes a 64x64 output
-// tile; each of its four waves owns a 32x32 quarter made of 2x2 16x16 MFMA
-// blocks:
-//   FP64   v_mfma_f64_16x16x4f64, FP64 operands and accumulation;
-//   FP32   v_mfma_f32_16x16x4f32, FP32 operands and accumulation.
+// FP32 (k_gemm): one 256-thread workgroup computes a 64x64 output tile; each
+// of its four waves owns a 32x32 quarter made of 2x2 16x16 MFMA blocks on
+// v_mfma_f32_16x16x4f32, FP32 operands and accumulation.
 // Split BF16 (k_gemm_bf3): 128x128 output tiles on operands stored as two
 // bf16 planes (hi, lo), v_mfma_f32_16x16x32_bf16 with FP32 accumulation:
 //   BF16x3 a b ~ a_hi b_hi + a_hi b_lo + a_lo b_hi;
@@ -54,70 +53,38 @@ __device__ __forceinline__ int xcd_logical(int nwork) {
 }
 
 // Problem description of one work item.
-template <class T>
 struct Prob {
-    const T *A;  // row-major, rows of the output tile, K contiguous (lda)
-    const T *B;  // NN: row-major K x N (ldb);  NT: row-major N x K (ldb)
+    const float *A;  // row-major, rows of the output tile, K contiguous (lda)
+    const float *B;  // row-major N x K (ldb)
     int lda, ldb;
     int kbeg, kend;
     int arows, brows;   // valid rows of A / B^T (members for the Gram); others read as 0
-    bool nt;
 };
 
-// ------------------------------------------------------ FP64 / FP32 path --
-template <class T> struct MF;
-template <> struct MF<double> {
-    using acc_t = d4;
-    static __device__ __forceinline__ acc_t mfma(double a, double b, acc_t c) {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-};
-template <> struct MF<float> {
-    using acc_t = f4;
-    static __device__ __forceinline__ acc_t mfma(float a, float b, acc_t c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-};
-
-template <class T>
-__device__ __forceinline__ void mainloop_k4(const Prob<T> &p, int I0, int J0,
-                                            typename MF<T>::acc_t (&acc)[2][2]) {
+// --------------------------------------------------------------- FP32 path --
+__device__ __forceinline__ void mainloop_k4(const Prob &p, int I0, int J0, f4 (&acc)[2][2]) {
     constexpr int KB = 16, PAD = 4;
-    __shared__ T As[KB][64 + PAD];
-    __shared__ T Bs[KB][64 + PAD];
+    __shared__ float As[KB][64 + PAD];
+    __shared__ float Bs[KB][64 + PAD];
     const int tid = threadIdx.x, lane = tid % 64, w = tid / 64;
     const int wm = w / 2, wn = w % 2;
-    // A pattern: row tid/4, four consecutive k at (tid%4)*4
+    // row tid/4, four consecutive k at (tid%4)*4
     const int ar = tid / 4, ak = (tid % 4) * 4;
-    // NN pattern for B: k row tid/16, four consecutive n at (tid%16)*4
-    const int bk = tid / 16, bn = (tid % 16) * 4;
-    T ra[4], rb[4];
+    float ra[4], rb[4];
     auto gload = [&](int k0) {
-        const bool aok = (I0 + ar) < p.arows;
-        const T *pa = p.A + (size_t)(I0 + ar) * p.lda + k0 + ak;
+        const bool aok = (I0 + ar) < p.arows, bok = (J0 + ar) < p.brows;
+        const float *pa = p.A + (size_t)(I0 + ar) * p.lda + k0 + ak;
+        const float *pb = p.B + (size_t)(J0 + ar) * p.ldb + k0 + ak;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) ra[u] = aok ? pa[u] : (T)0;
-        if (p.nt) {
-            const bool bok = (J0 + ar) < p.brows;
-            const T *pb = p.B + (size_t)(J0 + ar) * p.ldb + k0 + ak;
+        for (int u = 0; u < 4; ++u) ra[u] = aok ? pa[u] : 0.0f;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) rb[u] = bok ? pb[u] : (T)0;
-        } else {
-            const T *pb = p.B + (size_t)(k0 + bk) * p.ldb + J0 + bn;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) rb[u] = pb[u];
-        }
+        for (int u = 0; u < 4; ++u) rb[u] = bok ? pb[u] : 0.0f;
     };
     auto sstore = [&]() {
 #pragma unroll
         for (int u = 0; u < 4; ++u) As[ak + u][ar] = ra[u];
-        if (p.nt) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) Bs[ak + u][ar] = rb[u];
-        } else {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) Bs[bk][bn + u] = rb[u];
-        }
+        for (int u = 0; u < 4; ++u) Bs[ak + u][ar] = rb[u];
     };
     if (p.kbeg >= p.kend) return;
     gload(p.kbeg);
@@ -128,7 +95,7 @@ __device__ __forceinline__ void mainloop_k4(const Prob<T> &p, int I0, int J0,
         if (more) gload(k0 + KB);
 #pragma unroll
         for (int kk = 0; kk < KB; kk += 4) {
-            T a[2], b[2];
+            float a[2], b[2];
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 a[q] = As[kk + lane / 16][wm * 32 + q * 16 + lane % 16];
@@ -137,7 +104,8 @@ __device__ __forceinline__ void mainloop_k4(const Prob<T> &p, int I0, int J0,
 #pragma unroll
             for (int x = 0; x < 2; ++x)
 #pragma unroll
-                for (int y = 0; y < 2; ++y) acc[x][y] = MF<T>::mfma(a[x], b[y], acc[x][y]);
+                for (int y = 0; y < 2; ++y)
+                    acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], b[y], acc[x][y], 0, 0, 0);
         }
         __syncthreads();
         if (more) sstore();
@@ -146,18 +114,17 @@ __device__ __forceinline__ void mainloop_k4(const Prob<T> &p, int I0, int J0,
 }
 
 // ------------------------------------------------------------------ kernel --
-template <int PREC, int MODE>
+template <int MODE>
 __global__ __launch_bounds__(256) void k_gemm(const ChunkDev *cs, const Work *work, int nwork,
                                               const void *Abase, const void *Bbase, void *Cbase, int jlo) {
-    using T = typename std::conditional<PREC == 0, double, float>::type;
-    using acc_t = typename std::conditional<PREC == 0, d4, f4>::type;
+    using T = float;
     const int li = xcd_logical(nwork);
     if (li >= nwork) return;
     const Work wk = work[li];
     const ChunkDev c = cs[wk.c];
     const int Np = c.Np;
     const size_t msz = (size_t)Np * Np;
-    Prob<T> p;
+    Prob p;
     int I0, J0;
     if (MODE == MODE_LEFT) {
         p.A = (const T *)Abase + c.lic_off;
@@ -167,7 +134,6 @@ __global__ __launch_bounds__(256) void k_gemm(const ChunkDev *cs, const Work *wo
         p.kbeg = 0;
         p.kend = (wk.I + 1) * TILE;
         p.arows = p.brows = Np;
-        p.nt = (PREC != 0);
         I0 = wk.I * TILE;
         J0 = wk.J * TILE;
     } else if (MODE == MODE_RIGHT) {
@@ -177,7 +143,6 @@ __global__ __launch_bounds__(256) void k_gemm(const ChunkDev *cs, const Work *wo
         p.kbeg = 0;
         p.kend = (wk.J + 1) * TILE;
         p.arows = p.brows = Np;
-        p.nt = true;
         I0 = wk.I * TILE;
         J0 = wk.J * TILE;
     } else {
@@ -188,24 +153,22 @@ __global__ __launch_bounds__(256) void k_gemm(const ChunkDev *cs, const Work *wo
         p.kbeg = wk.j * TILE * TILE;
         p.kend = p.kbeg + TILE * TILE;
         p.arows = p.brows = c.m;
-        p.nt = true;
         I0 = wk.I * TILE;
         J0 = wk.J * TILE;
     }
-    acc_t acc[2][2];
+    f4 acc[2][2];
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y)
 #pragma unroll
             for (int u = 0; u < 4; ++u) acc[x][y][u] = 0;
-    mainloop_k4<T>(p, I0, J0, acc);
+    mainloop_k4(p, I0, J0, acc);
 
     const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
     const int wm = w / 2, wn = w % 2;
-    // row of accumulator element u inside a 16x16 block: the FP64 MFMA
-    // holds rows u*4 + lane/16, the FP32-output MFMAs rows 4*(lane/16) + u
-    auto brow = [&](int u) { return (PREC == 0) ? (4 * u + lane / 16) : (4 * (lane / 16) + u); };
+    // row of accumulator element u inside a 16x16 block
+    auto brow = [&](int u) { return 4 * (lane / 16) + u; };
     if (MODE == MODE_LEFT) {
         T *C = (T *)Cbase + c.stk_off + (wk.j - jlo) * msz;
 #pragma unroll
@@ -261,22 +224,31 @@ static void launch_mode(hipStream_t st, int prec, int nst, const ChunkDev *chunk
         return;
     }
     const int grid = 8 * ((nwork + 7) / 8);
-    if (prec == 0)
-        k_gemm<0, MODE><<<grid, 256, 0, st>>>(chunks, work, nwork, A, B, C, jlo);
-    else
-        k_gemm<1, MODE><<<grid, 256, 0, st>>>(chunks, work, nwork, A, B, C, jlo);
+    k_gemm<MODE><<<grid, 256, 0, st>>>(chunks, work, nwork, A, B, C, jlo);
 }
 
 void launch_gemm_whiten_left(hipStream_t st, int prec, int nst, const ChunkDev *chunks, const Work *work,
                              int nwork, const void *li, const void *X, void *Y, int jlo) {
+    if (prec == 0) {
+        if (nwork > 0) launch_gemm64_left(st, chunks, work, nwork, (const double *)li, (const double *)X, (double *)Y, jlo);
+        return;
+    }
     launch_mode<MODE_LEFT>(st, prec, nst, chunks, work, nwork, li, X, Y, jlo);
 }
 void launch_gemm_whiten_right(hipStream_t st, int prec, int nst, const ChunkDev *chunks, const Work *work,
                               int nwork, const void *li, const void *Y, void *G, int jlo) {
+    if (prec == 0) {
+        if (nwork > 0) launch_gemm64_right(st, chunks, work, nwork, (const double *)li, (const double *)Y, (double *)G, jlo);
+        return;
+    }
     launch_mode<MODE_RIGHT>(st, prec, nst, chunks, work, nwork, Y, li, G, jlo);
 }
 void launch_gemm_gram(hipStream_t st, int prec, int nst, const ChunkDev *chunks, const Work *work, int nwork,
                       const void *G, double *gram) {
+    if (prec == 0) {
+        if (nwork > 0) launch_gram64(st, chunks, work, nwork, (const double *)G, gram);
+        return;
+    }
     launch_mode<MODE_GRAM>(st, prec, nst, chunks, work, nwork, G, G, gram, 0);
 }
 

@@ -782,8 +782,8 @@ int plan_batches(qml_ctx *c) {
             if (!rmat_layout_ok(B.rm_lay)) return fail(QML_ERR_LIMIT, "qml_commit: no sandwich kernel for the resolution matrices");
         }
         // Output tiles of the whitening products: 64x64 for FP64 and FP32,
-        // 128x128 for split BF16, whose left product P = Li M is lower
-        // triangular (J <= I only).  The lists run slab by slab (one slab of
+        // 128x128 for split BF16.  The left product P = Li M of FP64 and split
+        // BF16 is lower triangular (J <= I only).  The lists run slab by slab (one slab of
         // every member without slabbing), chunk by chunk within a slab.
         {
             int mmax = 0;
@@ -805,7 +805,7 @@ int plan_batches(qml_ctx *c) {
                     // order does not change any result
                     for (int j0 = ja; j0 < jb; j0 += 4)
                         for (int I = 0; I < nt; ++I)
-                            for (int J = 0; J < ((c->prec >= 2) ? I + 1 : nt); ++J)
+                            for (int J = 0; J < ((c->prec != 1) ? I + 1 : nt); ++J)
                                 for (int j = j0; j < std::min(jb, j0 + 4); ++j) wl.push_back({li, j, I, J});
                     for (int j = ja; j < jb; ++j)
                         for (int I = 0; I < nt; ++I)

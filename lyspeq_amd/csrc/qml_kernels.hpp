@@ -89,6 +89,15 @@ void launch_gemm_whiten_right(hipStream_t st, int prec, int nst, const ChunkDev 
 void launch_gemm_gram(hipStream_t st, int prec, int nst, const ChunkDev *chunks, const Work *work, int nwork,
                       const void *G, double *gram);
 
+// kernels_gemm64.hip: the FP64 products (the work lists hold the lower tiles
+// for the left product, the upper ones for the right).
+void launch_gemm64_left(hipStream_t st, const ChunkDev *chunks, const Work *work, int nwork, const double *li,
+                        const double *X, double *Y, int jlo);
+void launch_gemm64_right(hipStream_t st, const ChunkDev *chunks, const Work *work, int nwork, const double *li,
+                         const double *Y, double *G, int jlo);
+void launch_gram64(hipStream_t st, const ChunkDev *chunks, const Work *work, int nwork, const double *G,
+                   double *gram);
+
 // kernels_boot.hip: FastBootstrap realisations, their mean and covariance.
 // qptr/qchunk: CSR list of each spectrum's chunk ids (nqso + 1 offsets); P is
 // nqso x nboots Poisson weights; theta nqso x T and R nboots x T scratch.
