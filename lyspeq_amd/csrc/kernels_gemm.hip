@@ -121,6 +121,7 @@ __global__ __launch_bounds__(256) void k_gemm(const ChunkDev *cs, const Work *wo
     const int li = xcd_logical(nwork);
     if (li >= nwork) return;
     const Work wk = work[li];
+    if (wk.c < 0) return;
     const ChunkDev c = cs[wk.c];
     const int Np = c.Np;
     const size_t msz = (size_t)Np * Np;
@@ -478,6 +479,7 @@ void k_gemm_bf3(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *A
     const int li = xcd_logical(nwork);
     if (li >= nwork) return;
     const Work wk = work[li];
+    if (wk.c < 0) return;
     const ChunkDev c = cs[wk.c];
     const int I0 = wk.I * BM, J0 = wk.J * BN;
     const Bf3Item it = bf3_item<MODE>(c, wk, jlo, Abase, Bbase);
@@ -704,6 +706,7 @@ void k_gemm_bf3d(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *
     const int li = xcd_logical(nwork);
     if (li >= nwork) return;
     const Work wk = work[li];
+    if (wk.c < 0) return;
     const ChunkDev c = cs[wk.c];
     const int I0 = wk.I * BF3_BM, J0 = wk.J * BF3_BN;
     const Bf3Item it = bf3_item<MODE>(c, wk, jlo, Abase, Bbase);

@@ -56,6 +56,7 @@ __global__ __launch_bounds__(256, 4) void k_gemm64(const ChunkDev *cs, const Wor
     const int li = xcd_item(nwork);
     if (li >= nwork) return;
     const Work wk = work[li];
+    if (wk.c < 0) return;
     const ChunkDev c = cs[wk.c];
     const int Np = c.Np, N = c.N, I0 = wk.I * TILE, J0 = wk.J * TILE;
     const size_t mem = (size_t)c.stk_off + (size_t)(wk.j - jlo) * Np * Np;
@@ -186,6 +187,7 @@ __global__ __launch_bounds__(64 * GW, 2) void k_gram64(const ChunkDev *cs, const
     const int li = xcd_item(nwork);
     if (li >= nwork) return;
     const Work wk = work[li];
+    if (wk.c < 0) return;
     const ChunkDev c = cs[wk.c];
     constexpr int KW = TILE * TILE / GW;   // terms per wave
     __shared__ double red[2][GW][256];

@@ -129,6 +129,34 @@ void jacobi_svd(std::vector<double> &V, int N, int nt, std::vector<double> &sv) 
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+// One launch's work items, dealt to the eight XCDs.  A product's workgroup b
+// runs on XCD b % 8 and takes item (b % 8) per + b / 8 of the list, so the
+// list is eight runs of equal length (the short ones end in empty items).
+// Each chunk's members (or Gram splits) are cut into eight even ranges, one
+// per XCD, the range rotating with the chunk so that the remainders even out:
+// chunks differ in the length of their sums (K grows with N), so whole chunks
+// to an XCD, as consecutive eighths of a list sorted by size, left the XCDs
+// of the smaller chunks idle.  Li is then read by every XCD of the batch,
+// which is little next to a chunk's hundred members.
+struct XcdLists {
+    std::vector<Work> q[8];
+    // bounds of XCD x's share of [lo, hi) for the chunk at place li
+    static void share(int lo, int hi, int x, int li, int &a, int &b) {
+        const int r = (x + li) % 8, n = hi - lo;
+        a = lo + n * r / 8;
+        b = lo + n * (r + 1) / 8;
+    }
+    void flush(std::vector<Work> &out) {
+        size_t per = 0;
+        for (const auto &v : q) per = std::max(per, v.size());
+        for (auto &v : q) {
+            v.resize(per, Work{-1, 0, 0, 0});
+            out.insert(out.end(), v.begin(), v.end());
+            v.clear();
+        }
+    }
+};
+
 }  // namespace
 
 struct qml_ctx {
@@ -751,6 +779,7 @@ int plan_batches(qml_ctx *c) {
         B.ids = groups[bi];
         const auto &cd = devs[bi];
         std::vector<Work> wl, wr, wg;
+        XcdLists xl, xr, xg;
         int ra_max = 0, rb_max = 0, nb_max = 0;
         for (int li = 0; li < (int)cd.size(); ++li) {
             const ChunkDev &d = cd[li];
@@ -768,10 +797,15 @@ int plan_batches(qml_ctx *c) {
             }
             const int g = (c->prec >= 2) ? 2 : 1;
             const int mtg = (d.mt + g - 1) / g;
-            for (int s = 0; s < d.ntu; ++s)
-                for (int I = 0; I < mtg; ++I)
-                    for (int J = I; J < mtg; ++J) wg.push_back({li, s, I, J});
+            for (int x = 0; x < 8; ++x) {
+                int sa, sb;
+                XcdLists::share(0, d.ntu, x, li, sa, sb);
+                for (int s = sa; s < sb; ++s)
+                    for (int I = 0; I < mtg; ++I)
+                        for (int J = I; J < mtg; ++J) xg.q[x].push_back({li, s, I, J});
+            }
         }
+        xg.flush(wg);
         if (B.rm_kbu >= 0) {
             // 16 x 32 output tiles where their LDS fits in 64 KB, their a range
             // in 80 rows and their b range in 4 passes; else 16 x 16 (which
@@ -797,20 +831,25 @@ int plan_batches(qml_ctx *c) {
                 for (int li = 0; li < (int)cd.size(); ++li) {
                     const ChunkDev &d = cd[li];
                     const int nt = (d.nt + g - 1) / g;
-                    const int ja = sb * S, jb = std::min(d.m, (sb + 1) * S);
-                    // the left product's tiles go four members at a time, tile by
-                    // tile, so that the workgroups in flight on an XCD share Li
-                    // rows across members (5 % faster than member by member on
-                    // DESI-like batches); every tile is computed alone, so the
-                    // order does not change any result
-                    for (int j0 = ja; j0 < jb; j0 += 4)
-                        for (int I = 0; I < nt; ++I)
-                            for (int J = 0; J < ((c->prec != 1) ? I + 1 : nt); ++J)
-                                for (int j = j0; j < std::min(jb, j0 + 4); ++j) wl.push_back({li, j, I, J});
-                    for (int j = ja; j < jb; ++j)
-                        for (int I = 0; I < nt; ++I)
-                            for (int J = I; J < nt; ++J) wr.push_back({li, j, I, J});
+                    for (int x = 0; x < 8; ++x) {
+                        int ja, jb;
+                        XcdLists::share(sb * S, std::max(sb * S, std::min(d.m, (sb + 1) * S)), x, li, ja, jb);
+                        // the left product's tiles go four members at a time, tile by
+                        // tile, so that the workgroups in flight on an XCD share Li
+                        // rows across members (5 % faster than member by member on
+                        // DESI-like batches); every tile is computed alone, so the
+                        // order does not change any result
+                        for (int j0 = ja; j0 < jb; j0 += 4)
+                            for (int I = 0; I < nt; ++I)
+                                for (int J = 0; J < ((c->prec != 1) ? I + 1 : nt); ++J)
+                                    for (int j = j0; j < std::min(jb, j0 + 4); ++j) xl.q[x].push_back({li, j, I, J});
+                        for (int j = ja; j < jb; ++j)
+                            for (int I = 0; I < nt; ++I)
+                                for (int J = I; J < nt; ++J) xr.q[x].push_back({li, j, I, J});
+                    }
                 }
+                xl.flush(wl);
+                xr.flush(wr);
                 B.sl_off.push_back((int)wl.size());
                 B.sr_off.push_back((int)wr.size());
             }

@@ -100,7 +100,8 @@ struct ChunkOut {        // per chunk id, persistent
     int nq, fis;
 };
 
-// GEMM work item: (local chunk, member or split, tile row, tile col)
+// GEMM work item: (local chunk, member or split, tile row, tile col); c < 0
+// is no work (the lists are padded to eight runs of equal length, one per XCD)
 struct Work {
     int c, j, I, J;
 };
