@@ -562,9 +562,8 @@ template <> struct XStore4<__bf16> {
 // type, with arithmetic in CT (FP64 for the FP64 path, FP32 otherwise).
 // FP64 and the split form store T = M^T instead, M the lower triangle of X_j
 // with its diagonal halved (X_j = M + M^T): element (i, b) is X_j[i,b] above
-// the diagonal, half of it on the diagonal and zero below; the products'
-// tiles (64 wide in FP64, 128 in the split form) strictly below the diagonal
-// are not written at all (the products never read them).
+// the diagonal, half of it on the diagonal and zero below; 64-blocks strictly
+// below the diagonal are not written at all (the products never multiply them).
 //
 // A workgroup covers 16 EPT rows x 64 columns (EPT = 2 in FP32, 1 in
 // FP64); thread t owns the four consecutive columns 4(t%16).. and rows
@@ -589,11 +588,10 @@ __global__ __launch_bounds__(256, OCC) void k_xgen(const ChunkDev *cs, const dou
     constexpr int NSL = 4, NAT = 4;   // prefetch registers: slice values, At values
     constexpr bool BLK = std::is_same<OutT, __bf16>::value;    // blocked layout
     constexpr bool UPPER = !std::is_same<OutT, float>::value;   // the T form
-    constexpr int TSH = BLK ? 7 : 6;                            // log2 of the products' tile
     const ChunkDev c = cs[blockIdx.z];
     const int i0 = blockIdx.y * TR, b0 = blockIdx.x * TC;
     if (i0 >= c.Np || b0 >= c.Np) return;
-    if (UPPER && (b0 >> TSH) < (i0 >> TSH)) return;
+    if (UPPER && (b0 >> 6) < (i0 >> 6)) return;
     const int Np = c.Np, N = c.N, nu = c.nu, tid = threadIdx.x, nzq = c.nzq, kbu = c.kbu;
     const int cg = tid % 16, rl = tid / 16;
     const int bb = b0 + 4 * cg;            // first of the thread's columns

@@ -27,7 +27,7 @@
 #include "qml_common.hpp"
 #include "qml_kernels.hpp"
 
-#include <climits>
+#include <type_traits>
 
 namespace qml {
 
@@ -300,6 +300,15 @@ constexpr int BF3_PL = BF3_BM * BK;   // elements per LDS plane
 constexpr int BF3_STG = 4 * BF3_PL;   // elements per stage: A hi, A lo, B hi, B lo
 constexpr int BF3_EP = 72;            // row pitch of the staged epilogue block, in bf16
 
+// First row (column) of tile row (column) I of a whitening product.  Where Np
+// is an odd number of 64-blocks the half tile comes first, not last: tile row 0
+// then starts 64 rows before the matrix.  The sums of a row tile run to its
+// last row, so a half tile costs the right product half its waves over 64 terms
+// there and over all of Np at the end (13 % of the steps over N ~ U[150, 700]).
+__device__ __forceinline__ int bf3_origin(int I, int Np) { return I * 128 - ((Np & 64) ? 64 : 0); }
+// a byte in the global address space
+typedef const char __attribute__((address_space(1))) GlobalB;
+
 // Operands and K range of one work item (tile I, J of member or split j).
 struct Bf3Item {
     const __bf16 *Ahi, *Bhi;   // hi planes; the lo planes follow at alo / blo elements
@@ -313,7 +322,7 @@ __device__ __forceinline__ Bf3Item bf3_item(const ChunkDev &c, const Work &wk, i
     Bf3Item t;
     const int Np = c.Np;
     const long long msz = (long long)Np * Np;
-    const int I0 = wk.I * BF3_BM, J0 = wk.J * BF3_BN;
+    const int I0 = bf3_origin(wk.I, Np), J0 = bf3_origin(wk.J, Np);
     t.kbeg = 0;
     if (MODE == MODE_LEFT) {
         // P = Li M, lower tiles (J <= I): Li[i,k] needs k <= i and the stored
@@ -323,7 +332,7 @@ __device__ __forceinline__ Bf3Item bf3_item(const ChunkDev &c, const Work &wk, i
         t.lda = t.ldb = Np;
         t.alo = t.blo = msz;
         t.arows = t.brows = Np;
-        t.kbeg = J0;
+        t.kbeg = max(0, J0);
         t.kend = min(Np, I0 + BF3_BM);
         t.Mv = t.Nv = Np;
     } else if (MODE == MODE_RIGHT) {
@@ -356,20 +365,39 @@ __device__ __forceinline__ Bf3Item bf3_item(const ChunkDev &c, const Work &wk, i
     return t;
 }
 
-// One BK step of a wave's 64x64 quarter out of LDS stage s0: fragment row
-// offsets aoff / boff (rows 16x + lane%16 of the wave's slab, chunk lane/16).
+// The K steps [tlo, thi) of a term that a wave multiplies: those whose products
+// are not exact zeros.  Li[i][k] = 0 for k > i, the stored T[n][k] = 0 for k < n
+// and P is lower triangular, so LEFT (rows i of Li, rows n of T) needs k in
+// [c0, r0 + 64), and RIGHT (P or Li rows i in both terms) k < r0 + 64.  Past the
+// chunk's N pixels (D = 0) T, P and G vanish, so k < N and a wave whose rows or
+// columns all lie past N multiplies nothing.  The accumulators start at +0 and
+// no sum of exact zeros changes them, so the results are those of the full
+// sweep, bit for bit; and what is never multiplied need not be written: T's
+// 64-blocks below the diagonal and P's above it are not.
+template <int MODE>
+__device__ __forceinline__ void bf3_steps(const ChunkDev &c, bool active, int r0, int c0, int kbeg, int kend, int &tlo,
+                                          int &thi) {
+    const int kn32 = (c.N + BK - 1) / BK * BK;
+    const bool pad = MODE != MODE_GRAM && (r0 >= c.N || c0 >= c.N);
+    tlo = (MODE == MODE_LEFT) ? max(0, (c0 - kbeg) / BK) : 0;
+    thi = (!active || pad) ? 0 : (MODE == MODE_GRAM) ? (kend - kbeg) / BK : (min(r0 + 64, kn32) - kbeg) / BK;
+}
+
+// One BK step of a wave's 64x64 quarter out of LDS, the hi planes of A and B
+// at sa and sb and their lo planes behind them: fragment row offsets aoff /
+// boff (rows 16x + lane%16 of the wave's slab, chunk lane/16).
 template <int NPROD>
-__device__ __forceinline__ void bf3_mfma(const __bf16 *s0, int aoff, int boff, f4 (&acc)[4][4]) {
+__device__ __forceinline__ void bf3_mfma(const __bf16 *sa, const __bf16 *sb, int aoff, int boff, f4 (&acc)[4][4]) {
     bf8 bh[4], bl[4];
 #pragma unroll
     for (int y = 0; y < 4; ++y) {
-        bh[y] = *(const bf8 *)(s0 + 2 * BF3_PL + boff + y * 16 * BK);
-        bl[y] = *(const bf8 *)(s0 + 3 * BF3_PL + boff + y * 16 * BK);
+        bh[y] = *(const bf8 *)(sb + boff + y * 16 * BK);
+        bl[y] = *(const bf8 *)(sb + BF3_PL + boff + y * 16 * BK);
     }
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
-        const bf8 ah = *(const bf8 *)(s0 + aoff + x * 16 * BK);
-        const bf8 al = *(const bf8 *)(s0 + BF3_PL + aoff + x * 16 * BK);
+        const bf8 ah = *(const bf8 *)(sa + aoff + x * 16 * BK);
+        const bf8 al = *(const bf8 *)(sa + BF3_PL + aoff + x * 16 * BK);
 #pragma unroll
         for (int y = 0; y < 4; ++y) {
             if constexpr (NPROD == 4)
@@ -481,7 +509,8 @@ void k_gemm_bf3(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *A
     const Work wk = work[li];
     if (wk.c < 0) return;
     const ChunkDev c = cs[wk.c];
-    const int I0 = wk.I * BM, J0 = wk.J * BN;
+    const int I0 = (MODE == MODE_GRAM) ? wk.I * BM : bf3_origin(wk.I, c.Np);
+    const int J0 = (MODE == MODE_GRAM) ? wk.J * BN : bf3_origin(wk.J, c.Np);
     const Bf3Item it = bf3_item<MODE>(c, wk, jlo, Abase, Bbase);
     const __bf16 *Ahi = it.Ahi, *Bhi = it.Bhi;
     const long long lda = it.lda, ldb = it.ldb, alo = it.alo, blo = it.blo;
@@ -491,8 +520,12 @@ void k_gemm_bf3(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *A
     const int tid = threadIdx.x, lane = tid % 64, w = tid / 64;
     const int wm = w / 2, wn = w % 2;
     const int r0 = I0 + 64 * wm, c0 = J0 + 64 * wn;
-    bool active = (r0 < Mv) && (c0 < Nv);
-    if (MODE != MODE_LEFT) active = active && (c0 >= r0);
+    bool active = r0 >= 0 && c0 >= 0 && r0 < Mv && c0 < Nv;
+    active = active && (MODE == MODE_LEFT ? c0 <= r0 : c0 >= r0);
+    // steps of a term that the wave multiplies (bf3_steps)
+    int tlo, thi;
+    bf3_steps<MODE>(c, active, r0, c0, kbeg, kend, tlo, thi);
+    const auto on = [&](int st) { return st >= tlo && st < thi; };
     f4 acc[4][4];
 #pragma unroll
     for (int x = 0; x < 4; ++x)
@@ -506,8 +539,8 @@ void k_gemm_bf3(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *A
     // therefore unconditional (no exec branches).
     static_assert(PA >= 1 && PA <= 2 && PB >= 1 && PB <= 2, "staging passes");
     const int lr = tid / 4, lc = tid % 4;
-    const auto arow = [&](int q) { const int r = I0 + lr + RP * q; return r < arows ? r : 0; };
-    const auto brow = [&](int q) { const int r = J0 + lr + RP * q; return r < brows ? r : 0; };
+    const auto arow = [&](int q) { const int r = I0 + lr + RP * q; return r >= 0 && r < arows ? r : 0; };
+    const auto brow = [&](int q) { const int r = J0 + lr + RP * q; return r >= 0 && r < brows ? r : 0; };
     // per-thread element offsets of the staged rows; the operand bases are
     // workgroup-uniform.  The whitening products' offsets stay below Np^2
     // (32 bits); the Gram's rows are whole members of 2 ntu TILE^2 elements,
@@ -561,7 +594,7 @@ void k_gemm_bf3(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *A
             *(uint4 *)(s0 + 2 * PLA + PLB + wb1) = R##rbl1;                      \
         }                                                                        \
     }
-#define QML_BF3_MFMA(st) bf3_mfma<NPROD>(smem + (st) * STG, aoff, boff, acc);
+#define QML_BF3_MFMA(st) bf3_mfma<NPROD>(smem + (st) * STG, smem + (st) * STG + 2 * BF3_PL, aoff, boff, acc);
 // One K sweep over n = (kend - kbeg)/BK stages, two steps per pass: the
 // loads of stage s+2 are issued (into the register set just stored), stage
 // s is multiplied out of LDS, and stage s+1 (loaded a whole step earlier)
@@ -579,16 +612,16 @@ void k_gemm_bf3(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *A
         for (; s + 1 < ns; s += 2) {                                          \
             const int k0 = kbeg + s * BK;                                     \
             QML_BF3_GLOAD(P, min(k0 + 2 * BK, klast))                         \
-            if (DO_MFMA) QML_BF3_MFMA(0)                                      \
+            if (DO_MFMA && on(s)) QML_BF3_MFMA(0)                             \
             QML_BF3_SSTORE(Q, 1)                                              \
             __syncthreads();                                                  \
             QML_BF3_GLOAD(Q, min(k0 + 3 * BK, klast))                         \
-            if (DO_MFMA) QML_BF3_MFMA(1)                                      \
+            if (DO_MFMA && on(s + 1)) QML_BF3_MFMA(1)                         \
             if (s + 2 < ns) QML_BF3_SSTORE(P, 0)                              \
             __syncthreads();                                                  \
         }                                                                     \
         if (s < ns) {                                                         \
-            if (DO_MFMA) QML_BF3_MFMA(0)                                      \
+            if (DO_MFMA && on(s)) QML_BF3_MFMA(0)                             \
             __syncthreads();                                                  \
         }                                                                     \
     }
@@ -604,12 +637,12 @@ void k_gemm_bf3(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *A
         __syncthreads();                                                      \
         for (int s = 0; s + 1 < ns; ++s) {                                    \
             QML_BF3_GLOAD(P, kbeg + (s + 1) * BK)                             \
-            if (DO_MFMA) QML_BF3_MFMA(0)                                      \
+            if (DO_MFMA && on(s)) QML_BF3_MFMA(0)                             \
             __syncthreads();                                                  \
             QML_BF3_SSTORE(P, 0)                                              \
             __syncthreads();                                                  \
         }                                                                     \
-        if (DO_MFMA) QML_BF3_MFMA(0)                                          \
+        if (DO_MFMA && on(ns - 1)) QML_BF3_MFMA(0)                            \
         __syncthreads();                                                      \
     }
 #define QML_BF3_RUN                                                           \
@@ -635,12 +668,12 @@ void k_gemm_bf3(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *A
             const bool second = sn >= ns;                                     \
             const __bf16 *xa = second ? Bhi : Ahi, *xb = second ? Ahi : Bhi;  \
             QML_BF3_GLOADX(P, xa, xb, kbeg + (second ? sn - ns : sn) * BK)    \
-            if (DO_MFMA) QML_BF3_MFMA(0)                                      \
+            if (DO_MFMA && on(s < ns ? s : s - ns)) QML_BF3_MFMA(0)           \
             __syncthreads();                                                  \
             QML_BF3_SSTORE(P, 0)                                              \
             __syncthreads();                                                  \
         }                                                                     \
-        if (DO_MFMA) QML_BF3_MFMA(0)                                          \
+        if (DO_MFMA && on(ns - 1)) QML_BF3_MFMA(0)                            \
         __syncthreads();                                                      \
     }
     if (kbeg < kend) {
@@ -669,121 +702,142 @@ void k_gemm_bf3(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *A
 // same results, bit for bit), with the operands staged by
 // global_load_lds_dwordx4: each load moves 16 bytes per lane from global
 // memory straight into LDS at (M0 base) + 16 x lane, with no register
-// round trip, so NS stages can be in flight at once without registers held
-// for them.  Wave w fills plane w of a stage (A hi, A lo, B hi, B lo), eight
-// 16-row blocks of 1 KB.  For the whitening products a block is stored in
-// slot order (bf3_tiled), so lane i loads the block's 16 bytes at 16 i; for
-// the Gram lane i loads row i/4 of the block at the chunk that the swizzle
-// places in slot i, (i%4) ^ bf3_swz(i/4).  Rows past the operand read row
-// 0, as in k_gemm_bf3.
+// round trip, so several steps can be in flight at once without registers
+// held for them.  Each operand has its own ring of slots (16 KB: its hi and lo
+// planes, 128 rows of 32): NM for the member's (the stack T, or P; the Gram's
+// rows I), NL for Li (the Gram's rows J).  Each wave loads four 1 KB blocks of
+// 16 rows of either operand per step.  For the whitening products a block is
+// stored in slot order (bf3_tiled), so lane i loads the block's 16 bytes at
+// 16 i; for the Gram lane i loads row i/4 of the block at the chunk that the
+// swizzle places in slot i, (i%4) ^ bf3_swz(i/4).  Rows outside the operand
+// read row 0, as in k_gemm_bf3.
 //
-// Step s waits for its own stage (s_waitcnt vmcnt counting the stages issued
-// after it), passes one barrier, issues stage s + NS - 1 into the buffer
-// that step s - 1 read (every wave is past that step), then multiplies
-// stage s.  The barrier is the bare s_barrier (no memory fence, which would
-// wait for every load in flight), with compiler-level memory clobbers so
-// that no LDS access moves across it.  NS = 2: two workgroups per CU (64 KB
-// of LDS each); NS = 3: one (96 KB).
-template <int NS>
-__device__ __forceinline__ void bf3_wait_stage(bool last) {
-    // s_waitcnt: vmcnt <= 8 (NS - 2) (the later stages' loads, eight per
-    // wave each), or 0 on the last step; lgkmcnt 0; expcnt not waited on.
-    // Encoding: vmcnt[3:0] and [15:14], expcnt[6:4], lgkmcnt[11:8].
-    constexpr int V = 8 * (NS - 2);
-    constexpr int ENC = (V & 15) | (7 << 4) | ((V >> 4) << 14);
-    if (NS == 2 || last) __builtin_amdgcn_s_waitcnt(7 << 4);
+// Step s waits for its own blocks (s_waitcnt vmcnt counting what was issued
+// after them), passes one barrier, issues Li's step s + NL - 1 and the
+// member's s + NM - 1 into the slots that step s - 1 read (every wave is past
+// that step), then multiplies step s.  The barrier is the bare s_barrier (no
+// memory fence, which would wait for every load in flight), with compiler-level
+// memory clobbers so that no LDS access moves across it.
+//
+// The whitening products take (NM, NL) = (3, 2): the member's panels come from
+// HBM and have two steps to arrive, Li's from L2 one, and two workgroups of
+// 80 KB fill a CU.  (2, 2) took 6 % longer for the left product and 3 % for the
+// right; the Gram, whose operands are the same rows, is 4 % faster with (2, 2).
+// What bounds the products is the traffic past L2, not the steps' structure:
+// on 640 chunks of 150-700 pixels the left moves 86 GB at 4.4 TB/s (a copy runs
+// at 4.4 to 5.3), the right 109 GB at 3.5, P about 1.7 times over.  Reading
+// the next step's fragments a step ahead, or running a workgroup through up to
+// eight items without a break, changed nothing (the latter cost locality: 24
+// echelle chunks 18.6 -> 22.9 ms).  (3, 3): one workgroup of 96 KB, 1.7 x
+// slower.
+template <int PENDING>
+__device__ __forceinline__ void bf3_wait_step(bool last) {
+    // s_waitcnt: vmcnt <= PENDING, or 0 on the last step; lgkmcnt 0; expcnt not
+    // waited on.  Encoding: vmcnt[3:0] and [15:14], expcnt[6:4], lgkmcnt[11:8].
+    constexpr int ENC = (PENDING & 15) | (7 << 4) | ((PENDING >> 4) << 14);
+    if (PENDING == 0 || last) __builtin_amdgcn_s_waitcnt(7 << 4);
     else __builtin_amdgcn_s_waitcnt(ENC);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
 
-template <int MODE, int NS, int NPROD>
-__global__ __launch_bounds__(256, NS == 2 ? 2 : 1)
+template <int MODE, int NM, int NL, int NPROD>
+__global__ __launch_bounds__(256, NM + NL < 6 ? 2 : 1)
 void k_gemm_bf3d(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *Abase, const __bf16 *Bbase,
                  void *Cbase, int jlo) {
-    static_assert(NS == 2 || NS == 3, "two or three stages");
+    static_assert(NM >= NL && NL >= 2 && NM <= 3, "two or three slots");
     const int li = xcd_logical(nwork);
     if (li >= nwork) return;
     const Work wk = work[li];
     if (wk.c < 0) return;
     const ChunkDev c = cs[wk.c];
-    const int I0 = wk.I * BF3_BM, J0 = wk.J * BF3_BN;
+    const int I0 = (MODE == MODE_GRAM) ? wk.I * BF3_BM : bf3_origin(wk.I, c.Np);
+    const int J0 = (MODE == MODE_GRAM) ? wk.J * BF3_BN : bf3_origin(wk.J, c.Np);
     const Bf3Item it = bf3_item<MODE>(c, wk, jlo, Abase, Bbase);
-    constexpr int SMEM = (NS * BF3_STG > 4 * 64 * BF3_EP) ? NS * BF3_STG : 4 * 64 * BF3_EP;
+    constexpr int SLOT = 2 * BF3_PL;   // elements
+    constexpr int SMEM = ((NM + NL) * SLOT > 4 * 64 * BF3_EP) ? (NM + NL) * SLOT : 4 * 64 * BF3_EP;
     __shared__ __attribute__((aligned(1024))) __bf16 smem[SMEM];
     const int tid = threadIdx.x, lane = tid % 64;
     const int w = __builtin_amdgcn_readfirstlane(tid / 64);
     const int wm = w / 2, wn = w % 2;
     const int r0 = I0 + 64 * wm, c0 = J0 + 64 * wn;
-    bool active = (r0 < it.Mv) && (c0 < it.Nv);
-    if (MODE != MODE_LEFT) active = active && (c0 >= r0);
+    const bool active = r0 >= 0 && c0 >= 0 && r0 < it.Mv && c0 < it.Nv && (MODE == MODE_LEFT ? c0 <= r0 : c0 >= r0);
     f4 acc[4][4];
 #pragma unroll
     for (int x = 0; x < 4; ++x)
 #pragma unroll
         for (int y = 0; y < 4; ++y) acc[x][y] = f4{0.f, 0.f, 0.f, 0.f};
-    // this wave's plane: A (w < 2) or B rows, hi (w even) or lo
-    const bool pa = w < 2;
-    const int prow0 = pa ? I0 : J0, prows = pa ? it.arows : it.brows;
-    const long long pld = pa ? it.lda : it.ldb, plo = (w & 1) ? (pa ? it.alo : it.blo) : 0;
-    using off_t = typename std::conditional<MODE == MODE_GRAM, long long, int>::type;
+    // the member's operand is B of the left product and A of the others; the
+    // right product's second term exchanges the roles
+    constexpr bool mb = MODE == MODE_LEFT;
+    const __bf16 *Mhi = mb ? it.Bhi : it.Ahi, *Lhi = mb ? it.Ahi : it.Bhi;
+    // byte offsets of the lanes from a uniform base: the whitening products'
+    // planes fit 32 bits (Np <= 16384), the Gram's rows do not
+    using off_t = typename std::conditional<MODE == MODE_GRAM, long long, unsigned>::type;
     const int rl = lane / 4;
     const int ch = (lane % 4) ^ bf3_swz(rl);
-    // blocked layout: the 16 rows of a block lie all inside the operand or
-    // all past it (Np is a multiple of 64), and lane i reads slot i of the
-    // block; K step k (a multiple of 32) adds 16 k
-    off_t roff[8];
+    // this wave's blocks of a slot: plane w / 2 (hi, lo), rows 64 (w % 2) + 16 b;
+    // blocked layout: the 16 rows of a block lie all inside the operand or all
+    // outside it (Np is a multiple of 64), and lane i reads slot i of the block
+    const auto offset = [&](int row0, int b, int rows, long long ld, long long lo) -> off_t {
+        const int rb = row0 + 64 * (w % 2) + 16 * b, r = rb + rl;
+        const bool in = r >= 0 && r < rows;
+        const off_t plane = (off_t)((w / 2) ? lo : 0);
+        if constexpr (MODE == MODE_GRAM) return 2 * ((off_t)(in ? r : 0) * (off_t)ld + plane + 8 * ch);
+        else return 2 * ((off_t)bf3_tiled(in ? rb : 0, 0, (int)ld) + plane + 8 * lane);
+    };
+    // by row panel (I0 or J0); the right product stages both panels of both
+    // operands, which share their layout
+    off_t oi[4], oj[4];
 #pragma unroll
-    for (int b = 0; b < 8; ++b) {
-        const int r = prow0 + 16 * b + rl;
-        if constexpr (MODE == MODE_GRAM) roff[b] = (off_t)(r < prows ? r : 0) * (off_t)pld + (off_t)plo + 8 * ch;
-        else roff[b] = (off_t)bf3_tiled(r < prows ? prow0 + 16 * b : 0, 0, (int)pld) + (off_t)plo + 8 * lane;
+    for (int b = 0; b < 4; ++b) {
+        oi[b] = offset(I0, b, it.arows, it.lda, it.alo);
+        oj[b] = offset(J0, b, it.brows, it.ldb, it.blo);
     }
-    constexpr int KSC = (MODE == MODE_GRAM) ? 1 : 16;
+    constexpr int STEP = 2 * BK * (MODE == MODE_GRAM ? 1 : 16);   // bytes from step to step
     const int kbeg = it.kbeg;
     const int ns = (it.kend - kbeg) / BK;
     const int total = (MODE == MODE_RIGHT) ? 2 * ns : ns;
-    // stage s: operands (the right product's second term swaps them) and k
-    const auto issue = [&](int s) {
-        const bool second = MODE == MODE_RIGHT && s >= ns;
-        const __bf16 *x = (pa != second) ? it.Ahi : it.Bhi;
-        const int k = kbeg + (second ? s - ns : s) * BK;
-        __bf16 *dst = smem + (s % NS) * BF3_STG + w * BF3_PL;
+    GlobalB *const m0 = (GlobalB *)Mhi + (size_t)kbeg * (STEP / BK), *const l0 = (GlobalB *)Lhi + (size_t)kbeg * (STEP / BK);
+    const int dst0 = (w / 2) * BF3_PL + (w % 2) * 64 * BK;
+    const auto issue = [&](GlobalB *x, bool rows_i, int s, int slot) {
+        x += (size_t)((MODE == MODE_RIGHT && s >= ns) ? s - ns : s) * STEP;
+        __bf16 *dst = smem + slot * SLOT + dst0;
 #pragma unroll
-        for (int b = 0; b < 8; ++b)
-            __builtin_amdgcn_global_load_lds((const void *)(x + roff[b] + KSC * k),
-                                             (__attribute__((address_space(3))) void *)(dst + b * 16 * BK), 16, 0, 0);
+        for (int b = 0; b < 4; ++b)
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void *)(x + (rows_i ? oi[b] : oj[b])),
+                (__attribute__((address_space(3))) void *)(dst + b * 16 * BK), 16, 0, 0);
     };
+    const auto issue_m = [&](int s, int slot) { issue(m0, mb ? false : !(MODE == MODE_RIGHT && s >= ns), s, slot); };
+    const auto issue_l = [&](int s, int slot) { issue(l0, mb ? true : (MODE == MODE_RIGHT && s >= ns), s, NM + slot); };
     const int rr = lane % 16, cq = lane / 16;
     const int aoff = bf3_slot(64 * wm + rr, cq), boff = bf3_slot(64 * wn + rr, cq);
-    // K steps whose products are exact zeros for this wave are not
-    // multiplied: Li[i][k] = 0 for k > i, the stored T[n][k] = 0 for k < n,
-    // and P is lower triangular.  LEFT (rows i of Li, rows n of T) needs k in
-    // [c0, r0 + 64); RIGHT (P or Li rows i in both terms) k < r0 + 64.  Past
-    // the chunk's N pixels (D = 0) T, P and G vanish, so k < N and a wave
-    // whose rows or columns all lie past N multiplies nothing.  The
-    // accumulators start at +0 and no sum of exact zeros changes them, so the
-    // results are those of the full sweep, bit for bit.
-    const int kn32 = (c.N + BK - 1) / BK * BK;
-    const bool pad = MODE != MODE_GRAM && (r0 >= c.N || c0 >= c.N);
-    const int klo = (MODE == MODE_LEFT) ? c0 : INT_MIN;
-    const int khi = (MODE == MODE_GRAM) ? INT_MAX : pad ? INT_MIN : min(r0 + 64, kn32);
+    int tlo, thi;
+    bf3_steps<MODE>(c, active, r0, c0, kbeg, it.kend, tlo, thi);
     if (total > 0) {
-#pragma unroll
-        for (int s = 0; s < NS - 1; ++s)
-            if (s < total) issue(s);
+        issue_m(0, 0);
+        issue_l(0, 0);
+        if (NL == 3 && total > 1) issue_l(1, 1);
+        if (NM == 3 && total > 1) issue_m(1, 1);
+        int sm = 0, sl = 0;   // the slots of step s
         for (int s = 0; s < total; ++s) {
-            bf3_wait_stage<NS>(s + NS - 2 >= total);
-            if (s + NS - 1 < total) issue(s + NS - 1);
-            const int kk = kbeg + ((MODE == MODE_RIGHT && s >= ns) ? s - ns : s) * BK;
-            if (active && kk + BK > klo && kk < khi) bf3_mfma<NPROD>(smem + (s % NS) * BF3_STG, aoff, boff, acc);
+            bf3_wait_step<4 * (NM + NL - 4)>(s + 1 >= total);
+            const int pm = sm == 0 ? NM - 1 : sm - 1, pl = sl == 0 ? NL - 1 : sl - 1;   // step s - 1's
+            if (s + NL - 1 < total) issue_l(s + NL - 1, pl);
+            if (s + NM - 1 < total) issue_m(s + NM - 1, pm);
+            const bool second = MODE == MODE_RIGHT && s >= ns;
+            const int k = second ? s - ns : s;
+            if (k >= tlo && k < thi) {
+                const __bf16 *m = smem + sm * SLOT, *l = smem + (NM + sl) * SLOT;
+                bf3_mfma<NPROD>((mb || second) ? l : m, (mb || second) ? m : l, aoff, boff, acc);
+            }
+            sm = sm + 1 == NM ? 0 : sm + 1;
+            sl = sl + 1 == NL ? 0 : sl + 1;
         }
-        // every wave is done with the stages before the epilogue reuses LDS
-        __builtin_amdgcn_s_waitcnt(7 << 4);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        // every wave is done with the slots before the epilogue reuses LDS
+        bf3_wait_step<0>(true);
     }
     if (!active) return;
     bf3_epilogue<MODE>(acc, c, wk, jlo, r0, c0, Cbase, smem + w * 64 * BF3_EP, lane);
@@ -797,23 +851,24 @@ static void launch_bf3_np(hipStream_t st, int mode, int nst, const ChunkDev *chu
     // per CU, the next stage in registers); 2 two LDS stages (two workgroups
     // per CU, a second register set two stages ahead; not for the right
     // product, whose two-term sweep uses 1 instead); 3 and 4 direct-to-LDS
-    // loads with two (two workgroups per CU) and three (one) stages.  Each
+    // loads with two stages (three of the member's operand in the whitening
+    // products; two workgroups per CU) and three (one).  Each
     // output sums its K steps in the same order either way, so the results
     // are identical.
 #define QML_BF3_LAUNCH(M, N) k_gemm_bf3<M, N, NPROD><<<grid, 256, 0, st>>>(chunks, work, nwork, a, b, C, jlo)
-#define QML_BF3D_LAUNCH(M, N) k_gemm_bf3d<M, N, NPROD><<<grid, 256, 0, st>>>(chunks, work, nwork, a, b, C, jlo)
+#define QML_BF3D_LAUNCH(M, N, K) k_gemm_bf3d<M, N, K, NPROD><<<grid, 256, 0, st>>>(chunks, work, nwork, a, b, C, jlo)
     if (mode == MODE_LEFT) {
-        if (nst == 4) QML_BF3D_LAUNCH(MODE_LEFT, 3);
-        else if (nst == 3) QML_BF3D_LAUNCH(MODE_LEFT, 2);
+        if (nst == 4) QML_BF3D_LAUNCH(MODE_LEFT, 3, 3);
+        else if (nst == 3) QML_BF3D_LAUNCH(MODE_LEFT, 3, 2);
         else if (nst == 2) QML_BF3_LAUNCH(MODE_LEFT, 2);
         else QML_BF3_LAUNCH(MODE_LEFT, 1);
     } else if (mode == MODE_RIGHT) {
-        if (nst == 4) QML_BF3D_LAUNCH(MODE_RIGHT, 3);
-        else if (nst == 3) QML_BF3D_LAUNCH(MODE_RIGHT, 2);
+        if (nst == 4) QML_BF3D_LAUNCH(MODE_RIGHT, 3, 3);
+        else if (nst == 3) QML_BF3D_LAUNCH(MODE_RIGHT, 3, 2);
         else QML_BF3_LAUNCH(MODE_RIGHT, 1);
     } else {
-        if (nst == 4) QML_BF3D_LAUNCH(MODE_GRAM, 3);
-        else if (nst == 3) QML_BF3D_LAUNCH(MODE_GRAM, 2);
+        if (nst == 4) QML_BF3D_LAUNCH(MODE_GRAM, 3, 3);
+        else if (nst == 3) QML_BF3D_LAUNCH(MODE_GRAM, 2, 2);
         else if (nst == 1) QML_BF3_LAUNCH(MODE_GRAM, 1);
         else QML_BF3_LAUNCH(MODE_GRAM, 2);
     }
