@@ -150,117 +150,197 @@ __global__ __launch_bounds__(256) void k_boot_cov(const double *R, const double 
 // zeroed).
 
 // Each spectrum's collapsed Fisher matrix (OneQSOEstimate::collapseBootstrap,
-// core/one_qso_estimate.cpp:224-234): the upper triangle of ndim x ndim at
-// fq_off[q], summed over its chunks in chunk order.  One block per spectrum.
+// core/one_qso_estimate.cpp:224-234): ndim x ndim at fq_off[q], summed over its
+// chunks in chunk order, the lower triangle (element (r, c), c <= r, is the
+// chunks' (c, r)), so that k_boot_build reads along c.  A block takes 32 rows r
+// of one spectrum; each 32 x 32 tile is read along r and turned in LDS.
 __global__ __launch_bounds__(256) void k_boot_collapse_fisher(const ChunkOut *outs, const double *fc,
                                                               const int *qptr, const int *qchunk,
                                                               const int *qstart, const int *qdim,
                                                               const long long *fq_off, double *fq) {
-    const int q = blockIdx.x;
+    __shared__ double tile[32][33];
+    const int q = blockIdx.x, r0 = blockIdx.y * 32;
     const int c0 = qptr[q], c1 = qptr[q + 1], is = qstart[q], nd = qdim[q];
+    if (r0 >= nd) return;
     double *F = fq + fq_off[q];
-    for (int e = threadIdx.x; e < nd * nd; e += blockDim.x) {
-        const int i = e / nd, j = e - i * nd;
-        double acc = 0.0;
-        if (j >= i) {
-            for (int k = c0; k < c1; ++k) {
-                const ChunkOut o = outs[qchunk[k]];
-                const int a = i + is - o.fis, b = j + is - o.fis;
-                if (a < 0 || b >= o.nq) continue;   // a <= b
-                acc += fc[o.fc_off + (size_t)a * o.nq + b];
-            }
-        }
-        F[e] = acc;
-    }
-}
-
-// F_b (full symmetric, Np x Np with identity padding, empty diagonals set to
-// 1) at mat + b * 3 Np^2 and the right-hand side at rhs + b * Np, for the
-// realisations b0 .. b0 + nb - 1 of the batch.  Grid (Np / 64, Np / 64, nb),
-// upper tiles only.  Element (i, j), j >= i, sums over the spectra covering
-// band i (band_q[band_ptr[i] ..], in queue order) that also cover j.
-__global__ __launch_bounds__(256) void k_boot_build(const int *W, int nqso, int b0, int T, int Np,
-                                                    const int *band_ptr, const int *band_q, const int *qstart,
-                                                    const int *qdim, const long long *fq_off, const double *fq,
-                                                    const double *theta, double *mat, double *rhs) {
-    const int I = blockIdx.y, J = blockIdx.x, b = blockIdx.z;
-    if (J < I) return;
-    const int *w = W + (size_t)(b0 + b) * nqso;
-    double *A = mat + (size_t)b * 3 * Np * Np;
-    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-        const int i = I * 64 + e / 64, j = J * 64 + e % 64;
-        if (j < i) continue;
-        double acc = 0.0;
-        if (i < T && j < T) {
-            for (int k = band_ptr[i]; k < band_ptr[i + 1]; ++k) {
-                const int q = band_q[k];
-                const int p = w[q];
-                const int is = qstart[q];
-                if (p == 0 || j >= is + qdim[q]) continue;
-                acc += (double)p * fq[fq_off[q] + (size_t)(i - is) * qdim[q] + (j - is)];
-            }
-            if (i == j && acc == 0.0) acc = 1.0;
-        } else if (i == j) {
-            acc = 1.0;
-        }
-        A[(size_t)i * Np + j] = acc;
-        A[(size_t)j * Np + i] = acc;
-    }
-    if (I == 0 && J == 0) {
-        for (int i = threadIdx.x; i < Np; i += 256) {
+    const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;
+    for (int k0 = 0; k0 <= r0; k0 += 32) {
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int i = k0 + ty + 8 * s, j = r0 + tx;   // the chunks' row and column
             double acc = 0.0;
-            if (i < T)
-                for (int k = band_ptr[i]; k < band_ptr[i + 1]; ++k) {
-                    const int q = band_q[k];
-                    const int p = w[q];
-                    if (p != 0) acc += (double)p * theta[(size_t)q * T + i];
+            if (i <= j && j < nd) {
+                for (int k = c0; k < c1; ++k) {
+                    const ChunkOut o = outs[qchunk[k]];
+                    const int a = i + is - o.fis, b = j + is - o.fis;
+                    if (a < 0 || b >= o.nq) continue;   // a <= b
+                    acc += fc[o.fc_off + (size_t)a * o.nq + b];
                 }
-            rhs[(size_t)b * Np + i] = acc;
+            }
+            tile[ty + 8 * s][tx] = acc;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int r = r0 + ty + 8 * s, c = k0 + tx;
+            if (r < nd && c <= r) F[(size_t)r * nd + c] = tile[tx][ty + 8 * s];
         }
     }
 }
 
-// x = Li^T (Li rhs) per realisation (one block each), written to R[b0 + b]
-// (T values).  A band no weighted spectrum covers has a zero row and a zero
-// right-hand side with its diagonal set to 1, so its x is zero, as
-// safeSolveCho leaves it.
-__global__ __launch_bounds__(256) void k_boot_solve(const double *mat, const double *rhs, int b0, int T, int Np,
+// The batch's weights as doubles, realisation contiguous: Wt[q][b], zero past nb.
+__global__ __launch_bounds__(256) void k_boot_weights(const int *W, int nqso, int b0, int nb, double *Wt) {
+    const int e = blockIdx.x * 256 + threadIdx.x, q = e / BOOT_BATCH, b = e % BOOT_BATCH;
+    if (q < nqso) Wt[e] = (b < nb) ? (double)W[(size_t)(b0 + b) * nqso + q] : 0.0;
+}
+
+// F_b's lower triangle (identity past T, empty diagonals set to 1) in the L
+// slot of realisation b's matrices.  A wave takes one row r, 64 columns and RB
+// realisations: the spectra covering band r in queue order are the same for
+// the whole wave, so their weights are scalars and each Fisher element is
+// loaded once for RB realisations (read for every realisation by itself it
+// was 82 GB a batch at 4096 spectra: 3.8 ms a batch of 128 at 200 spectra,
+// 0.20 ms now).  The sums run in queue order; a spectrum of weight zero adds
+// nothing, also where its element is not finite.
+template <int RB>
+__global__ __launch_bounds__(256) void k_boot_build(const double *__restrict__ Wt, int nb, int T, int Np,
+                                                    const int *__restrict__ band_ptr,
+                                                    const BandEntry *__restrict__ band, const double *__restrict__ fq,
+                                                    double *mat) {
+    const int r = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int cb = blockIdx.x * 64, c = cb + threadIdx.x % 64, g0 = blockIdx.z * RB;
+    if (cb > r) return;
+    double acc[RB];
+#pragma unroll
+    for (int u = 0; u < RB; ++u) acc[u] = 0.0;
+    if (r < T) {
+        const int k1 = band_ptr[r + 1];
+        for (int k = band_ptr[r]; k < k1; ++k) {
+            const BandEntry e = band[k];
+            if (e.is > cb + 63) continue;
+            const double f = (c >= e.is && c <= r) ? fq[e.off + (long long)(r - e.is) * e.nd + (c - e.is)] : 0.0;
+            const double *w = Wt + (size_t)e.q * BOOT_BATCH + g0;
+            if (__builtin_expect(__any(!(fabs(f) <= 1.79769313486231571e308)), 0)) {
+#pragma unroll
+                for (int u = 0; u < RB; ++u)
+                    if (w[u] != 0.0) acc[u] = fma(w[u], f, acc[u]);
+            } else {
+#pragma unroll
+                for (int u = 0; u < RB; ++u) acc[u] = fma(w[u], f, acc[u]);
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < RB; ++u) {
+        if (g0 + u >= nb) break;
+        double v = acc[u];
+        if (c == r && (r >= T || v == 0.0)) v = 1.0;
+        mat[(size_t)(2 * (g0 + u) + 1) * Np * Np + (size_t)r * Np + c] = v;
+    }
+}
+
+// The right-hand sides, one workgroup per band, a thread per realisation.
+__global__ __launch_bounds__(BOOT_BATCH) void k_boot_rhs(const double *Wt, int nb, int T, int Np, const int *band_ptr,
+                                                         const BandEntry *band, const double *theta, double *rhs) {
+    const int i = blockIdx.x, b = threadIdx.x;
+    double acc = 0.0;
+    if (i < T)
+        for (int k = band_ptr[i]; k < band_ptr[i + 1]; ++k) {
+            const int q = band[k].q;
+            const double w = Wt[(size_t)q * BOOT_BATCH + b];
+            if (w != 0.0) acc = fma(w, theta[(size_t)q * T + i], acc);
+        }
+    if (b < nb) rhs[(size_t)b * Np + i] = acc;
+}
+
+// x of L L^T x = rhs per realisation (one block each) by block substitution
+// with the inverted diagonal blocks, written to R[b0 + b] (T values): one
+// right-hand side needs no more of the inverse, whose other blocks were two
+// thirds of the factorisation's work.  A band no weighted spectrum covers has a
+// zero row and a zero right-hand side with its diagonal set to 1, so its x is
+// zero, as safeSolveCho leaves it.  Each block row is a matrix-vector product of
+// all 512 threads: forward eight threads to a row, 128 bytes of it each time;
+// backward a wave to every eighth row, 512 bytes of it.
+__global__ __launch_bounds__(512) void k_boot_solve(const double *mat, const double *rhs, int b0, int T, int Np,
                                                     double *R) {
-    const int b = blockIdx.x;
-    const double *Li = mat + (size_t)b * 3 * Np * Np + 2 * (size_t)Np * Np;
+    const int b = blockIdx.x, tid = threadIdx.x, nt = Np / 64;
+    const double *L = mat + (size_t)(2 * b + 1) * Np * Np, *Li = L + (size_t)Np * Np;
     extern __shared__ double sh[];
-    double *y = sh;          // Np
-    const double *r = rhs + (size_t)b * Np;
-    for (int i = threadIdx.x; i < Np; i += 256) {
-        double s = 0.0;
-        for (int k = 0; k <= i; ++k) s += Li[(size_t)i * Np + k] * r[k];
-        y[i] = s;
-    }
+    double *y = sh, *t = sh + Np, *red = t + 64;   // Np, 64, 8 x 64
+    const int row = tid / 8, o = tid % 8, w = tid / 64, l = tid % 64;
+    for (int i = tid; i < Np; i += 512) y[i] = rhs[(size_t)b * Np + i];
     __syncthreads();
-    for (int i = threadIdx.x; i < T; i += 256) {
+    auto row_sum = [&](double s) {
+        for (int d = 4; d >= 1; d >>= 1) s += __shfl_xor(s, d, 64);
+        return s;
+    };
+    for (int p = 0; p < nt; ++p) {
+        const double *Lr = L + (size_t)(64 * p + row) * Np;
         double s = 0.0;
-        for (int k = i; k < Np; ++k) s += Li[(size_t)k * Np + i] * y[k];
-        R[(size_t)(b0 + b) * T + i] = s;
+#pragma unroll 4
+        for (int k = 2 * o; k < 64 * p; k += 16) {
+            const dvec2 v = *(const dvec2 *)(Lr + k);
+            s += v.x * y[k] + v.y * y[k + 1];
+        }
+        s = row_sum(s);
+        if (o == 0) t[row] = y[64 * p + row] - s;
+        __syncthreads();
+        const double *Ir = Li + (size_t)(64 * p + row) * Np + 64 * p;
+        s = 0.0;
+#pragma unroll
+        for (int k = 2 * o; k < 64; k += 16) {
+            const dvec2 v = *(const dvec2 *)(Ir + k);
+            s += v.x * t[k] + v.y * t[k + 1];
+        }
+        s = row_sum(s);
+        __syncthreads();
+        if (o == 0) y[64 * p + row] = s;
+        __syncthreads();
     }
+    auto col_sum = [&](double s, double *dst, double sign, const double *add) {
+        red[64 * w + l] = s;
+        __syncthreads();
+        if (w == 0) {
+            double v = 0.0;
+            for (int q = 0; q < 8; ++q) v += red[64 * q + l];
+            dst[l] = (add ? add[l] : 0.0) + sign * v;
+        }
+        __syncthreads();
+    };
+    for (int p = nt - 1; p >= 0; --p) {
+        double s = 0.0;
+#pragma unroll 8
+        for (int i = 64 * (p + 1) + w; i < Np; i += 8) s += L[(size_t)i * Np + 64 * p + l] * y[i];
+        col_sum(s, t, -1.0, y + 64 * p);
+        s = 0.0;
+#pragma unroll
+        for (int i = w; i < 64; i += 8) s += Li[(size_t)(64 * p + i) * Np + 64 * p + l] * t[i];
+        col_sum(s, y + 64 * p, 1.0, nullptr);
+    }
+    for (int i = tid; i < T; i += 512) R[(size_t)(b0 + b) * T + i] = y[i];
 }
 
 void launch_boot_collapse_fisher(hipStream_t st, const ChunkOut *outs, const double *fc, const int *qptr,
                                  const int *qchunk, const int *qstart, const int *qdim, const long long *fq_off,
-                                 int nqso, double *fq) {
-    k_boot_collapse_fisher<<<nqso, 256, 0, st>>>(outs, fc, qptr, qchunk, qstart, qdim, fq_off, fq);
+                                 int nqso, int dim_max, double *fq) {
+    k_boot_collapse_fisher<<<dim3(nqso, (dim_max + 31) / 32), 256, 0, st>>>(outs, fc, qptr, qchunk, qstart, qdim,
+                                                                           fq_off, fq);
 }
 
 void launch_boot_build(hipStream_t st, const int *W, int nqso, int b0, int nb, int T, int Np, const int *band_ptr,
-                       const int *band_q, const int *qstart, const int *qdim, const long long *fq_off,
-                       const double *fq, const double *theta, double *mat, double *rhs) {
-    const int t = Np / 64;
-    k_boot_build<<<dim3(t, t, nb), 256, 0, st>>>(W, nqso, b0, T, Np, band_ptr, band_q, qstart, qdim, fq_off, fq,
-                                                 theta, mat, rhs);
+                       const BandEntry *band, const double *fq, const double *theta, double *Wt, double *mat,
+                       double *rhs) {
+    constexpr int RB = 32;
+    static_assert(BOOT_BATCH % RB == 0, "whole groups of realisations");
+    k_boot_weights<<<((size_t)nqso * BOOT_BATCH + 255) / 256, 256, 0, st>>>(W, nqso, b0, nb, Wt);
+    k_boot_build<RB><<<dim3(Np / 64, Np / 4, (nb + RB - 1) / RB), 256, 0, st>>>(Wt, nb, T, Np, band_ptr, band, fq, mat);
+    k_boot_rhs<<<Np, BOOT_BATCH, 0, st>>>(Wt, nb, T, Np, band_ptr, band, theta, rhs);
 }
 
 void launch_boot_solve(hipStream_t st, const double *mat, const double *rhs, int b0, int nb, int T, int Np,
                        double *R) {
-    k_boot_solve<<<nb, 256, (size_t)Np * sizeof(double), st>>>(mat, rhs, b0, T, Np, R);
+    k_boot_solve<<<nb, 512, ((size_t)Np + 64 + 512) * sizeof(double), st>>>(mat, rhs, b0, T, Np, R);
 }
 
 void launch_boot_collapse(hipStream_t st, const ChunkOut *outs, const double *dbt, const int *qptr,

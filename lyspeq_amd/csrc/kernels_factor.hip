@@ -331,7 +331,7 @@ __global__ __launch_bounds__(256) void k_chol_diag(const ChunkDev *cs, double *m
     }
 }
 
-__global__ __launch_bounds__(256, 4) void k_chol_panel(const ChunkDev *cs, double *mat, int p, int ntmax) {
+__global__ __launch_bounds__(256, 4) void k_chol_panel(const ChunkDev *cs, double *mat, int p, int ntrsm) {
     const ChunkDev c = cs[blockIdx.y];
     const int Np = c.Np, nt = Np / FB, p0 = p * FB, bx = blockIdx.x;
     if (p >= nt) return;
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(256, 4) void k_chol_panel(const ChunkDev *cs, doubl
     __shared__ double sb[FB * KLD];
     fd4 acc[2][2];
     tile_zero(acc);
-    if (bx < ntmax) {
+    if (bx < ntrsm) {
         // TRSM tile: L[i,p] = A[i,p] Li[p,p]^T
         const int i = p + 1 + bx;
         if (i >= nt) return;
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(256, 4) void k_chol_panel(const ChunkDev *cs, doubl
         return;
     }
     // block row p of the inverse: T = sum_{k=j}^{p-1} L[p,k] Li[k,j]
-    const int j = bx - ntmax;
+    const int j = bx - ntrsm;
     if (j >= p) return;
 #pragma unroll 1
     for (int k = j; k < p; ++k) block_nt(sa, sb, L, p0, k * FB, Li, k * FB, j * FB, true, Np, acc);
@@ -403,17 +403,22 @@ __global__ __launch_bounds__(256, 4) void k_chol_update(const ChunkDev *cs, doub
     tile_each(acc, [&](int r, int q, double x) { L[(size_t)(bi * FB + r) * Np + bj * FB + q] -= x; });
 }
 
-void launch_cholesky(const LaunchCtx &L, int *status) {
+static void factor(const LaunchCtx &L, int *status, bool inverse) {
     const int ntmax = L.np_max / FB;
-    k_chol_init<<<dim3(64, L.nchunks), 256, 0, L.stream>>>(L.chunks, L.mat);
     for (int p = 0; p < ntmax; ++p) {
-        k_chol_diag<<<L.nchunks, 256, 0, L.stream>>>(L.chunks, L.mat, status, p);
-        const int gx = ntmax + p;   // TRSM tiles (< ntmax) and inverse tiles j < p
-        k_chol_panel<<<dim3(gx, L.nchunks), 256, 0, L.stream>>>(L.chunks, L.mat, p, ntmax);
         const int m = ntmax - p - 1;
+        k_chol_diag<<<L.nchunks, 256, 0, L.stream>>>(L.chunks, L.mat, status, p);
+        // TRSM tiles (m of them), then the inverse's tiles j < p
+        const int gx = m + (inverse ? p : 0);
+        if (gx > 0) k_chol_panel<<<dim3(gx, L.nchunks), 256, 0, L.stream>>>(L.chunks, L.mat, p, m);
         if (m > 0) k_chol_update<<<dim3(m * (m + 1) / 2, L.nchunks), 256, 0, L.stream>>>(L.chunks, L.mat, p);
     }
 }
+void launch_cholesky(const LaunchCtx &L, int *status) {
+    k_chol_init<<<dim3(64, L.nchunks), 256, 0, L.stream>>>(L.chunks, L.mat);
+    factor(L, status, true);
+}
+void launch_cholesky_in_place(const LaunchCtx &L, int *status) { factor(L, status, false); }
 
 // The inverse is formed inside the blocked factorisation.
 void launch_trinv(const LaunchCtx &) {}

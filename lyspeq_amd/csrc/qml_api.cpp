@@ -1631,16 +1631,18 @@ int qml_bootstrap_complete(qml_ctx *c, int nboots, unsigned long long seed, int 
         qdim[q] = hi - lo;
         fq_off[q + 1] = fq_off[q] + (long long)qdim[q] * qdim[q];
     }
-    std::vector<int> band_ptr(T + 1, 0), band_q;
+    std::vector<int> band_ptr(T + 1, 0);
     for (int q = 0; q < nqso; ++q)
         for (int i = qstart[q]; i < qstart[q] + qdim[q]; ++i) ++band_ptr[i + 1];
     for (int i = 0; i < T; ++i) band_ptr[i + 1] += band_ptr[i];
-    band_q.resize(band_ptr[T]);
+    std::vector<BandEntry> band(std::max(band_ptr[T], 1));
     {
         std::vector<int> fill(band_ptr.begin(), band_ptr.end() - 1);
         for (int q = 0; q < nqso; ++q)
-            for (int i = qstart[q]; i < qstart[q] + qdim[q]; ++i) band_q[fill[i]++] = q;
+            for (int i = qstart[q]; i < qstart[q] + qdim[q]; ++i)
+                band[fill[i]++] = BandEntry{q, qstart[q], qdim[q], 0, fq_off[q]};
     }
+    const int dim_max = *std::max_element(qdim.begin(), qdim.end());
     // weights: realisation-major, one draw per spectrum (_oneBoot draws one
     // per spectrum in queue order for every realisation)
     std::vector<int> W((size_t)nboots * nqso);
@@ -1653,7 +1655,7 @@ int qml_bootstrap_complete(qml_ctx *c, int nboots, unsigned long long seed, int 
     HIPCHK(hipSetDevice(c->device));
     HIPCHK(hipStreamSynchronize(c->st));
     HIPCHK(hipStreamSynchronize(c->st2));
-    const int BATCH = std::min(nboots, 128);
+    const int BATCH = std::min(nboots, BOOT_BATCH);
     std::vector<void *> allocs;
     auto dalloc = [&](void **p, size_t bytes) -> hipError_t {
         const hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 8));
@@ -1663,9 +1665,10 @@ int qml_bootstrap_complete(qml_ctx *c, int nboots, unsigned long long seed, int 
     std::vector<double> R((size_t)nboots * T);
     std::vector<int> status(nboots, 0);
     auto run = [&]() -> int {
-        int *d_qptr, *d_qchunk, *d_qstart, *d_qdim, *d_bptr, *d_bq, *d_W, *d_status;
+        int *d_qptr, *d_qchunk, *d_qstart, *d_qdim, *d_bptr, *d_W, *d_status;
+        BandEntry *d_band;
         long long *d_fqoff;
-        double *d_fq, *d_theta, *d_mat, *d_rhs, *d_R, *d_mean, *d_cov;
+        double *d_fq, *d_theta, *d_Wt, *d_mat, *d_rhs, *d_R, *d_mean, *d_cov;
         ChunkDev *d_cd;
         HIPCHK(dalloc((void **)&d_qptr, qptr.size() * sizeof(int)));
         HIPCHK(dalloc((void **)&d_qchunk, qchunk.size() * sizeof(int)));
@@ -1673,14 +1676,15 @@ int qml_bootstrap_complete(qml_ctx *c, int nboots, unsigned long long seed, int 
         HIPCHK(dalloc((void **)&d_qdim, nqso * sizeof(int)));
         HIPCHK(dalloc((void **)&d_fqoff, (nqso + 1) * sizeof(long long)));
         HIPCHK(dalloc((void **)&d_bptr, band_ptr.size() * sizeof(int)));
-        HIPCHK(dalloc((void **)&d_bq, band_q.size() * sizeof(int)));
+        HIPCHK(dalloc((void **)&d_band, band.size() * sizeof(BandEntry)));
+        HIPCHK(dalloc((void **)&d_Wt, (size_t)nqso * BOOT_BATCH * sizeof(double)));
         HIPCHK(dalloc((void **)&d_W, W.size() * sizeof(int)));
         HIPCHK(dalloc((void **)&d_fq, (size_t)fq_off[nqso] * sizeof(double)));
         HIPCHK(dalloc((void **)&d_theta, (size_t)nqso * T * sizeof(double)));
-        HIPCHK(dalloc((void **)&d_mat, (size_t)BATCH * 3 * Np * Np * sizeof(double)));
+        HIPCHK(dalloc((void **)&d_mat, (size_t)(2 * BATCH + 1) * Np * Np * sizeof(double)));
         HIPCHK(dalloc((void **)&d_rhs, (size_t)BATCH * Np * sizeof(double)));
         HIPCHK(dalloc((void **)&d_R, R.size() * sizeof(double)));
-        HIPCHK(dalloc((void **)&d_status, BATCH * sizeof(int)));
+        HIPCHK(dalloc((void **)&d_status, nboots * sizeof(int)));
         HIPCHK(dalloc((void **)&d_mean, (size_t)T * sizeof(double)));
         HIPCHK(dalloc((void **)&d_cov, (size_t)T * T * sizeof(double)));
         HIPCHK(dalloc((void **)&d_cd, BATCH * sizeof(ChunkDev)));
@@ -1690,11 +1694,11 @@ int qml_bootstrap_complete(qml_ctx *c, int nboots, unsigned long long seed, int 
         HIPCHK(hipMemcpy(d_qdim, qdim.data(), nqso * sizeof(int), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(d_fqoff, fq_off.data(), (nqso + 1) * sizeof(long long), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(d_bptr, band_ptr.data(), band_ptr.size() * sizeof(int), hipMemcpyHostToDevice));
-        if (!band_q.empty())
-            HIPCHK(hipMemcpy(d_bq, band_q.data(), band_q.size() * sizeof(int), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(d_band, band.data(), band.size() * sizeof(BandEntry), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(d_W, W.data(), W.size() * sizeof(int), hipMemcpyHostToDevice));
-        // realisation b of a batch is factorised as a "chunk" of size Np at
-        // b * 3 Np^2 (A, L, Li), its status at b
+        // realisation b of a batch is factorised as a "chunk" of size Np whose
+        // A, L, Li would start at 2 b Np^2 (A, unused, lies over the Li of the
+        // one before), its status at b
         std::vector<ChunkDev> cd(BATCH);
         for (int b = 0; b < BATCH; ++b) {
             cd[b] = ChunkDev{};
@@ -1702,12 +1706,12 @@ int qml_bootstrap_complete(qml_ctx *c, int nboots, unsigned long long seed, int 
             cd[b].Np = Np;
             cd[b].nt = Np / TILE;
             cd[b].gidx = b;
-            cd[b].mat_off = (long long)b * 3 * Np * Np;
+            cd[b].mat_off = (long long)b * 2 * Np * Np;
         }
         HIPCHK(hipMemcpy(d_cd, cd.data(), BATCH * sizeof(ChunkDev), hipMemcpyHostToDevice));
         launch_boot_collapse(c->st, c->d_outs, c->d_dbt, d_qptr, d_qchunk, nqso, T, d_theta);
         launch_boot_collapse_fisher(c->st, c->d_outs, c->d_fc, d_qptr, d_qchunk, d_qstart, d_qdim, d_fqoff, nqso,
-                                    d_fq);
+                                    dim_max, d_fq);
         HIPCHK(hipGetLastError());
         LaunchCtx L{};
         L.stream = c->st;
@@ -1717,14 +1721,13 @@ int qml_bootstrap_complete(qml_ctx *c, int nboots, unsigned long long seed, int 
         for (int b0 = 0; b0 < nboots; b0 += BATCH) {
             const int nb = std::min(BATCH, nboots - b0);
             L.nchunks = nb;
-            launch_boot_build(c->st, d_W, nqso, b0, nb, T, Np, d_bptr, d_bq, d_qstart, d_qdim, d_fqoff, d_fq,
-                              d_theta, d_mat, d_rhs);
-            launch_cholesky(L, d_status);
+            launch_boot_build(c->st, d_W, nqso, b0, nb, T, Np, d_bptr, d_band, d_fq, d_theta, d_Wt, d_mat, d_rhs);
+            launch_cholesky_in_place(L, d_status + b0);
             launch_boot_solve(c->st, d_mat, d_rhs, b0, nb, T, Np, d_R);
             HIPCHK(hipGetLastError());
-            HIPCHK(hipMemcpyAsync(status.data() + b0, d_status, nb * sizeof(int), hipMemcpyDeviceToHost, c->st));
-            HIPCHK(hipStreamSynchronize(c->st));
         }
+        HIPCHK(hipStreamSynchronize(c->st));
+        HIPCHK(hipMemcpy(status.data(), d_status, nboots * sizeof(int), hipMemcpyDeviceToHost));
         HIPCHK(hipMemcpy(R.data(), d_R, R.size() * sizeof(double), hipMemcpyDeviceToHost));
         // the valid realisations, in order (allpowers + ii T, ii counting the valid ones)
         int nv = 0;

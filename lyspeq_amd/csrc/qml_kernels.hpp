@@ -48,8 +48,11 @@ void launch_assemble(const LaunchCtx &L, const double *theta);
 // no kernel matches the batch's layout (nothing is launched).
 bool launch_rmat(const LaunchCtx &L);
 // kernels_factor.hip: L = chol(A) and Li = L^-1 (both formed by
-// launch_cholesky; launch_trinv is kept for the timing slot and is empty)
+// launch_cholesky; launch_trinv is kept for the timing slot and is empty).
+// launch_cholesky_in_place factors the lower triangle in the L slot and inverts
+// its diagonal blocks only.
 void launch_cholesky(const LaunchCtx &L, int *status);
+void launch_cholesky_in_place(const LaunchCtx &L, int *status);
 void launch_trinv(const LaunchCtx &L);
 void launch_solve(const LaunchCtx &L);
 void launch_dpass(const LaunchCtx &L);
@@ -121,16 +124,23 @@ constexpr long long BOOT_NOALLOC_MAX = 1LL << 23;
 constexpr int BOOT_NOALLOC_DEVICES = 64;
 int boot_noalloc_setup(int device);
 double *boot_noalloc_scratch(int device);
-// The complete form: per-spectrum collapsed Fisher upper blocks (ndim x ndim
-// at fq_off); per batch of nb realisations from b0, F_b and its right-hand
-// side in the matrix layout of the batched Cholesky (A, L, Li per
-// realisation, Np x Np each), then x = Li^T Li rhs into R.
+// The complete form: per-spectrum collapsed Fisher lower triangles (ndim x ndim
+// at fq_off); per batch of nb <= BOOT_BATCH realisations from b0, F_b in the L
+// slot and its right-hand side; then x = F_b^-1 rhs into R.  Realisation b's
+// matrices are L at (2 b + 1) Np^2 and Li at (2 b + 2) Np^2 of mat (the A slot
+// of the batched Cholesky's layout is not used).
+constexpr int BOOT_BATCH = 128;
+// A spectrum covering a band: its index, first band, bands and Fisher block.
+struct BandEntry {
+    int q, is, nd, pad;
+    long long off;
+};
 void launch_boot_collapse_fisher(hipStream_t st, const ChunkOut *outs, const double *fc, const int *qptr,
                                  const int *qchunk, const int *qstart, const int *qdim, const long long *fq_off,
-                                 int nqso, double *fq);
+                                 int nqso, int dim_max, double *fq);
 void launch_boot_build(hipStream_t st, const int *W, int nqso, int b0, int nb, int T, int Np, const int *band_ptr,
-                       const int *band_q, const int *qstart, const int *qdim, const long long *fq_off,
-                       const double *fq, const double *theta, double *mat, double *rhs);
+                       const BandEntry *band, const double *fq, const double *theta, double *Wt, double *mat,
+                       double *rhs);
 void launch_boot_solve(hipStream_t st, const double *mat, const double *rhs, int b0, int nb, int T, int Np,
                        double *R);
 
