@@ -7,20 +7,22 @@
 //                     (OneQSOEstimate::collapseBootstrap)
 //   k_boot_realize    R[b][i] = sum over spectra q, in queue order, of
 //                     p[q][b] theta_q[i] (addBootPowerOnly: one dger per spectrum)
-//   k_boot_mean       mean[i] = (sum over b of R[b][i]) / nboots, as sum * (1/n)
-//   k_boot_cov        cov[i][j] = sum over b of (R[b][i] - mean[i])(R[b][j] -
+//   k_boot_mean(_part) mean[i] = (sum over b of R[b][i]) / nboots, as sum * (1/n)
+//   k_boot_cov(_part) cov[i][j] = sum over b of (R[b][i] - mean[i])(R[b][j] -
 //                     mean[j]), times 1/(nboots - 1) (dsyr per realisation)
 //
 // The complete form (k_boot_collapse_fisher, k_boot_build, the chunk
 // engine's batched Cholesky, k_boot_solve) follows below.
 //
-// All FP64.  Every output is summed in the reference's order (chunks, spectra,
-// realisations ascending), one thread per output element of a 64 x 64 tile,
-// with the operands staged through LDS 16 terms at a time.  HBM traffic is
+// All FP64.  The sums over chunks and spectra run in the reference's order, one
+// thread per output element of a 64 x 64 tile, with the operands staged through
+// LDS 16 terms at a time; those over realisations run in ranges whose partial
+// sums are added in order.  HBM traffic is
 // small next to the chunk step (nboots x nspectra ints, nboots x T doubles).
 #include "qml_common.hpp"
 #include "qml_kernels.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 namespace qml {
@@ -87,59 +89,121 @@ __global__ __launch_bounds__(256) void k_boot_realize(const int *P, const double
         }
 }
 
-__global__ __launch_bounds__(256) void k_boot_mean(const double *R, int nboots, int T, double *mean) {
+// Sums over a range of realisations, blockIdx.y of gridDim.y: part[y][i].  One
+// thread per band ran down all realisations (968 us at 4000 x 455).
+__global__ __launch_bounds__(256) void k_boot_mean_part(const double *R, int nboots, int T, double *part) {
+    __shared__ double red[4][64];
+    const int l = threadIdx.x % 64, w = threadIdx.x / 64, i = blockIdx.x * 64 + l;
+    const int b0 = (int)((long long)nboots * blockIdx.y / gridDim.y);
+    const int b1 = (int)((long long)nboots * (blockIdx.y + 1) / gridDim.y);
+    double s = 0.0;
+    if (i < T)
+#pragma unroll 4
+        for (int b = b0 + w; b < b1; b += 4) s += R[(size_t)b * T + i];
+    red[w][l] = s;
+    __syncthreads();
+    if (w == 0 && i < T) part[(size_t)blockIdx.y * T + i] = (red[0][l] + red[1][l]) + (red[2][l] + red[3][l]);
+}
+__global__ __launch_bounds__(256) void k_boot_mean(const double *part, int nparts, int nboots, int T, double *mean) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= T) return;
     double s = 0.0;
-    for (int b = 0; b < nboots; ++b) s += R[(size_t)b * T + i];
+    for (int p = 0; p < nparts; ++p) s += part[(size_t)p * T + i];
     mean[i] = s * (1.0 / nboots);
 }
 
-// Upper 64 x 64 tiles of the covariance, mirrored into the lower triangle.
-__global__ __launch_bounds__(256) void k_boot_cov(const double *R, const double *mean, int nboots, int T,
-                                                  double *cov) {
-    const int I = blockIdx.y, J = blockIdx.x;
-    if (J < I) return;
-    __shared__ double sa[KT][BT + 1], sb[KT][BT + 1];
-    const int i0 = I * BT, j0 = J * BT;
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    double acc[4][4] = {};
-    for (int b0 = 0; b0 < nboots; b0 += KT) {
-        for (int e = threadIdx.x; e < KT * BT; e += 256) {
-            const int k = e / BT, c = e % BT;
-            const int b = b0 + k;
-            sa[k][c] = (b < nboots && i0 + c < T) ? R[(size_t)b * T + i0 + c] - mean[i0 + c] : 0.0;
-            sb[k][c] = (b < nboots && j0 + c < T) ? R[(size_t)b * T + j0 + c] - mean[j0 + c] : 0.0;
-        }
-        __syncthreads();
-        const int kn = min(KT, nboots - b0);
-        for (int k = 0; k < kn; ++k) {
-            double a[4], bb[4];
+// Upper 64 x 64 tiles of sum over b of (R - mean)(R - mean)^T on the matrix
+// cores: a workgroup takes one tile and the range blockIdx.y of the
+// realisations, a quarter of it per wave, whose 16 blocks of 16 x 16 stay in
+// registers; a fragment is 16 consecutive bands of four realisations, loaded
+// one step ahead.  36 tiles at T = 455 would leave the chip empty without the
+// split over realisations (798 us at 4000 x 455 with one workgroup a tile).
+typedef double bd4 __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(256, 2) void k_boot_cov_part(const double *R, const double *mean, int nboots, int T,
+                                                          double *part) {
+    __shared__ double red[2][4][256];
+    int t = blockIdx.x, J = 0;   // tile t of the upper triangle by columns: I <= J
+    while (t > J) { t -= J + 1; ++J; }
+    const int I = t, tid = threadIdx.x, lane = tid % 64, lr = lane % 16, lq = lane / 16;
+    const int w = __builtin_amdgcn_readfirstlane(tid / 64);
+    const long long s0 = 4LL * blockIdx.y + w, ns = 4LL * gridDim.y;
+    const int b0 = (int)(nboots * s0 / ns), b1 = (int)(nboots * (s0 + 1) / ns);
+    int ia[4], ja[4];
+    double mi[4], mj[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                a[u] = sa[k][ty + 16 * u];
-                bb[u] = sb[k][tx + 16 * u];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc[u][v] += a[u] * bb[v];
-        }
-        __syncthreads();
+    for (int x = 0; x < 4; ++x) {
+        ia[x] = min(64 * I + 16 * x + lr, T - 1);
+        ja[x] = min(64 * J + 16 * x + lr, T - 1);
+        mi[x] = mean[ia[x]];
+        mj[x] = mean[ja[x]];
     }
-    const double scale = 1.0 / (nboots - 1);
+    bd4 acc[4][4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int x = 0; x < 4; ++x)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int i = i0 + ty + 16 * u, j = j0 + tx + 16 * v;
-            if (i < T && j < T && j >= i) {
-                const double c = acc[u][v] * scale;
-                cov[(size_t)i * T + j] = c;
-                cov[(size_t)j * T + i] = c;
-            }
+        for (int y = 0; y < 4; ++y) acc[x][y] = bd4{0.0, 0.0, 0.0, 0.0};
+    double va[4], vb[4];
+    auto fetch = [&](int b) {
+        const double *row = R + (size_t)min(b + lq, nboots - 1) * T;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            va[x] = row[ia[x]];
+            vb[x] = row[ja[x]];
+        }
+    };
+    if (b0 < b1) fetch(b0);
+    for (int b = b0; b < b1; b += 4) {
+        double a[4], c[4];
+        const bool in = b + lq < b1;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            a[x] = in ? va[x] - mi[x] : 0.0;
+            c[x] = in ? vb[x] - mj[x] : 0.0;
+        }
+        fetch(b + 4);
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[x], c[y], acc[x][y], 0, 0, 0);
+    }
+    double *C = part + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * BT * BT;
+    int flip = 0;
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) red[flip][w][64 * u + lane] = acc[x][y][u];
+            __syncthreads();
+            C[(16 * x + tid / 16) * BT + 16 * y + tid % 16] =
+                (red[flip][0][tid] + red[flip][1][tid]) + (red[flip][2][tid] + red[flip][3][tid]);
+            flip ^= 1;
         }
 }
+// cov from the ranges' partial tiles, mirrored into the lower triangle.
+__global__ __launch_bounds__(256) void k_boot_cov(const double *part, int nparts, int nboots, int T, double *cov) {
+    int t = blockIdx.x, J = 0;
+    while (t > J) { t -= J + 1; ++J; }
+    const int I = t;
+    const double scale = 1.0 / (nboots - 1);
+    for (int e = blockIdx.y * 256 + threadIdx.x; e < BT * BT; e += 256 * gridDim.y) {
+        const int i = I * BT + e / BT, j = J * BT + e % BT;
+        if (i >= T || j >= T || j < i) continue;
+        double s = 0.0;
+        for (int p = 0; p < nparts; ++p) s += part[((size_t)p * gridDim.x + blockIdx.x) * BT * BT + e];
+        s *= scale;
+        cov[(size_t)i * T + j] = s;
+        cov[(size_t)j * T + i] = s;
+    }
+}
+
+// Ranges of realisations for the covariance: enough for about two workgroups
+// per CU, at least 16 realisations each; for the mean, at least 64.
+static int cov_parts(int nboots, int T) {
+    const int nt = (T + BT - 1) / BT, tiles = nt * (nt + 1) / 2;
+    return std::max(1, std::min((512 + tiles - 1) / tiles, nboots / 16));
+}
+static int mean_parts(int nboots) { return std::max(1, std::min(64, nboots / 64)); }
 
 // ------------------------------------------------ complete bootstrap --
 // The complete form (PoissonBootstrapper::_oneBoot, core/bootstrapper.hpp:
@@ -348,19 +412,26 @@ void launch_boot_collapse(hipStream_t st, const ChunkOut *outs, const double *db
     k_boot_collapse<<<nqso, 256, 0, st>>>(outs, dbt, qptr, qchunk, T, theta);
 }
 
-void launch_boot_meancov(hipStream_t st, const double *R, int nboots, int T, double *mean, double *cov) {
-    const int tt = (T + BT - 1) / BT;
-    k_boot_mean<<<(T + 255) / 256, 256, 0, st>>>(R, nboots, T, mean);
-    k_boot_cov<<<dim3(tt, tt), 256, 0, st>>>(R, mean, nboots, T, cov);
+size_t boot_meancov_scratch(int nboots, int T) {
+    const size_t nt = (T + BT - 1) / BT;
+    return std::max((size_t)mean_parts(nboots) * T, (size_t)cov_parts(nboots, T) * (nt * (nt + 1) / 2) * BT * BT);
+}
+void launch_boot_meancov(hipStream_t st, const double *R, int nboots, int T, double *scratch, double *mean,
+                         double *cov) {
+    const int nt = (T + BT - 1) / BT, tiles = nt * (nt + 1) / 2, mp = mean_parts(nboots), cp = cov_parts(nboots, T);
+    k_boot_mean_part<<<dim3(nt, mp), 256, 0, st>>>(R, nboots, T, scratch);
+    k_boot_mean<<<(T + 255) / 256, 256, 0, st>>>(scratch, mp, nboots, T, mean);
+    k_boot_cov_part<<<dim3(tiles, cp), 256, 0, st>>>(R, mean, nboots, T, scratch);
+    k_boot_cov<<<dim3(tiles, 4), 256, 0, st>>>(scratch, cp, nboots, T, cov);
 }
 
 void launch_bootstrap(hipStream_t st, const ChunkOut *outs, const double *dbt, const int *qptr, const int *qchunk,
-                      int nqso, int T, const int *P, int nboots, double *theta, double *R, double *mean,
-                      double *cov) {
+                      int nqso, int T, const int *P, int nboots, double *theta, double *R, double *scratch,
+                      double *mean, double *cov) {
     launch_boot_collapse(st, outs, dbt, qptr, qchunk, nqso, T, theta);
     const int tt = (T + BT - 1) / BT;
     k_boot_realize<<<dim3(tt, (nboots + BT - 1) / BT), 256, 0, st>>>(P, theta, nqso, nboots, T, R);
-    launch_boot_meancov(st, R, nboots, T, mean, cov);
+    launch_boot_meancov(st, R, nboots, T, scratch, mean, cov);
 }
 
 // ---------------------------------------------------------------------------

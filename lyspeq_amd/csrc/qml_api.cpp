@@ -1572,9 +1572,9 @@ int qml_bootstrap(qml_ctx *c, int nboots, unsigned long long seed, int nqso, con
     HIPCHK(hipStreamSynchronize(c->st));
     HIPCHK(hipStreamSynchronize(c->st2));
     int *d_qptr = nullptr, *d_qchunk = nullptr, *d_P = nullptr;
-    double *d_theta = nullptr, *d_R = nullptr, *d_mean = nullptr, *d_cov = nullptr;
+    double *d_theta = nullptr, *d_R = nullptr, *d_mean = nullptr, *d_cov = nullptr, *d_scr = nullptr;
     auto release = [&]() {
-        void *ps[] = {d_qptr, d_qchunk, d_P, d_theta, d_R, d_mean, d_cov};
+        void *ps[] = {d_qptr, d_qchunk, d_P, d_theta, d_R, d_mean, d_cov, d_scr};
         for (void *p : ps) if (p) hipFree(p);
     };
     auto run = [&]() -> int {
@@ -1585,12 +1585,13 @@ int qml_bootstrap(qml_ctx *c, int nboots, unsigned long long seed, int nqso, con
         HIPCHK(hipMalloc(&d_R, (size_t)nboots * T * sizeof(double)));
         HIPCHK(hipMalloc(&d_mean, (size_t)T * sizeof(double)));
         HIPCHK(hipMalloc(&d_cov, (size_t)T * T * sizeof(double)));
+        HIPCHK(hipMalloc(&d_scr, boot_meancov_scratch(nboots, T) * sizeof(double)));
         HIPCHK(hipMemcpy(d_qptr, qptr.data(), qptr.size() * sizeof(int), hipMemcpyHostToDevice));
         if (!qchunk.empty())
             HIPCHK(hipMemcpy(d_qchunk, qchunk.data(), qchunk.size() * sizeof(int), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(d_P, P.data(), P.size() * sizeof(int), hipMemcpyHostToDevice));
-        launch_bootstrap(c->st, c->d_outs, c->d_dbt, d_qptr, d_qchunk, nqso, T, d_P, nboots, d_theta, d_R, d_mean,
-                         d_cov);
+        launch_bootstrap(c->st, c->d_outs, c->d_dbt, d_qptr, d_qchunk, nqso, T, d_P, nboots, d_theta, d_R, d_scr,
+                         d_mean, d_cov);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(c->st));
         if (realizations)
@@ -1668,7 +1669,7 @@ int qml_bootstrap_complete(qml_ctx *c, int nboots, unsigned long long seed, int 
         int *d_qptr, *d_qchunk, *d_qstart, *d_qdim, *d_bptr, *d_W, *d_status;
         BandEntry *d_band;
         long long *d_fqoff;
-        double *d_fq, *d_theta, *d_Wt, *d_mat, *d_rhs, *d_R, *d_mean, *d_cov;
+        double *d_fq, *d_theta, *d_Wt, *d_mat, *d_rhs, *d_R, *d_mean, *d_cov, *d_scr;
         ChunkDev *d_cd;
         HIPCHK(dalloc((void **)&d_qptr, qptr.size() * sizeof(int)));
         HIPCHK(dalloc((void **)&d_qchunk, qchunk.size() * sizeof(int)));
@@ -1687,6 +1688,7 @@ int qml_bootstrap_complete(qml_ctx *c, int nboots, unsigned long long seed, int 
         HIPCHK(dalloc((void **)&d_status, nboots * sizeof(int)));
         HIPCHK(dalloc((void **)&d_mean, (size_t)T * sizeof(double)));
         HIPCHK(dalloc((void **)&d_cov, (size_t)T * T * sizeof(double)));
+        HIPCHK(dalloc((void **)&d_scr, boot_meancov_scratch(nboots, T) * sizeof(double)));
         HIPCHK(dalloc((void **)&d_cd, BATCH * sizeof(ChunkDev)));
         HIPCHK(hipMemcpy(d_qptr, qptr.data(), qptr.size() * sizeof(int), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(d_qchunk, qchunk.data(), qchunk.size() * sizeof(int), hipMemcpyHostToDevice));
@@ -1741,7 +1743,7 @@ int qml_bootstrap_complete(qml_ctx *c, int nboots, unsigned long long seed, int 
         if (realizations) std::copy(R.begin(), R.begin() + (size_t)nv * T, realizations);
         if (nv < 2) return fail(QML_ERR_ARG, "qml_bootstrap_complete: fewer than two valid realisations");
         HIPCHK(hipMemcpy(d_R, R.data(), (size_t)nv * T * sizeof(double), hipMemcpyHostToDevice));
-        launch_boot_meancov(c->st, d_R, nv, T, d_mean, d_cov);
+        launch_boot_meancov(c->st, d_R, nv, T, d_scr, d_mean, d_cov);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(c->st));
         HIPCHK(hipMemcpy(mean, d_mean, (size_t)T * sizeof(double), hipMemcpyDeviceToHost));

@@ -105,12 +105,15 @@ void launch_gram64(hipStream_t st, const ChunkDev *chunks, const Work *work, int
 // qptr/qchunk: CSR list of each spectrum's chunk ids (nqso + 1 offsets); P is
 // nqso x nboots Poisson weights; theta nqso x T and R nboots x T scratch.
 void launch_bootstrap(hipStream_t st, const ChunkOut *outs, const double *dbt, const int *qptr, const int *qchunk,
-                      int nqso, int T, const int *P, int nboots, double *theta, double *R, double *mean,
-                      double *cov);
+                      int nqso, int T, const int *P, int nboots, double *theta, double *R, double *scratch,
+                      double *mean, double *cov);
 
 void launch_boot_collapse(hipStream_t st, const ChunkOut *outs, const double *dbt, const int *qptr,
                           const int *qchunk, int nqso, int T, double *theta);
-void launch_boot_meancov(hipStream_t st, const double *R, int nboots, int T, double *mean, double *cov);
+// mean and covariance of R; scratch is boot_meancov_scratch(nboots, T) doubles.
+size_t boot_meancov_scratch(int nboots, int T);
+void launch_boot_meancov(hipStream_t st, const double *R, int nboots, int T, double *scratch, double *mean,
+                         double *cov);
 // Median bootstrap: R nboots x T (device) -> median (T) and the median
 // covariance (T x T); X is T x nboots scratch (deviations from the median).
 void launch_boot_median(hipStream_t st, const double *R, int nboots, int T, double *X, double *median,
