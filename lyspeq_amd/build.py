@@ -15,7 +15,7 @@ LIB = os.path.join(HERE, "libqmlhip.so")
 
 SOURCES = ["kernels_chunk.hip", "kernels_factor.hip", "kernels_gemm.hip", "kernels_gemm64.hip", "kernels_rmat.hip", "kernels_tables.hip",
            "kernels_boot.hip", "qml_api.cpp",
-           "rmat_prep.cpp"]
+           "rmat_prep.cpp", "poisson.cpp"]
 
 HIPCC_FLAGS = [
     "-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC",

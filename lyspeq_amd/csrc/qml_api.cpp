@@ -1,6 +1,7 @@
 // C ABI of the QML engine: chunk registration (the Chunk constructor's
 // bookkeeping), batch planning, and the per-iteration launch sequence.
 #include "lyspeq_qml.h"
+#include "poisson.hpp"
 #include "qml_kernels.hpp"
 
 #include <algorithm>
@@ -9,7 +10,6 @@
 #include <cstdlib>
 #include <cstring>
 #include <numeric>
-#include <random>
 #include <string>
 #include <vector>
 
@@ -1515,11 +1515,7 @@ int qml_set_chunk_active(qml_ctx *c, int id, int active) {
 
 int qml_poisson_draws(unsigned long long seed, long long n, int *out) {
     if (n < 0 || (n > 0 && !out)) return fail(QML_ERR_ARG, "qml_poisson_draws: bad count or null output");
-    // PoissonRNG of core/bootstrapper.hpp:19-37: a 64-bit Mersenne twister
-    // seeded once, unit-mean Poisson draws from the standard library
-    std::mt19937_64 rng(seed);
-    std::poisson_distribution<int> pd;
-    for (long long i = 0; i < n; ++i) out[i] = pd(rng);
+    poisson_draws(seed, n, out);
     return QML_OK;
 }
 
