@@ -1837,13 +1837,15 @@ int qml_make_tables(qml_ctx *c, const qml_table_spec *s, int npairs, const int *
     const double dxv = s->v_length / (nv - 1.0);
     // the signal grid (core/sq_table.cpp:221-227)
     const long long nrft = 1LL << ((int)std::ceil(std::log2(4.0 * nv)) + 1);
-    const int nhalf = (int)(nrft / 2), nmode = nhalf + 1;
+    const int nhalf = (int)(nrft / 2);
+    const SignalGrid grid = signal_grid(nhalf, nz);
     const double length = dxv / 2.0 * (double)nrft, dk = 2.0 * 3.14159265358979323846 / length;
     const double z1 = c->zcenters[0] - c->bins.z_bin_width;
     const double dz = c->bins.z_bin_width * (c->bins.nz + 1) / (nz - 1.0);
     const PD13 pd{s->pd13[0], s->pd13[1], s->pd13[2], s->pd13[3], s->pd13[4], s->pd13[5]};
-    // pairs per pass: outputs of up to 2 GiB on the device
-    const size_t per = (size_t)8 * ((deriv ? (size_t)nk * nv : 0) + (signal ? (size_t)nv * nz : 0));
+    // pairs per pass: outputs and the signal's partial sums of up to 2 GiB on the device
+    const size_t per = (size_t)8 * ((deriv ? (size_t)nk * nv : 0) +
+                                    (signal ? (size_t)nv * nz * (1 + grid.parts) + grid.mpad : 0));
     const int nb = (int)std::max<size_t>(1, std::min<size_t>(npairs, ((size_t)2 << 30) / per));
     struct Bufs {
         std::vector<void *> p;
@@ -1854,18 +1856,21 @@ int qml_make_tables(qml_ctx *c, const qml_table_spec *s, int npairs, const int *
         if (e == hipSuccess) bufs.p.push_back(*ptr);
         return e;
     };
-    double *d_pairs = nullptr, *d_ke = nullptr, *d_pk = nullptr, *d_q = nullptr, *d_s = nullptr;
+    double *d_pairs = nullptr, *d_ke = nullptr, *d_pk = nullptr, *d_q = nullptr, *d_s = nullptr, *d_w2 = nullptr,
+           *d_part = nullptr;
     int *d_mend = nullptr;
     HIPCHK(dalloc((void **)&d_pairs, (size_t)2 * nb * sizeof(double)));
     HIPCHK(dalloc((void **)&d_mend, (size_t)nb * sizeof(int)));
     HIPCHK(dalloc((void **)&d_ke, (size_t)(nk + 1) * sizeof(double)));
     if (deriv) HIPCHK(dalloc((void **)&d_q, (size_t)nb * nk * nv * sizeof(double)));
     if (signal) {
-        HIPCHK(dalloc((void **)&d_pk, (size_t)nz * nmode * sizeof(double)));
+        HIPCHK(dalloc((void **)&d_pk, (size_t)grid.mpad * grid.nzp * sizeof(double)));
+        HIPCHK(dalloc((void **)&d_w2, (size_t)nb * grid.mpad * sizeof(double)));
+        HIPCHK(dalloc((void **)&d_part, (size_t)grid.parts * nb * nv * nz * sizeof(double)));
         HIPCHK(dalloc((void **)&d_s, (size_t)nb * nv * nz * sizeof(double)));
     }
     HIPCHK(hipMemcpy(d_ke, c->kedges.data(), (nk + 1) * sizeof(double), hipMemcpyHostToDevice));
-    if (signal) launch_pfid_grid(c->st, dk, nmode, z1, dz, nz, pd, d_pk);
+    if (signal) launch_pfid_grid(c->st, grid, dk, z1, dz, nz, pd, d_pk);
     std::vector<double> hp(2 * (size_t)nb);
     std::vector<int> hm(nb);
     for (int p0 = 0; p0 < npairs; p0 += nb) {
@@ -1879,16 +1884,23 @@ int qml_make_tables(qml_ctx *c, const qml_table_spec *s, int npairs, const int *
         }
         HIPCHK(hipMemcpyAsync(d_pairs, hp.data(), 2 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, c->st));
         HIPCHK(hipMemcpyAsync(d_mend, hm.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice, c->st));
-        if (deriv) launch_deriv_tables(c->st, d_pairs, n, d_ke, nk, nv, dxv, M, d_q);
+        // the derivative tables are copied on the second stream while the
+        // signal tables are summed
+        if (deriv) {
+            launch_deriv_tables(c->st, d_pairs, n, d_ke, nk, nv, dxv, M, d_q);
+            HIPCHK(hipEventRecord(c->ev_fork, c->st));
+            HIPCHK(hipStreamWaitEvent(c->st2, c->ev_fork, 0));
+        }
         if (signal)
-            launch_signal_tables(c->st, d_pairs, d_mend, n, d_pk, nmode, nhalf, dk, dxv, 1.0 / length, nv, nz, d_s);
+            launch_signal_tables(c->st, grid, d_pairs, d_mend, n, d_pk, dk, 1.0 / length, nv, nz, d_w2, d_part, d_s);
         HIPCHK(hipGetLastError());
         if (deriv)
             HIPCHK(hipMemcpyAsync(deriv + (size_t)p0 * nk * nv, d_q, (size_t)n * nk * nv * sizeof(double),
-                                  hipMemcpyDeviceToHost, c->st));
+                                  hipMemcpyDeviceToHost, c->st2));
         if (signal)
             HIPCHK(hipMemcpyAsync(signal + (size_t)p0 * nv * nz, d_s, (size_t)n * nv * nz * sizeof(double),
                                   hipMemcpyDeviceToHost, c->st));
+        HIPCHK(hipStreamSynchronize(c->st2));
         HIPCHK(hipStreamSynchronize(c->st));
     }
     return QML_OK;

@@ -153,8 +153,18 @@ struct PD13 {
 };
 void launch_deriv_tables(hipStream_t st, const double *pairs, int npairs, const double *kedges, int nk, int nv,
                          double dxv, int M, double *out);
-void launch_pfid_grid(hipStream_t st, double dk, int nmode, double z1, double dz, int nz, PD13 pd, double *pk);
-void launch_signal_tables(hipStream_t st, const double *pairs, const int *mend, int npairs, const double *pk,
-                          int nmode, int nhalf, double dk, double dxv, double inv_len, int nv, int nz, double *out);
+// Layout of the signal sums: the modes 0 .. nhalf padded to mpad rows and the
+// redshifts to nzp columns; parts partial tables per pair.
+struct SignalGrid {
+    int nhalf, mpad, nzp, parts;
+};
+SignalGrid signal_grid(int nhalf, int nz);
+// pk: mpad x nzp
+void launch_pfid_grid(hipStream_t st, const SignalGrid &g, double dk, double z1, double dz, int nz, PD13 pd,
+                      double *pk);
+// w2: npairs x mpad, part: parts x npairs x nv x nz (scratch)
+void launch_signal_tables(hipStream_t st, const SignalGrid &g, const double *pairs, const int *mend, int npairs,
+                          const double *pk, double dk, double inv_len, int nv, int nz, double *w2, double *part,
+                          double *out);
 
 }  // namespace qml
