@@ -22,6 +22,22 @@
 // - cos(k u_b) sin(k u_a): sines and cosines are evaluated once per grid point
 // and edge, not once per grid pair and band.
 //
+// That is the form for any band.  Where the band is narrow on the scale of the
+// chunk's velocities v <= vmax (all practical ones), the window's definition
+//   Qhat_k(v) = 1/pi int_{k_n}^{k_n+1} cos(k v) dk
+// is summed over n Gauss-Legendre nodes instead, exact to 1e-17 of Qhat(0) at
+// n = dk vmax / 4 + O(n^1/3) of them (rmat_nodes), and since v = u_b - u_a,
+//   Q_k = sum_m w_m/pi (R c_m)(R c_m)^T + (R s_m)(R s_m)^T,
+// with c_m, s_m the cosine and sine of k_m u on the fine grid: R is applied to
+// 2 n vectors (k_rm_nodes), and Q_k is the product of an N x 2n matrix with its
+// transpose (k_rm_bands).  The phases k_m u carry both operands' rounding, so
+// that the nodes' errors stay at the rounding of a cosine.  An element of Q_k
+// costs 2 n multiply-adds on the matrix cores (30 to 130 on 100 to 1200 pixels of
+// 55 km/s), against about 800 by the edges, whose taps go through LDS.  160
+// chunks of 100 to 1200 pixels oversampled three times, 29 bands: 37 -> 7 ms
+// (k_rm_nodes 1.8, k_rm_bands 5.1 for 13 GB written), and the largest error
+// against extended precision falls from 1.5e-12 to 2.5e-13 of Q_k's peak.
+//
 // The host lays every R row inside the grid (rcol0 >= 0; a diagonal-storage
 // matrix gets nelem/2 extrapolated grid points on each side, whose weights
 // are zero), so every tap loop below has the same trip count.
@@ -67,7 +83,7 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
         for (int o = 0; o < NO; ++o) {
             const int j = J0 + tj + 16 * o;
             if (j < i) continue;
-            for (int k = 0; k <= kbu; ++k) {
+            for (int k = c.ngrp ? kbu : 0; k <= kbu; ++k) {
                 Qb[k * NN + (size_t)i * Np + j] = 0.0;
                 Qb[k * NN + (size_t)j * Np + i] = 0.0;
             }
@@ -117,6 +133,7 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
     // 1/(pi v) of this thread's entries in every pass (v = u_b - u_a does not
     // depend on the edge); the entry on the shared grid point (v = 0, at most
     // one per pass and column) gets 0 here and k_e/pi written after the rest
+    const int elast = c.ngrp ? -1 : kbu;          // the bands of a chunk with groups come from k_rm_bands
     double inv[NPM][EM];
     int dsel[NPM];
 #pragma unroll
@@ -132,7 +149,7 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
         }
     }
 
-    for (int e = -1; e <= kbu; ++e) {
+    for (int e = -1; e <= elast; ++e) {
         double kpi = 0.0;
         if (e >= 0) {
             const double ke = bins.ke[e];
@@ -252,6 +269,160 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
     }
 }
 
+namespace {
+constexpr int RN_ROWS = 64, RN_NODES = 8;   // rows and nodes of a k_rm_nodes step
+typedef double gd4 __attribute__((ext_vector_type(4)));
+}  // namespace
+
+// V[col + 2m][i] = a_m sum_t R[i][t] cos(k_m u(i, t)), V[col + 2m + 1][i] the
+// sine's: 64 rows of R per workgroup, eight nodes at a time.  The phases of the
+// rows' fine points are evaluated once per node in LDS (a row shares nb - os of
+// its points with the next); a thread then sums the taps of its row for two
+// nodes.  V is stored node by node, so that both sides of k_rm_bands read it
+// along i.  Rows past N have no weights and give zeros.  Bound by the LDS reads
+// of the taps.
+__global__ __launch_bounds__(256) void k_rm_nodes(const ChunkDev *cs, const double *rin, const RmBand *bands,
+                                                  const RmNode *nodes, int grp, double *mat) {
+    const ChunkDev c = cs[blockIdx.z];
+    const int I0 = blockIdx.x * RN_ROWS, k = blockIdx.y;
+    if (!c.ngrp || k >= c.kbu || I0 >= c.Np) return;
+    const RmBand b = bands[c.rmb_off + k];
+    if (b.grp != grp) return;
+    const int N = c.N, M = c.rM, nb = c.rnb, os = c.ros, ra = (RN_ROWS - 1) * os + nb;
+    const int amin = c.rcol0 + I0 * os;
+    const double *R = rin + c.rin_off, *grid = R + (size_t)N * nb;
+    extern __shared__ double lds[];
+    double2 *cs2 = reinterpret_cast<double2 *>(lds);   // RN_NODES x ra
+    double *Ri = lds + 2 * RN_NODES * ra;              // RN_ROWS x nb
+    double *ush = Ri + RN_ROWS * nb;                   // ra
+    const int tid = threadIdx.x;
+    for (int e = tid; e < RN_ROWS * nb; e += 256) {
+        const int r = e / nb;
+        Ri[e] = (I0 + r < N) ? R[(size_t)I0 * nb + e] : 0.0;
+    }
+    const double gref = grid[M / 2];
+    // log1p of the difference: u to its own rounding, where a rounded ratio leaves c eps
+    for (int p = tid; p < ra; p += 256)
+        ush[p] = SPEED_OF_LIGHT * log1p((grid[min(M - 1, amin + p)] - gref) / gref);
+    __syncthreads();
+    const int row = tid & 63, q = tid >> 6;
+    const double *w = Ri + row * nb;
+    const double2 *x0 = cs2 + q * ra + row * os, *x1 = x0 + (RN_NODES / 2) * ra;
+    double *V = mat + c.mat_off + (size_t)b.col * c.Np + I0 + row;
+    const RmNode *nd = nodes + b.node;
+    for (int m0 = 0; m0 < b.n; m0 += RN_NODES) {
+        for (int e = tid; e < RN_NODES * ra; e += 256) {
+            const int m = e / ra;
+            const RmNode x = nd[m0 + m];
+            const double u = ush[e - m * ra], p = x.kh * u, d = __builtin_fma(x.kh, u, -p) + x.kl * u;
+            double sv, cv;
+            sincos(p, &sv, &cv);
+            cs2[e] = make_double2(cv - d * sv, sv + d * cv);
+        }
+        __syncthreads();
+        double c0 = 0.0, s0 = 0.0, c1 = 0.0, s1 = 0.0;
+        for (int t = 0; t < nb; ++t) {
+            const double r = w[t];
+            const double2 y0 = x0[t], y1 = x1[t];
+            c0 += r * y0.x;
+            s0 += r * y0.y;
+            c1 += r * y1.x;
+            s1 += r * y1.y;
+        }
+        const int m = m0 + q;
+        const double a0 = nd[m].a, a1 = nd[m + RN_NODES / 2].a;
+        V[(size_t)(2 * m) * c.Np] = a0 * c0;
+        V[(size_t)(2 * m + 1) * c.Np] = a0 * s0;
+        V[(size_t)(2 * m + RN_NODES) * c.Np] = a1 * c1;
+        V[(size_t)(2 * m + RN_NODES + 1) * c.Np] = a1 * s1;
+        __syncthreads();
+    }
+}
+
+// Q_k = V^T V over the band's 2n rows of V: one upper 64 x 64 tile per
+// workgroup, a 32 x 32 quarter per wave, written to both triangles.  A lane
+// loads two neighbouring i of one row of V, which are the operands of two
+// 16-row blocks (block x holds the rows i0 + 2 r + x), straight from L1 and L2:
+// two 16-byte loads feed four MFMAs, so LDS would only add its barriers.  The
+// loads of the next 16 rows are issued before the products of these.
+__global__ __launch_bounds__(256) void k_rm_bands(const ChunkDev *cs, const RmBand *bands, int grp, double *mat) {
+    const ChunkDev c = cs[blockIdx.z];
+    const int k = blockIdx.y, x = blockIdx.x;
+    if (!c.ngrp || k >= c.kbu || x >= c.ntu) return;
+    const RmBand b = bands[c.rmb_off + k];
+    if (b.grp != grp) return;
+    // tile x of the upper triangle, column by column
+    int J = (int)((sqrtf(8.0f * x + 1.0f) - 1.0f) * 0.5f);
+    while (J * (J + 1) / 2 > x) --J;
+    while ((J + 1) * (J + 2) / 2 <= x) ++J;
+    const int I = x - J * (J + 1) / 2;
+    const int Np = c.Np, tid = threadIdx.x, lane = tid % 64, lr = lane % 16, lq = lane / 16;
+    const int wv = __builtin_amdgcn_readfirstlane(tid / 64), wm = wv / 2, wn = wv % 2;
+    if (I == J && wm > wn) return;   // the mirror image of quarter (0, 1)
+    const int r0 = I * TILE + 32 * wm, c0 = J * TILE + 32 * wn;
+    const double *V = mat + c.mat_off + (size_t)(b.col + lq) * Np + 2 * lr;
+    const size_t step = (size_t)4 * Np;
+    gd4 acc[2][2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int f = 0; f < 2; ++f) acc[e][f] = gd4{0.0, 0.0, 0.0, 0.0};
+    dvec2 na[4], nb[4];
+    auto fetch = [&](int s) {
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            na[h] = *(GlobalD2 *)(V + (4 * s + h) * step + r0);
+            nb[h] = *(GlobalD2 *)(V + (4 * s + h) * step + c0);
+        }
+        asm volatile("" ::: "memory");   // issued here, not where the values are first needed
+    };
+    const int ns = b.n / 8;   // 16 rows of V each
+    fetch(0);
+    for (int s = 0; s < ns; ++s) {
+        dvec2 a[4], d[4];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            a[h] = na[h];
+            d[h] = nb[h];
+        }
+        if (s + 1 < ns) fetch(s + 1);
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int f = 0; f < 2; ++f)
+                    acc[e][f] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[h][e], d[h][f], acc[e][f], 0, 0, 0);
+    }
+    double *Q = mat + c.qb_off + (size_t)k * Np * Np;
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            *(dvec2 *)(Q + (size_t)(r0 + 8 * u + 2 * lq + e) * Np + c0 + 2 * lr) = dvec2{acc[e][0][u], acc[e][1][u]};
+    if (r0 == c0) return;   // symmetric in itself
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            *(dvec2 *)(Q + (size_t)(c0 + 2 * lr + f) * Np + r0 + 8 * u + 2 * lq) = dvec2{acc[0][f][u], acc[1][f][u]};
+}
+
+size_t rmat_node_lds(int os, int nb) {
+    const size_t ra = (RN_ROWS - 1) * os + nb;
+    return 8 * (2 * RN_NODES * ra + RN_ROWS * nb + ra);   // at most 61 KB under 15 os + nb <= RM_ROWS
+}
+
+int rmat_nodes(double dk, double vmax) {
+    // n nodes integrate cos(x t) over [-1, 1] to 1e-17 up to x = 2 (n - 8.75 n^(1/3) + 9.6)
+    // (found from n = 8 to 256); beyond 256 nodes the edges cost no more
+    const double x = 0.5 * dk * vmax;
+    if (!(dk > 0 && vmax >= 0)) return 0;
+    for (int n = 8; n <= 256; n += 8)
+        if (x <= 2.0 * (n - 8.75 * std::cbrt((double)n) + 9.6)) return n;
+    return 0;
+}
+
 RmLayout rmat_layout(int tj, int ra_max, int rb_max, int nb_max) {
     RmLayout l;
     const int npass = (rb_max + RM_BW - 1) / RM_BW;
@@ -284,6 +455,13 @@ bool launch_rmat(const LaunchCtx &L) {
         k_rm_sandwich<16, RM_ROWS / 8, 3><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.tables, L.bins, lay, L.mat);
     else
         return false;
+    const int nt = L.np_max / TILE;
+    for (int gr = 0; gr < L.rm_groups; ++gr) {
+        k_rm_nodes<<<dim3(L.np_max / RN_ROWS, L.rm_kbu, L.nchunks), 256, L.rm_lds, L.stream>>>(
+            L.chunks, L.rin, L.rm_bands, L.rm_nodes, gr, L.mat);
+        k_rm_bands<<<dim3(nt * (nt + 1) / 2, L.rm_kbu, L.nchunks), 256, 0, L.stream>>>(L.chunks, L.rm_bands, gr,
+                                                                                       L.mat);
+    }
     return true;
 }
 

@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <numeric>
 #include <string>
 #include <vector>
@@ -54,6 +55,7 @@ struct ChunkHost {
     int rdia = 0;   // the matrix came in diagonal storage (its grid is the pixels')
     std::vector<double> rband, fine;
     long long rin_off = 0;
+    int ngrp = 0, rmb_off = 0;   // quadrature of its Q_k (see ChunkDev)
 };
 
 struct Batch {
@@ -71,6 +73,8 @@ struct Batch {
     int nq_max = 0;             // most N_Q_MATRICES of a chunk in the batch
     int rm_kbu = -1;   // resolution-matrix chunks: largest KBIN_UPP
     RmLayout rm_lay;   // and the LDS layout of their sandwich launch
+    int rm_groups = 0;        // quadrature: most band groups
+    size_t rm_lds = 0;        // and the LDS of the node launch
     hipEvent_t evA[7]{};   // stage A (assembly .. solves) on stream st
     hipEvent_t evB[6]{};   // stage B (stack generation .. Gram) on stream st2
     hipEvent_t evR{};      // after the resolution-matrix sandwiches (stage A)
@@ -198,6 +202,8 @@ struct qml_ctx {
     double max_chunk_bytes = 0;   // the largest chunk's scratch in the current plan
     double *d_theta = nullptr, *d_F = nullptr, *d_dbtsum = nullptr;
     double *d_rin = nullptr;   // resolution-matrix rows and fine grids
+    RmBand *d_rmb = nullptr;   // their bands' quadrature in k
+    RmNode *d_rmn = nullptr;
     std::vector<Batch> batches;
     hipEvent_t ev_begin{}, ev_end{}, ev_acc{};
     hipEvent_t ev_fork{}, ev_join{};   // order stage B's stream inside one iteration
@@ -277,7 +283,7 @@ int qml_destroy(qml_ctx *c) {
     for (auto &t : c->tables) { hipFree(t.d_qt); hipFree(t.d_q2); hipFree(t.d_s); }
     release_plan(c);
     void *ptrs[] = {c->d_tables, c->d_in, c->d_outs, c->d_fc, c->d_dbt, c->d_status, c->d_skip,
-                    c->d_theta, c->d_F, c->d_dbtsum, c->d_rin};
+                    c->d_theta, c->d_F, c->d_dbtsum, c->d_rin, c->d_rmb, c->d_rmn};
     for (void *p : ptrs) if (p) hipFree(p);
     if (c->ev_begin) hipEventDestroy(c->ev_begin);
     if (c->ev_end) hipEventDestroy(c->ev_end);
@@ -650,6 +656,95 @@ void release_plan(qml_ctx *c) {
     c->d_X = c->d_Y = c->d_G = nullptr;
 }
 
+// Gauss-Legendre nodes and weights on [-1, 1], by Newton's method on the
+// three-term recurrence from the asymptotic roots: in double precision to
+// convergence, then one step and the weight in long double.
+template <class T>
+T legendre(int n, T t, T &dp) {
+    T p0 = 1, p1 = t;
+    for (int j = 2; j <= n; ++j) {
+        const T p2 = t * p1 + (t * p1 - p0) * ((T)(j - 1) / j);
+        p0 = p1;
+        p1 = p2;
+    }
+    dp = n * (t * p1 - p0) / (t * t - 1);
+    return p1;
+}
+void gauss_legendre(int n, std::vector<long double> &x, std::vector<long double> &w) {   // n even
+    x.resize(n);
+    w.resize(n);
+    for (int i = 0; i < n / 2; ++i) {
+        double t = std::cos(M_PI * (i + 0.75) / (n + 0.5)), d;
+        for (int it = 0; it < 6; ++it) {
+            const double dt = legendre(n, t, d) / d;
+            t -= dt;
+            if (std::fabs(dt) < 1e-14) break;
+        }
+        long double y = t, dp;
+        y -= legendre(n, y, dp) / dp;
+        legendre(n, y, dp);
+        x[i] = y;
+        x[n - 1 - i] = -y;
+        w[i] = w[n - 1 - i] = 2 / ((1 - y * y) * dp * dp);
+    }
+}
+
+// The quadrature in k of every resolution-matrix chunk's bands: node counts
+// from the chunk's velocity range, and the bands packed into groups whose node
+// matrices fit the 4 Np columns of the A, L, Li and S slots, free until the
+// chunk's assembly.  A chunk with a band of more nodes keeps to the band edges.
+int plan_quadrature(qml_ctx *c) {
+    std::vector<RmBand> bands;
+    std::vector<RmNode> nodes;
+    std::map<std::pair<int, int>, int> at;   // (band, n) -> nodes
+    std::map<int, std::pair<std::vector<long double>, std::vector<long double>>> rule;
+    for (auto &ch : c->chunks) {
+        ch.ngrp = 0;
+        if (!ch.rm || ch.kbu < 1) continue;
+        const auto mm = std::minmax_element(ch.fine.begin(), ch.fine.end());
+        if (!(*mm.first > 0 && std::isfinite(*mm.second))) continue;
+        const double vmax = SPEED_OF_LIGHT * std::log(*mm.second / *mm.first);
+        std::vector<RmBand> bs;
+        int grp = 0, col = 0;
+        for (int k = 0; k < ch.kbu; ++k) {
+            const int n = rmat_nodes(c->kedges[k + 1] - c->kedges[k], vmax);
+            if (n == 0 || 2 * n > 4 * ch.Np) break;
+            if (col + 2 * n > 4 * ch.Np) {
+                ++grp;
+                col = 0;
+            }
+            bs.push_back({grp, col, n, 0});
+            col += 2 * n;
+        }
+        if ((int)bs.size() < ch.kbu) continue;
+        for (int k = 0; k < ch.kbu; ++k) {
+            const auto f = at.emplace(std::make_pair(k, bs[k].n), (int)nodes.size());
+            bs[k].node = f.first->second;
+            if (!f.second) continue;
+            auto &r = rule[bs[k].n];
+            if (r.first.empty()) gauss_legendre(bs[k].n, r.first, r.second);
+            const long double k0 = c->kedges[k], k1 = c->kedges[k + 1];
+            for (int m = 0; m < bs[k].n; ++m) {
+                const long double kn = (k0 + k1 + (k1 - k0) * r.first[m]) / 2;
+                RmNode nd;
+                nd.kh = (double)kn;
+                nd.kl = (double)(kn - nd.kh);
+                nd.a = (double)std::sqrt((k1 - k0) / 2 * r.second[m] / 3.14159265358979323846264338328L);
+                nodes.push_back(nd);
+            }
+        }
+        ch.ngrp = grp + 1;
+        ch.rmb_off = (int)bands.size();
+        bands.insert(bands.end(), bs.begin(), bs.end());
+    }
+    if (bands.empty()) return QML_OK;
+    HIPCHK(hipMalloc(&c->d_rmb, bands.size() * sizeof(RmBand)));
+    HIPCHK(hipMemcpy(c->d_rmb, bands.data(), bands.size() * sizeof(RmBand), hipMemcpyHostToDevice));
+    HIPCHK(hipMalloc(&c->d_rmn, nodes.size() * sizeof(RmNode)));
+    HIPCHK(hipMemcpy(c->d_rmn, nodes.data(), nodes.size() * sizeof(RmNode), hipMemcpyHostToDevice));
+    return QML_OK;
+}
+
 // Size-bucketed batch plan: chunks sorted by padded size (then stored Q
 // count), descending, are cut into batches of at most c->max_batch chunks
 // whose scratch fits c->scratch_gb; allocates the arenas of the largest
@@ -733,6 +828,8 @@ int plan_batches(qml_ctx *c) {
             d.rM = ch.rM;
             d.rin_off = ch.rin_off;
             d.qb_off = (long long)(acc.mat + 4 * (size_t)ch.Np * ch.Np);
+            d.ngrp = ch.ngrp;
+            d.rmb_off = ch.rmb_off;
             acc.mat += n.mat; acc.vec += n.vec; acc.pj += n.pj; acc.sj += n.sj;
             acc.stk += n.stk; acc.lic += n.lic; acc.gram += n.gram; acc.g += n.g;
             c->max_chunk_bytes = std::max(c->max_chunk_bytes, (double)bytes(n));
@@ -794,6 +891,8 @@ int plan_batches(qml_ctx *c) {
                 ra_max = std::max(ra_max, 15 * d.ros + d.rnb);
                 rb_max = std::max(rb_max, 31 * d.ros + d.rnb);
                 nb_max = std::max(nb_max, d.rnb);
+                B.rm_groups = std::max(B.rm_groups, d.ngrp);
+                B.rm_lds = std::max(B.rm_lds, rmat_node_lds(d.ros, d.rnb));
             }
             const int g = (c->prec >= 2) ? 2 : 1;
             const int mtg = (d.mt + g - 1) / g;
@@ -954,6 +1053,8 @@ int qml_commit(qml_ctx *c) {
             HIPCHK(hipMalloc(&c->d_rin, rin_total * sizeof(double)));
             HIPCHK(hipMemcpy(c->d_rin, hr.data(), rin_total * sizeof(double), hipMemcpyHostToDevice));
         }
+        const int rc = plan_quadrature(c);
+        if (rc != QML_OK) return rc;
     }
     HIPCHK(hipMalloc(&c->d_outs, std::max(nch, 1) * sizeof(ChunkOut)));
     if (nch) HIPCHK(hipMemcpy(c->d_outs, c->outs.data(), nch * sizeof(ChunkOut), hipMemcpyHostToDevice));
@@ -1007,6 +1108,10 @@ LaunchCtx batch_launch(const qml_ctx *c, size_t bi) {
     L.rin = c->d_rin;
     L.rm_kbu = B.rm_kbu;
     L.rm_lay = B.rm_lay;
+    L.rm_groups = B.rm_groups;
+    L.rm_lds = B.rm_lds;
+    L.rm_bands = c->d_rmb;
+    L.rm_nodes = c->d_rmn;
     L.in = c->d_in;
     L.tables = c->d_tables;
     L.bins = c->binsdev;

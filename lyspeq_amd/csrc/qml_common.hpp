@@ -84,6 +84,19 @@ struct ChunkDev {
     int rm, rnb, ros, rcol0, rM;
     long long rin_off;   // into the resolution-matrix input arena (doubles)
     long long qb_off;    // into the FP64 matrix arena
+    // the Q_k by quadrature in k: band groups (0: by band edges) and the
+    // chunk's kbu entries of the RmBand list
+    int ngrp, rmb_off;
+};
+
+// One band of a chunk whose Q_k are summed over n nodes in k: columns
+// [col, col + 2 n) of the node matrix that its group shares, RmNode list at node.
+struct RmBand {
+    int grp, col, n, node;
+};
+struct RmNode {
+    double kh, kl;   // the wavenumber, as a sum
+    double a;        // sqrt of its weight
 };
 // A double in the global address space: loads through it are global_load,
 // counted by vmcnt only (a flat load would also hold up the LDS waits).
