@@ -8,8 +8,8 @@
 // with v, z taken on the matrix's grid (core/chunk_estimate.cpp:384-480,
 // mathtools/matrix_helper.cpp:877-902,1075-1084), then applies the z-bin
 // weights on the pixel grid.  Here S and every Q_k (k < KBIN_UPP) are
-// materialised once per iteration in the chunk's FP64 matrix arena (qb_off)
-// by one launch over the whole batch.
+// materialised once per iteration in the chunk's FP64 matrix arena (qb_off),
+// over the whole batch at a time.
 //
 // The band window is a difference of edge terms: with the band edges
 // k_n, k_n+1 (k_c their mean, dk their difference),
@@ -42,11 +42,14 @@
 // matrix gets nelem/2 extrapolated grid points on each side, whose weights
 // are zero), so every tap loop below has the same trip count.
 //
+// S is formed by k_rm_signal, unless R's rows are too long for its LDS (more than
+// about 55 taps): then it is k_rm_sandwich's first pass, for every chunk.
+//
 // k_rm_sandwich<TJ>: one 16 x TJ output tile (I0.., J0..) per block, tiles
 // touching the upper triangle only.  The fine rows of its 16 R rows (the a
 // range, 15 ros + rnb) and the fine columns of its TJ R columns (the b range,
 // (TJ-1) ros + rnb, in passes of 32) are fixed for the block.  Per edge e
-// (and first for S):
+// (and first for S, where asked):
 //   per pass:  Qh (a x 32, LDS) <- P_e(a, b), or Shat
 //              T  (16 x b, LDS) <- R_I Qh                  (rnb taps, FP64 FMA)
 //   Z[i][j] = sum_t T[i][j ros + t] R[j][t]                (rnb taps, registers)
@@ -66,12 +69,12 @@ constexpr int RM_QP = 33;    // row pitch of Qh (doubles)
 
 template <int TJ, int EM, int NPM>
 __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const double *rin, const TableDev *tabs,
-                                                     BinsDev bins, RmLayout lay, double *mat) {
+                                                     BinsDev bins, RmLayout lay, int signal, double *mat) {
     constexpr int NO = TJ / 16;                   // outputs per thread
     // EM: Qh entries per thread (rows ar0 + 8 s, s < EM); 8 EM >= 15 ros + rnb.
     // NPM: passes at most ((TJ - 1) ros + rnb <= 32 NPM), their 1/(pi v) kept in registers
     const ChunkDev c = cs[blockIdx.z];
-    if (!c.rm) return;
+    if (!c.rm || (c.ngrp && !signal)) return;
     const int Np = c.Np, N = c.N, M = c.rM, nb = c.rnb, os = c.ros, kbu = c.kbu;
     const int I0 = blockIdx.y * 16, J0 = blockIdx.x * TJ;
     if (I0 >= Np || J0 >= Np || J0 + TJ - 1 < I0) return;
@@ -83,7 +86,7 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
         for (int o = 0; o < NO; ++o) {
             const int j = J0 + tj + 16 * o;
             if (j < i) continue;
-            for (int k = c.ngrp ? kbu : 0; k <= kbu; ++k) {
+            for (int k = c.ngrp ? kbu : 0; k < kbu + signal; ++k) {
                 Qb[k * NN + (size_t)i * Np + j] = 0.0;
                 Qb[k * NN + (size_t)j * Np + i] = 0.0;
             }
@@ -149,7 +152,7 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
         }
     }
 
-    for (int e = -1; e <= elast; ++e) {
+    for (int e = signal ? -1 : 0; e <= elast; ++e) {
         double kpi = 0.0;
         if (e >= 0) {
             const double ke = bins.ke[e];
@@ -272,6 +275,8 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
 namespace {
 constexpr int RN_ROWS = 64, RN_NODES = 8;   // rows and nodes of a k_rm_nodes step
 typedef double gd4 __attribute__((ext_vector_type(4)));
+// k_rm_signal's row pitch of R in LDS: 16 rows read at columns os apart fall on distinct banks
+__host__ __device__ inline int signal_pitch(int os, int nb) { return nb + ((nb - os) % 2 == 0); }
 }  // namespace
 
 // V[col + 2m][i] = a_m sum_t R[i][t] cos(k_m u(i, t)), V[col + 2m + 1][i] the
@@ -408,6 +413,109 @@ __global__ __launch_bounds__(256) void k_rm_bands(const ChunkDev *cs, const RmBa
             *(dvec2 *)(Q + (size_t)(c0 + 2 * lr + f) * Np + r0 + 8 * u + 2 * lq) = dvec2{acc[0][f][u], acc[1][f][u]};
 }
 
+// S = R Shat R^T: one upper 64 x 64 tile per workgroup, a 32 x 32 quarter per
+// wave, on the matrix cores without an intermediate in LDS.  For 16 fine columns
+// b at a time, each lane evaluates the signal at the (b, a) it holds as the first
+// operand of T^T = Shat^T R_I^T; the accumulator of T^T is laid out as the second
+// operand of S^T += R_J T^T.  A quarter evaluates 31 ros + rnb points a side, 1.7
+// times its own.  u and sqrt(lambda), in units of the table's steps, are formed
+// once per point, so that v and z are a difference and a product.  Bound by the
+// gathers of the table, two 16-byte rows a point.  160 chunks of 100 to 1200
+// pixels oversampled three times: 12.7 -> 1.7 ms (as the first pass of
+// k_rm_sandwich, whose registers leave two waves per SIMD to hide them), error
+// against extended precision 4e-14 -> 1.3e-15 of S's peak.
+__global__ __launch_bounds__(256) void k_rm_signal(const ChunkDev *cs, const double *rin, const TableDev *tabs,
+                                                   BinsDev bins, double *mat) {
+    typedef const double __attribute__((ext_vector_type(2), aligned(8), address_space(1))) GlobalD2u;
+    const ChunkDev c = cs[blockIdx.y];
+    const int x = blockIdx.x;
+    if (!c.rm || x >= c.ntu) return;
+    int J = (int)((sqrtf(8.0f * x + 1.0f) - 1.0f) * 0.5f);
+    while (J * (J + 1) / 2 > x) --J;
+    while ((J + 1) * (J + 2) / 2 <= x) ++J;
+    const int I = x - J * (J + 1) / 2;
+    const int Np = c.Np, N = c.N, M = c.rM, nb = c.rnb, os = c.ros;
+    const int pitch = signal_pitch(os, nb), npt = (TILE - 1) * os + nb + 16;
+    const double *R = rin + c.rin_off, *grid = R + (size_t)N * nb;
+    const TableDev t = tabs[c.table];
+    const int amin = c.rcol0 + I * TILE * os, bmin = c.rcol0 + J * TILE * os;
+    extern __shared__ double lds[];
+    double2 *pa = reinterpret_cast<double2 *>(lds), *pb = pa + npt;   // (u / dv, sqrt(lambda / dz))
+    double *Ri = lds + 4 * npt, *Rj = Ri + TILE * pitch;
+    const int tid = threadIdx.x, lane = tid % 64, lr = lane % 16, lq = lane / 16;
+    for (int e = tid; e < TILE * nb; e += 256) {
+        const int r = e / nb, o = r * pitch + (e - r * nb);
+        Ri[o] = (I * TILE + r < N) ? R[(size_t)I * TILE * nb + e] : 0.0;
+        Rj[o] = (J * TILE + r < N) ? R[(size_t)J * TILE * nb + e] : 0.0;
+    }
+    const double gref = grid[min(M - 1, (amin + bmin + npt) / 2)], rdz = sqrt(t.dz);
+    for (int p = tid; p < 2 * npt; p += 256) {
+        const double l = grid[min(M - 1, p < npt ? amin + p : bmin + p - npt)];
+        pa[p] = make_double2(SPEED_OF_LIGHT * log1p((l - gref) / gref) / t.dv, sqrt(l) / rdz);
+    }
+    __syncthreads();
+    const int wv = __builtin_amdgcn_readfirstlane(tid / 64), wm = wv / 2, wn = wv % 2;
+    if (I == J && wm > wn) return;   // the mirror image of quarter (0, 1)
+    const int a0 = 32 * wm * os, b0 = 32 * wn * os, ra = 31 * os + nb;
+    const int ns = bins.turn_off_sfid ? 0 : (ra + 3) / 4, nbb = bins.turn_off_sfid ? 0 : (ra + 15) / 16;
+    const double v0 = t.v1 / t.dv, z0 = (1.0 + t.z1) / t.dz;
+    const double *ri0 = Ri + (32 * wm + lr) * pitch, *ri1 = ri0 + 16 * pitch;
+    const double *rj0 = Rj + (32 * wn + lr) * pitch, *rj1 = rj0 + 16 * pitch;
+    auto tap = [&](const double *row, int p) {   // the row's weight at its point p, 0 past its ends
+        const double w = row[min((unsigned)p, (unsigned)(nb - 1))];
+        return (unsigned)p < (unsigned)nb ? w : 0.0;
+    };
+    gd4 z[2][2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int f = 0; f < 2; ++f) z[e][f] = gd4{0.0, 0.0, 0.0, 0.0};
+    for (int q = 0; q < nbb; ++q) {
+        const int bl = b0 + 16 * q + lr;
+        const double2 wb = pb[bl];
+        gd4 t0 = {0.0, 0.0, 0.0, 0.0}, t1 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+        for (int s = 0; s < ns; ++s) {
+            const int al = 4 * s + lq;
+            const double2 wa = pa[a0 + al];
+            const double yy = ((bmin + bl >= amin + a0 + al) ? wb.x - wa.x : wa.x - wb.x) - v0;
+            const double xx = wa.y * wb.y - z0;
+            const int nx = interp_index(xx, t.nz), ny = interp_index(yy, t.nv);
+            const double *p = t.s + ((size_t)nx + (size_t)t.nz * ny);
+            const dvec2 lo = *(GlobalD2u *)p, hi = *(GlobalD2u *)(p + t.nz);
+            const double dx = xx - nx, dy = yy - ny;
+            const double val = (lo.x * (1 - dx) + lo.y * dx) * (1 - dy) + (hi.x * (1 - dx) + hi.y * dx) * dy;
+            t0 = __builtin_amdgcn_mfma_f64_16x16x4f64(val, tap(ri0, al - lr * os), t0, 0, 0, 0);
+            t1 = __builtin_amdgcn_mfma_f64_16x16x4f64(val, tap(ri1, al - (16 + lr) * os), t1, 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int b = 16 * q + 4 * u + lq;
+            const double w0 = tap(rj0, b - lr * os), w1 = tap(rj1, b - (16 + lr) * os);
+            z[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(w0, t0[u], z[0][0], 0, 0, 0);
+            z[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(w1, t0[u], z[0][1], 0, 0, 0);
+            z[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(w0, t1[u], z[1][0], 0, 0, 0);
+            z[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(w1, t1[u], z[1][1], 0, 0, 0);
+        }
+    }
+    double *S = mat + c.qb_off + (size_t)c.kbu * Np * Np;
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = I * TILE + 32 * wm + 16 * e + lr, j = J * TILE + 32 * wn + 16 * f + 4 * u + lq;
+                if (j < i) continue;
+                S[(size_t)j * Np + i] = z[e][f][u];
+                S[(size_t)i * Np + j] = z[e][f][u];
+            }
+}
+
+size_t rmat_signal_lds(int os, int nb) {
+    return 8 * (4 * ((size_t)(TILE - 1) * os + nb + 16) + 2 * TILE * signal_pitch(os, nb));
+}
+
 size_t rmat_node_lds(int os, int nb) {
     const size_t ra = (RN_ROWS - 1) * os + nb;
     return 8 * (2 * RN_NODES * ra + RN_ROWS * nb + ra);   // at most 61 KB under 15 os + nb <= RM_ROWS
@@ -446,16 +554,24 @@ bool rmat_layout_ok(const RmLayout &lay) {
 bool launch_rmat(const LaunchCtx &L) {
     if (L.rm_kbu < 0) return true;
     const RmLayout &lay = L.rm_lay;
-    const dim3 g(L.np_max / lay.tj, L.np_max / 16, L.nchunks);
-    if (lay.tj == 32 && lay.em == 10 && lay.npass <= 4)
-        k_rm_sandwich<32, 10, 4><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.tables, L.bins, lay, L.mat);
-    else if (lay.tj == 16 && lay.em == 10 && lay.npass <= 3)
-        k_rm_sandwich<16, 10, 3><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.tables, L.bins, lay, L.mat);
-    else if (lay.tj == 16 && lay.em == RM_ROWS / 8 && lay.npass <= 3)
-        k_rm_sandwich<16, RM_ROWS / 8, 3><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.tables, L.bins, lay, L.mat);
-    else
-        return false;
-    const int nt = L.np_max / TILE;
+    const int nt = L.np_max / TILE, signal = L.rm_sig_lds == 0;   // S with the edges' kernel
+    if (!signal)
+        k_rm_signal<<<dim3(nt * (nt + 1) / 2, L.nchunks), 256, L.rm_sig_lds, L.stream>>>(L.chunks, L.rin, L.tables,
+                                                                                         L.bins, L.mat);
+    if (signal || L.rm_edges) {
+        const dim3 g(L.np_max / lay.tj, L.np_max / 16, L.nchunks);
+        if (lay.tj == 32 && lay.em == 10 && lay.npass <= 4)
+            k_rm_sandwich<32, 10, 4><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.tables, L.bins, lay, signal,
+                                                                      L.mat);
+        else if (lay.tj == 16 && lay.em == 10 && lay.npass <= 3)
+            k_rm_sandwich<16, 10, 3><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.tables, L.bins, lay, signal,
+                                                                      L.mat);
+        else if (lay.tj == 16 && lay.em == RM_ROWS / 8 && lay.npass <= 3)
+            k_rm_sandwich<16, RM_ROWS / 8, 3><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.tables, L.bins, lay,
+                                                                               signal, L.mat);
+        else
+            return false;
+    }
     for (int gr = 0; gr < L.rm_groups; ++gr) {
         k_rm_nodes<<<dim3(L.np_max / RN_ROWS, L.rm_kbu, L.nchunks), 256, L.rm_lds, L.stream>>>(
             L.chunks, L.rin, L.rm_bands, L.rm_nodes, gr, L.mat);

@@ -73,6 +73,8 @@ struct Batch {
     int nq_max = 0;             // most N_Q_MATRICES of a chunk in the batch
     int rm_kbu = -1;   // resolution-matrix chunks: largest KBIN_UPP
     RmLayout rm_lay;   // and the LDS layout of their sandwich launch
+    int rm_edges = 0;         // whether one of them takes its Q_k from the band edges
+    size_t rm_sig_lds = 0;    // LDS of the signal launch, 0 if it is too large
     int rm_groups = 0;        // quadrature: most band groups
     size_t rm_lds = 0;        // and the LDS of the node launch
     hipEvent_t evA[7]{};   // stage A (assembly .. solves) on stream st
@@ -891,6 +893,8 @@ int plan_batches(qml_ctx *c) {
                 ra_max = std::max(ra_max, 15 * d.ros + d.rnb);
                 rb_max = std::max(rb_max, 31 * d.ros + d.rnb);
                 nb_max = std::max(nb_max, d.rnb);
+                B.rm_edges |= d.ngrp == 0;
+                B.rm_sig_lds = std::max(B.rm_sig_lds, rmat_signal_lds(d.ros, d.rnb));
                 B.rm_groups = std::max(B.rm_groups, d.ngrp);
                 B.rm_lds = std::max(B.rm_lds, rmat_node_lds(d.ros, d.rnb));
             }
@@ -906,6 +910,7 @@ int plan_batches(qml_ctx *c) {
         }
         xg.flush(wg);
         if (B.rm_kbu >= 0) {
+            if (B.rm_sig_lds > 65536) B.rm_sig_lds = 0;   // rows of more than about 55 taps
             // 16 x 32 output tiles where their LDS fits in 64 KB, their a range
             // in 80 rows and their b range in 4 passes; else 16 x 16 (which
             // always fits under the registration limit on 15 ros + rnb)
@@ -1108,6 +1113,8 @@ LaunchCtx batch_launch(const qml_ctx *c, size_t bi) {
     L.rin = c->d_rin;
     L.rm_kbu = B.rm_kbu;
     L.rm_lay = B.rm_lay;
+    L.rm_edges = B.rm_edges;
+    L.rm_sig_lds = B.rm_sig_lds;
     L.rm_groups = B.rm_groups;
     L.rm_lds = B.rm_lds;
     L.rm_bands = c->d_rmb;

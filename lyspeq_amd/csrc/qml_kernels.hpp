@@ -15,8 +15,10 @@ struct RmLayout {
 // Layout for output tiles of 16 x tj and the batch's largest a range
 // (15 ros + rnb), b range ((tj - 1) ros + rnb) and rnb.
 RmLayout rmat_layout(int tj, int ra_max, int rb_max, int nb_max);
-// LDS bytes of the node kernel for a chunk with this oversampling and row length.
+// LDS bytes of the node kernel for a chunk with this oversampling and row length,
 size_t rmat_node_lds(int os, int nb);
+// and of the signal kernel.
+size_t rmat_signal_lds(int os, int nb);
 // Nodes of the quadrature over a band of width dk at velocities up to vmax
 // (a multiple of 8), or 0 where the band edges are used.
 int rmat_nodes(double dk, double vmax);
@@ -44,6 +46,8 @@ struct LaunchCtx {
     const double *rin;        // R rows and fine grids
     int rm_kbu;               // largest KBIN_UPP of the batch's resolution-matrix chunks; -1 if none
     RmLayout rm_lay;          // LDS layout of the batch's sandwich launch
+    int rm_edges;             // whether one of them has its Q_k by the band edges
+    size_t rm_sig_lds;        // LDS of the signal launch, 0 if it is too large for it
     int rm_groups;            // most band groups of a chunk in the batch
     size_t rm_lds;            // LDS of the batch's node launch
     const RmBand *rm_bands;
