@@ -312,8 +312,17 @@ typedef double dq4 __attribute__((ext_vector_type(4)));
 // work has no branches; blocks past a chunk's own counts are zero.  The table
 // rows of a K step (4 columns) are gathered two steps ahead into two named
 // register sets, so their latency overlaps the two intervening steps.
+// What bounds it is the issue of both kinds: a step's MFMAs (64 cycles) and its 35
+// other instructions (4) add up, and the vector work of the pixel pairs (log,
+// sqrt, weights) is a quarter more.  So the steps carry no tests, and address by
+// one add a block.  640 table chunks of 150 to 700 pixels: 9.9 -> 8.5 ms;
+// materialised matrices, read 16 bytes a lane and a load ahead: 6.3 -> 4.7 ms on
+// 160 chunks of 100 to 1200.  (Waves staggered to stand at one separation, so that
+// their gathers meet in L1: no difference.)  Three waves per SIMD up to four
+// accumulator blocks, even where a few registers spill (4 x 1: 2.8 -> 2.6 ms on
+// echelle chunks).
 template <int RBT, int CBT>
-__global__ __launch_bounds__(256, (RBT * CBT <= 3) ? 3 : 1) void k_dpass(const ChunkDev *cs, const double *in,
+__global__ __launch_bounds__(256, (RBT * CBT <= 4) ? 3 : 2) void k_dpass(const ChunkDev *cs, const double *in,
                                                const TableDev *tabs, BinsDev bins,
                                                const double *mat, const double *vec, double *P) {
     const ChunkDev c = cs[blockIdx.y];
@@ -326,20 +335,22 @@ __global__ __launch_bounds__(256, (RBT * CBT <= 3) ? 3 : 1) void k_dpass(const C
     const double *wave = in + c.in_off + IN_WAVE * (size_t)Np;
     const double *S = mat + c.mat_off + 3 * (size_t)Np * Np;
     const double *V = vec + c.vec_off;
-    __shared__ int siv[4][64];
+    // per wave: the columns' table rows (in pairs) and fractions, S, and the z-bin
+    // weights with a row of ones for the columns of S
+    __shared__ unsigned int siv[4][64];
     __shared__ double sfr[4][64], sS[4][64];
-    __shared__ double sw[4][DP_ZB][64];
+    __shared__ double sw[4][DP_ZB + 1][64];
     __shared__ double sR[64][1 + MAX_NU];
     const int nx = 1 + nu;
     const int ncq = c.nzq * nx, ncol = ncq + nx;
     const bool tab = !c.rm;
-    // this lane's B columns: (z bin m, component x); m = -1 for the S columns
+    // this lane's B columns: (z bin m, component x); DP_ZB for S, -2 past them
     int bm[CBT], bx[CBT];
 #pragma unroll
     for (int cb = 0; cb < CBT; ++cb) {
         const int col = cb * 16 + l % 16;
         if (col < ncq) { bm[cb] = col / nx; bx[cb] = col % nx; }
-        else if (col < ncol) { bm[cb] = -1; bx[cb] = col - ncq; }
+        else if (col < ncol) { bm[cb] = DP_ZB; bx[cb] = col - ncq; }
         else { bm[cb] = -2; bx[cb] = 0; }
     }
     dq4 acc[RBT][CBT];
@@ -348,87 +359,113 @@ __global__ __launch_bounds__(256, (RBT * CBT <= 3) ? 3 : 1) void k_dpass(const C
 #pragma unroll
         for (int cb = 0; cb < CBT; ++cb) acc[rb][cb] = dq4{0.0, 0.0, 0.0, 0.0};
     dvec2 gA[RBT], gB[RBT];
-    // both interpolation nodes of this lane's band at K slot kk + l/16, at a
-    // clamped (always valid) slot and band, so every gather is unconditional
+    // this lane's bands in the table, clamped so that every gather is valid, or
+    // its rows of the materialised matrices
+    GlobalD2 *q2[RBT];
+    GlobalD *qm[RBT];
+#pragma unroll
+    for (int rb = 0; rb < RBT; ++rb) {
+        const int kn = rb * 16 + l % 16;
+        if (tab) q2[rb] = (GlobalD2 *)t.q2 + min(kn, nk - 1);
+        else qm[rb] = (GlobalD *)mat + c.qb_off + ((size_t)min(kn, c.kbu - 1) * Np + min(i, Np - 1)) * Np + 2 * (l / 16);
+    }
+    // both interpolation nodes of this lane's bands at K slot kk + l/16
     auto gather = [&](int kk, dvec2 *g) {
-        const int iv = siv[wv][min(kk, 60) + l / 16];   // 0 for slots outside the chunk
+        const unsigned int iv = siv[wv][min(kk, 60) + l / 16];   // 0 for slots outside the chunk
+#pragma unroll
+        for (int rb = 0; rb < RBT; ++rb) g[rb] = q2[rb][iv];
+    };
+    // one K step: this lane's slot bl and its band values, then the MFMAs.  What
+    // needs no test here: outside the chunk the weights and R are zero, and the
+    // rows and columns past the stored ones are never read
+    auto step = [&](int bl, double *a) {
+        const double sv = sS[wv][bl];
+        double bv[CBT];
+#pragma unroll
+        for (int rb = 0; rb < RBT; ++rb) a[rb] = (rb * 16 + l % 16 == c.kbu) ? sv : a[rb];
+#pragma unroll
+        for (int cb = 0; cb < CBT; ++cb) bv[cb] = sw[wv][max(bm[cb], 0)][bl] * sR[bl][bx[cb]];
 #pragma unroll
         for (int rb = 0; rb < RBT; ++rb)
-            g[rb] = *(const GlobalD2 *)(t.q2 + 2 * ((size_t)iv * nk + min(rb * 16 + l % 16, nk - 1)));
+#pragma unroll
+            for (int cb = 0; cb < CBT; ++cb)
+                acc[rb][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[rb], bv[cb], acc[rb][cb], 0, 0, 0);
+    };
+    auto tab_step = [&](int kk, const dvec2 *g) {
+        const int bl = kk + l / 16;
+        const double fr = sfr[wv][bl];
+        double a[RBT];
+#pragma unroll
+        for (int rb = 0; rb < RBT; ++rb) a[rb] = g[rb].x * (1 - fr) + g[rb].y * fr;
+        step(bl, a);
     };
     for (int b0 = 0; b0 < c.N; b0 += 64) {
         __syncthreads();
         {
             const int b = b0 + l;
             const bool ok = rowok && b < c.N;
-            int iv = 0;
+            unsigned int iv = 0;
             double fr = 0.0, z = 0.0, sv = 0.0;
             if (ok) {
                 double v;
                 vz_pair(wave[i], wave[b], i, b, v, z);
                 const double xx = (v - t.v1) / t.dv;
                 iv = interp_index(xx, t.nv);
-                fr = xx - iv;
+                fr = xx - (int)iv;
                 sv = S[(size_t)i * Np + b];
             }
-            siv[wv][l] = iv;
+            siv[wv][l] = iv * (unsigned int)nk;
             sfr[wv][l] = fr;
             sS[wv][l] = sv;
-#pragma unroll
-            for (int m = 0; m < DP_ZB; ++m) sw[wv][m][l] = (ok && m < c.nzq) ? zweight(bins, z, c.zm0 + m) : 0.0;
+            for (int m = 0; m < c.nzq; ++m) sw[wv][m][l] = ok ? zweight(bins, z, c.zm0 + m) : 0.0;
+            sw[wv][DP_ZB][l] = ok ? 1.0 : 0.0;
         }
         for (int e = tid; e < 64 * (1 + MAX_NU); e += 256) {
             const int bb = e / (1 + MAX_NU), x = e % (1 + MAX_NU);
             const int b = b0 + bb;
             double val = 0.0;
-            if (b < c.N && x < nx) val = (x == 0) ? V[V_Y * (size_t)Np + b] : V[(V_W0 + x - 1) * (size_t)Np + b];
+            if (b < c.N && x < nx)
+                val = (x == 0) ? V[V_Y * (size_t)Np + b] : V[(V_W0 + x - 1) * (size_t)Np + b];
             sR[bb][x] = val;
         }
         __syncthreads();
         const int nb = min(64, c.N - b0);
-        // one K step: operands of columns kk.. from the band values (the
-        // gathered table nodes, or the materialised matrices), then the MFMAs
-        auto step = [&](int kk, const dvec2 *g, bool tabs_mode) {
-            const int bl = kk + l / 16;            // this lane's K slot
-            const bool bok = rowok && bl < nb;
-            const double fr = sfr[wv][bl];
-            const double sv = sS[wv][bl];
-            double a[RBT], bv[CBT];
-#pragma unroll
-            for (int rb = 0; rb < RBT; ++rb) {
-                const int kn = rb * 16 + l % 16;
-                double q;
-                if (tabs_mode) q = g[rb].x * (1 - fr) + g[rb].y * fr;
-                else q = mat[c.qb_off + ((size_t)min(kn, c.kbu - 1) * Np + i) * Np + b0 + bl];
-                a[rb] = (!bok) ? 0.0 : (kn < c.kbu) ? q : (kn == c.kbu) ? sv : 0.0;
-            }
-#pragma unroll
-            for (int cb = 0; cb < CBT; ++cb) {
-                const double r = sR[bl][bx[cb]];
-                const double wz = sw[wv][max(bm[cb], 0)][bl];
-                bv[cb] = (!bok || bm[cb] < -1) ? 0.0 : (bm[cb] >= 0) ? wz * r : r;
-            }
-#pragma unroll
-            for (int rb = 0; rb < RBT; ++rb)
-#pragma unroll
-                for (int cb = 0; cb < CBT; ++cb)
-                    acc[rb][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[rb], bv[cb], acc[rb][cb], 0, 0, 0);
-        };
         if (tab) {
             gather(0, gA);
             gather(4, gB);
             for (int kk = 0; kk < nb; kk += 8) {
-                step(kk, gA, true);
+                tab_step(kk, gA);
                 gather(kk + 8, gA);
                 if (kk + 4 < nb) {
-                    step(kk + 4, gB, true);
+                    tab_step(kk + 4, gB);
                     gather(kk + 12, gB);
                 }
             }
         } else {
-            // resolution-matrix mode (kbu >= 1 there; rows past the chunk read
-            // inside the padded matrix and are zeroed by the selects)
-            for (int kk = 0; kk < nb; kk += 4) step(kk, gA, false);
+            // resolution-matrix mode (kbu >= 1 there): two neighbouring columns a
+            // load, the operands of two steps, a load ahead; columns past the
+            // chunk lie inside the padded matrices, which are zero there
+            auto load = [&](int kk, dvec2 *g) {
+#pragma unroll
+                for (int rb = 0; rb < RBT; ++rb) g[rb] = *(GlobalD2 *)(qm[rb] + b0 + min(kk, 56));
+            };
+            auto two = [&](int kk, const dvec2 *g) {
+                double a[RBT], d[RBT];
+#pragma unroll
+                for (int rb = 0; rb < RBT; ++rb) {
+                    a[rb] = g[rb].x;
+                    d[rb] = g[rb].y;
+                }
+                step(kk + 2 * (l / 16), a);
+                step(kk + 2 * (l / 16) + 1, d);
+            };
+            load(0, gA);
+            for (int kk = 0; kk < nb; kk += 16) {
+                load(kk + 8, gB);
+                two(kk, gA);
+                load(kk + 16, gA);
+                if (kk + 8 < nb) two(kk + 8, gB);
+            }
         }
     }
     if (!rowok) return;
@@ -442,10 +479,10 @@ __global__ __launch_bounds__(256, (RBT * CBT <= 3) ? 3 : 1) void k_dpass(const C
             for (int u = 0; u < 4; ++u) {
                 const int kn = rb * 16 + 4 * u + l / 16;
                 const double val = acc[rb][cb][u];
-                if (bm[cb] >= 0 && kn < c.kbu) {
+                if (bm[cb] < DP_ZB && kn < c.kbu) {
                     const int j = bm[cb] * c.kbu + kn;
                     P[c.pj_off + ((size_t)j * Np + i) * (1 + MAX_NU) + bx[cb]] = val;
-                } else if (bm[cb] == -1 && kn == c.kbu) {
+                } else if (bm[cb] == DP_ZB && kn == c.kbu) {
                     P[c.pj_off + ((size_t)(c.n + 1) * Np + i) * (1 + MAX_NU) + bx[cb]] = val;
                 }
             }
