@@ -245,12 +245,12 @@ void launch_gemm_whiten_right(hipStream_t st, int prec, int nst, const ChunkDev 
     launch_mode<MODE_RIGHT>(st, prec, nst, chunks, work, nwork, Y, li, G, jlo);
 }
 void launch_gemm_gram(hipStream_t st, int prec, int nst, const ChunkDev *chunks, const Work *work, int nwork,
-                      const void *G, double *gram) {
+                      bool offdiag, const void *G, double *gram) {
     if (prec == 0) {
         if (nwork > 0) launch_gram64(st, chunks, work, nwork, (const double *)G, gram);
         return;
     }
-    launch_mode<MODE_GRAM>(st, prec, nst, chunks, work, nwork, G, G, gram, 0);
+    launch_mode<MODE_GRAM>(st, prec, nst, chunks, work, nwork, G, G, gram, offdiag);   // jlo is not the Gram's
 }
 
 }  // namespace qml
@@ -843,6 +843,118 @@ void k_gemm_bf3d(const ChunkDev *cs, const Work *work, int nwork, const __bf16 *
     bf3_epilogue<MODE>(acc, c, wk, jlo, r0, c0, Cbase, smem + w * 64 * BF3_EP, lane);
 }
 
+// The Gram where no chunk of the batch has more than 128 members (every work item
+// on the diagonal): all pairs of the members over one G tile, each member's row
+// staged once.  Wave W sums the upper 16 x 16 blocks of row
+// blocks W and 7 - W (nine; with 64 members or fewer row block W alone), so that
+// the waves carry equal parts, and blocks past the members are left out.  A block
+// sums its 4096 terms in the same order as k_gemm_bf3, so the same results, bit
+// for bit.  Three slots of 16 KB, two steps in flight, three workgroups per CU.
+// Bound by reading the G store, 64 bytes a row and plane at a time, or on small
+// batches by the latency of the 128 steps: 64 chunks of 256 pixels, 23 members, 190
+// -> 62 us against k_gemm_bf3d (whose 640 items take two turns on the chip), 640
+// chunks of 150 to 700 pixels 8.8 -> 8.6 ms.  With items off the diagonal that
+// kernel takes all: in a launch of their own they read the G tiles once more (160
+// chunks of up to 190 members 5.1 -> 6.3 ms).
+template <int NPROD, int MB, int W, class Issue>
+__device__ __forceinline__ void gram_sweep(const Issue &issue, const __bf16 *smem, int mb, const ChunkDev &c,
+                                           const Work &wk, double *gram) {
+    constexpr int X1 = (MB == 8) ? 7 - W : MB, N1 = (MB == 8) ? W + 1 : 1, ns = TILE * TILE / BK;
+    const int lane = threadIdx.x % 64, off = bf3_slot(lane % 16, lane / 16);
+    f4 acc0[MB - W], acc1[N1];
+#pragma unroll
+    for (int y = 0; y < MB - W; ++y) acc0[y] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int y = 0; y < N1; ++y) acc1[y] = f4{0.f, 0.f, 0.f, 0.f};
+    const auto mul = [](bf8 xh, bf8 xl, bf8 yh, bf8 yl, f4 acc) {
+        if constexpr (NPROD == 4) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(yl, xl, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(yh, xl, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(yl, xh, acc, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(yh, xh, acc, 0, 0, 0);
+    };
+    issue(0, 0);
+    issue(1, 1);
+    int sl = 0;
+    for (int s = 0; s < ns; ++s) {
+        bf3_wait_step<MB / 2>(s + 1 >= ns);
+        if (s + 2 < ns) issue(s + 2, sl == 0 ? 2 : sl - 1);
+        const __bf16 *st = smem + sl * 2 * BF3_PL + off;
+        const auto part = [&](int y, int pl) { return *(const bf8 *)(st + pl * BF3_PL + y * 16 * BK); };
+        if (W < mb) {
+            const bf8 ah = part(W, 0), al = part(W, 1);
+            bf8 bh = {}, bl = {};
+            if constexpr (MB == 8) {
+                bh = part(X1, 0);
+                bl = part(X1, 1);
+            }
+#pragma unroll
+            for (int y = W; y < MB; ++y) {
+                if (y >= mb) break;
+                const bf8 yh = (y == W) ? ah : part(y, 0), yl = (y == W) ? al : part(y, 1);
+                acc0[y - W] = mul(ah, al, yh, yl, acc0[y - W]);
+                if (y >= X1) acc1[y - X1] = mul(bh, bl, yh, yl, acc1[y - X1]);
+            }
+        }
+        sl = sl == 2 ? 0 : sl + 1;
+    }
+    // lane holds C[16x + lane%16][16y + 4(lane/16) + u], u = 0..3
+    const double wgt = packed_tile_is_diag(wk.j, c.nt) ? 1.0 : 2.0;
+    const int base = wk.I * (BF3_BM / TILE);
+    double *E = gram + c.gram_off + (size_t)wk.j * (c.mt * (c.mt + 1) / 2) * TILE * TILE;
+    const auto put = [&](int x, int y, f4 acc) {
+        double *o = E + (size_t)upper_tile_index(base + x / 4, base + y / 4, c.mt) * TILE * TILE
+                  + (16 * (x % 4) + lane % 16) * TILE + 16 * (y % 4) + 4 * (lane / 16);
+        *(double2 *)o = double2{wgt * (double)acc[0], wgt * (double)acc[1]};
+        *(double2 *)(o + 2) = double2{wgt * (double)acc[2], wgt * (double)acc[3]};
+    };
+#pragma unroll
+    for (int y = W; y < MB; ++y) {
+        if (y >= mb) break;
+        put(W, y, acc0[y - W]);
+        if (y >= X1) put(X1, y, acc1[y - X1]);
+    }
+}
+
+template <int NPROD>
+__global__ __launch_bounds__(256, 3) void k_gram_bf3(const ChunkDev *cs, const Work *work, int nwork,
+                                                     const __bf16 *G, double *gram) {
+    const int li = xcd_logical(nwork);
+    if (li >= nwork) return;
+    const Work wk = work[li];
+    if (wk.c < 0) return;
+    const ChunkDev c = cs[wk.c];
+    __shared__ __attribute__((aligned(1024))) __bf16 smem[3 * 2 * BF3_PL];
+    const int lane = threadIdx.x % 64, w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int I0 = wk.I * BF3_BM, mb = (min(BF3_BM, c.m - I0) + 15) / 16;
+    const long long ktot = (long long)c.ntu * TILE * TILE;
+    const int rl = lane / 4, ch = (lane % 4) ^ bf3_swz(rl);
+    const auto sweep = [&](auto size) {
+        constexpr int MB = decltype(size)::value, NB = MB / 2;   // NB blocks of 16 rows a wave and step
+        const int row0 = 16 * NB * (w % 2);
+        GlobalB *src[NB];   // plane w / 2 (hi, lo); rows past the members read the first
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int row = I0 + row0 + 16 * b + rl;
+            src[b] = (GlobalB *)(G + c.g_off + (row < c.m ? row : I0) * 2 * ktot + (w / 2) * ktot
+                                 + (long long)wk.j * TILE * TILE + 8 * ch);
+        }
+        __bf16 *const dst0 = smem + (w / 2) * BF3_PL + row0 * BK;
+        const auto issue = [&](int s, int slot) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                __builtin_amdgcn_global_load_lds(
+                    (const __attribute__((address_space(1))) void *)(src[b] + (size_t)s * (2 * BK)),
+                    (__attribute__((address_space(3))) void *)(dst0 + slot * 2 * BF3_PL + b * 16 * BK), 16, 0, 0);
+        };
+        if (w == 0) gram_sweep<NPROD, MB, 0>(issue, smem, mb, c, wk, gram);
+        else if (w == 1) gram_sweep<NPROD, MB, 1>(issue, smem, mb, c, wk, gram);
+        else if (w == 2) gram_sweep<NPROD, MB, 2>(issue, smem, mb, c, wk, gram);
+        else gram_sweep<NPROD, MB, 3>(issue, smem, mb, c, wk, gram);
+    };
+    if (mb <= 4) sweep(std::integral_constant<int, 4>{});
+    else sweep(std::integral_constant<int, 8>{});
+}
+
 template <int NPROD>
 static void launch_bf3_np(hipStream_t st, int mode, int nst, const ChunkDev *chunks, const Work *work, int nwork,
                           const __bf16 *a, const __bf16 *b, void *C, int jlo) {
@@ -868,6 +980,7 @@ static void launch_bf3_np(hipStream_t st, int mode, int nst, const ChunkDev *chu
         else QML_BF3_LAUNCH(MODE_RIGHT, 1);
     } else {
         if (nst == 4) QML_BF3D_LAUNCH(MODE_GRAM, 3, 3);
+        else if (nst == 3 && !jlo) k_gram_bf3<NPROD><<<grid, 256, 0, st>>>(chunks, work, nwork, a, (double *)C);
         else if (nst == 3) QML_BF3D_LAUNCH(MODE_GRAM, 2, 2);
         else if (nst == 1) QML_BF3_LAUNCH(MODE_GRAM, 1);
         else QML_BF3_LAUNCH(MODE_GRAM, 2);

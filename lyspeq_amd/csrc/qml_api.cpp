@@ -63,6 +63,7 @@ struct Batch {
     ChunkDev *d_chunks = nullptr;
     Work *d_wl = nullptr, *d_wr = nullptr, *d_wg = nullptr;
     int nwl = 0, nwr = 0, nwg = 0;
+    bool wg_off = false;   // Gram items off the diagonal
     // stack slabs: the left and right work lists of slab s are
     // [sl_off[s], sl_off[s + 1]) of d_wl and [sr_off[s], sr_off[s + 1]) of d_wr
     int nslab = 1;
@@ -900,6 +901,7 @@ int plan_batches(qml_ctx *c) {
             }
             const int g = (c->prec >= 2) ? 2 : 1;
             const int mtg = (d.mt + g - 1) / g;
+            B.wg_off |= mtg > 1;
             for (int x = 0; x < 8; ++x) {
                 int sa, sb;
                 XcdLists::share(0, d.ntu, x, li, sa, sb);
@@ -1186,7 +1188,7 @@ int enqueue_iteration(qml_ctx *c, bool timing) {
                                      B.sr_off[sb + 1] - B.sr_off[sb], li, c->d_Y, G, L2.jlo);
             HIPCHK(mark(last ? B.evB[3] : B.evS[3 * sb + 2], sB));
         }
-        launch_gemm_gram(sB, c->prec, c->nst_gram, B.d_chunks, B.d_wg, B.nwg, G, c->d_gram);
+        launch_gemm_gram(sB, c->prec, c->nst_gram, B.d_chunks, B.d_wg, B.nwg, B.wg_off, G, c->d_gram);
         HIPCHK(mark(B.evB[4], sB));
         launch_gram_finalize(L2, c->d_outs, c->d_gram, c->d_status, c->d_fc, c->d_dbt);
         HIPCHK(hipEventRecord(B.evB[5], sB));

@@ -102,7 +102,7 @@ void launch_gemm_whiten_left(hipStream_t st, int prec, int nst, const ChunkDev *
 void launch_gemm_whiten_right(hipStream_t st, int prec, int nst, const ChunkDev *chunks, const Work *work,
                               int nwork, const void *li, const void *Y, void *G, int jlo);
 // Gram partials E_s = sum over G tile s of G_j G_j'.
-void launch_gemm_gram(hipStream_t st, int prec, int nst, const ChunkDev *chunks, const Work *work, int nwork,
+void launch_gemm_gram(hipStream_t st, int prec, int nst, const ChunkDev *chunks, const Work *work, int nwork, bool offdiag,
                       const void *G, double *gram);
 
 // kernels_gemm64.hip: the FP64 products (the work lists hold the lower tiles
