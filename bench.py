@@ -61,7 +61,7 @@ def kernel_work(shapes, prec):
     for N, n, nt in shapes:
         m = n + 2
         N = float(N)
-        if prec in ("bf16x3", "bf16x4"):
+        if prec != "fp32":
             # X_j = M + M^T: P = Li M (lower x lower), G = P Li^T + Li P^T (upper half)
             w["whiten_left"] += m * N * (N + 1) * (N + 2) / 3.0
             w["whiten_right"] += 2.0 * m * N * (N + 1) * (N + 2) / 3.0
@@ -69,7 +69,8 @@ def kernel_work(shapes, prec):
             w["whiten_left"] += m * N * N * (N + 1)               # lower-triangular x dense
             w["whiten_right"] += m * N * (N + 1) * (N + 2) / 3.0  # upper half, triangular operand
         w["gram"] += m * (m + 1) / 2.0 * N * (N + 1)          # symmetric pairs over packed halves
-        w["xgen_bytes"] += m * N * N * es                      # projected Q stack written once
+        # the projected Q stack written once: its upper triangle, or all of it in FP32
+        w["xgen_bytes"] += m * N * (N if prec == "fp32" else (N + 1) / 2.0) * es
     return w
 
 

@@ -426,7 +426,8 @@ int qml_autotune(qml_ctx *ctx, const double *theta, const int *caps, int ncaps, 
  *      three workgroups per CU);
  *   2  through registers, two LDS stages (two workgroups per CU); not for
  *      the right product;
- *   3  direct-to-LDS loads (global_load_lds), two stages (two per CU);
+ *   3  direct-to-LDS loads (global_load_lds), two stages, three of the
+ *      member's operand (two per CU; small Grams three);
  *   4  direct-to-LDS loads, three stages (one per CU).
  * Defaults 3, 3 and 3.  Results are identical for every choice.  No
  * counterpart in the reference. */
