@@ -196,7 +196,9 @@ __global__ __launch_bounds__(256) void k_mv_rows(const ChunkDev *cs, const doubl
 
 // out_r = Li^T in_r: a workgroup takes 64 columns (lane = column, coalesced
 // row segments); the four waves split the rows i >= k0 and are combined in
-// LDS.
+// LDS.  Bound by the latency of a few workgroups' rows: with 16 of a wave's loads
+// in flight instead of four, and R loaded a lane a row and broadcast: one chunk
+// of 488 pixels 40 -> 14 us a launch, 64 of 256 29 -> 10.
 __global__ __launch_bounds__(256) void k_mv_cols(const ChunkDev *cs, const double *mat, double *vec, int in_slot,
                                                  int out_slot, int single) {
     constexpr int NR = 1 + MAX_NU;
@@ -204,7 +206,7 @@ __global__ __launch_bounds__(256) void k_mv_cols(const ChunkDev *cs, const doubl
     const int Np = c.Np, k0 = blockIdx.x * 64;
     if (k0 >= Np) return;
     const int nr = single ? 1 : 1 + c.nu;
-    const int w = threadIdx.x / 64, l = threadIdx.x % 64;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), l = threadIdx.x % 64;
     const double *Li = mat + c.mat_off + 2 * (size_t)Np * Np;
     double *V = vec + c.vec_off;
     const double *R = V + in_slot * (size_t)Np;
@@ -212,13 +214,25 @@ __global__ __launch_bounds__(256) void k_mv_cols(const ChunkDev *cs, const doubl
     double s[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) s[r] = 0.0;
-    // Li[i][k] is zero for i < k, so rows from k0 on cover the block
-#pragma unroll 4
-    for (int i = k0 + w; i < Np; i += 4) {
-        const double a = Li[(size_t)i * Np + k0 + l];
+    // Li[i][k] is zero for i < k, so rows from k0 on cover the block; 64 rows at a
+    // time (Np is a multiple of 64), a wave's 16 in flight together
+    for (int i0 = k0; i0 < Np; i0 += 64) {
+        double a[16], rv[NR];   // rv: lane l holds R of row i0 + l
+#pragma unroll
+        for (int u = 0; u < 16; ++u) a[u] = Li[(size_t)(i0 + w + 4 * u) * Np + k0 + l];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) rv[r] = R[min(r, nr - 1) * (size_t)Np + i0 + l];
 #pragma unroll
         for (int r = 0; r < NR; ++r)
-            if (r < nr) s[r] += a * R[r * (size_t)Np + i];
+            if (r < nr) {
+                const long long v = __double_as_longlong(rv[r]);
+#pragma unroll
+                for (int u = 0; u < 16; ++u) {
+                    const long long x = ((long long)__builtin_amdgcn_readlane((int)(v >> 32), w + 4 * u) << 32)
+                                      | (unsigned int)__builtin_amdgcn_readlane((int)v, w + 4 * u);
+                    s[r] += a[u] * __longlong_as_double(x);
+                }
+            }
     }
 #pragma unroll
     for (int r = 0; r < NR; ++r) red[w][r][l] = s[r];
