@@ -93,11 +93,13 @@ __global__ __launch_bounds__(256) void k_deriv_table(const double *pairs, const 
 }
 
 // P_fid(k_m, z_i) (core/fiducial_cosmology.cpp:273-282) on the signal grid:
-// pk[m * nzp + i], zero for i >= nz and past the last mode
+// pk[m * nzp + i], zero for i >= nz and past the last mode.  Eight modes and 32
+// redshifts a workgroup: mpad nzp may exceed 32 bits (4097 velocities at 65535
+// redshifts: 2.1e9)
 __global__ __launch_bounds__(256) void k_pfid_grid(double dk, int nmode, int mpad, double z1, double dz, int nz, int nzp,
                                                    PD13 pd, double *pk) {
-    const int e = blockIdx.x * 256 + threadIdx.x, m = e / nzp, iz = e % nzp;
-    if (m >= mpad) return;
+    const int m = blockIdx.x * 8 + threadIdx.x / 32, iz = blockIdx.y * 32 + threadIdx.x % 32;
+    if (m >= mpad || iz >= nzp) return;
     double p = 0.0;
     if (m < nmode && iz < nz) {
         const double k = m * dk, z = z1 + dz * iz;
@@ -108,7 +110,7 @@ __global__ __launch_bounds__(256) void k_pfid_grid(double dk, int nmode, int mpa
         p = pd.A * TAB_PI / K0 * pow(q0, 2.0 + pd.n + pd.alpha * lq + pd.beta * log(x0)) * pow(x0, pd.B) /
             (1.0 + pd.lambda * k * k);
     }
-    pk[e] = p;
+    pk[(size_t)m * nzp + iz] = p;
 }
 
 // W^2 of each pair's modes, doubled where the inverse transform counts a mode
@@ -229,8 +231,7 @@ SignalGrid signal_grid(int nhalf, int nz) {
 
 void launch_pfid_grid(hipStream_t st, const SignalGrid &g, double dk, double z1, double dz, int nz, PD13 pd,
                       double *pk) {
-    const int total = g.mpad * g.nzp;
-    k_pfid_grid<<<(total + 255) / 256, 256, 0, st>>>(dk, g.nhalf + 1, g.mpad, z1, dz, nz, g.nzp, pd, pk);
+    k_pfid_grid<<<dim3((g.mpad + 7) / 8, (g.nzp + 31) / 32), 256, 0, st>>>(dk, g.nhalf + 1, g.mpad, z1, dz, nz, g.nzp, pd, pk);
 }
 
 void launch_signal_tables(hipStream_t st, const SignalGrid &g, const double *pairs, const int *mend, int npairs,

@@ -1,0 +1,44 @@
+"""The device signal tables at the limits of their grids (needs an MI355X)."""
+import math
+
+import numpy as np
+import pytest
+
+from lyspeq_amd import synth
+from lyspeq_amd.qml import Binning, QMLEngine
+
+pytestmark = pytest.mark.gpu
+
+BINS = Binning(k0=0.0, nklin=10, dklin=0.002, nklog=0, dklog=0.1, z0=2.4, z_bin_width=0.2, nz=1, method=1,
+               cont_logl_order=1, cont_lam_order=-1, max_forest_length_v=2.0e3)
+
+
+def _columns(pair, nv, v_length, nz, cols, pd13):
+    """Columns of the signal table by the inverse real FFT, modes with
+    W^2 < 1e-40 left out."""
+    n = 1 << (math.ceil(math.log2(4 * nv)) + 1)
+    length = v_length / (nv - 1.0) / 2 * n
+    k = np.arange(n // 2 + 1) * (2 * math.pi / length)
+    R = synth.SPEED_OF_LIGHT / pair[0] / synth.ONE_SIGMA_2_FWHM
+    w2 = synth.window_sq(k, pair[1], R)
+    keep = k * R < 9.5
+    zc, width = BINS.zbin_centers()[0], BINS.z_bin_width
+    out = []
+    for iz in cols:
+        z = zc - width + width * (BINS.nz + 1) / (nz - 1.0) * iz
+        f = np.zeros(k.size)
+        f[keep] = w2[keep] * synth.pd13_power(k[keep], z, *pd13)
+        out.append(np.fft.irfft(f, n)[:2 * nv:2] * n / length)
+    return np.array(out).T
+
+
+def test_more_than_2_31_modes_times_redshifts():
+    """4097 velocities and 65535 redshifts: 32800 x 65536 elements of P_fid."""
+    print("[case] 4097 x 65535 signal table", flush=True)
+    pair, nv, v_length, nz = (2000, 50.0), 4097, 40960.0, 65535
+    eng = QMLEngine(BINS)
+    _, s = eng.make_tables([pair], nv, v_length, nz, synth.PD13_DEFAULT, deriv=False)
+    eng.close()
+    cols = [0, 1, 31, 32, 32767, 32768, 65533, 65534]
+    want = _columns(pair, nv, v_length, nz, cols, synth.PD13_DEFAULT)
+    assert np.max(np.abs(s[0][:, cols] - want)) < 1e-11 * np.max(np.abs(want))
