@@ -174,8 +174,9 @@ __global__ __launch_bounds__(256, 2) void k_signal_sum(const int *mend, const do
         for (int t = 0; t < 8; ++t) {
             const int mm = m + 4 * t + lq;
             const double wm = w[mm];
-            b[t][0] = wm * pz[(size_t)mm * nzp];
-            b[t][1] = wm * pz[(size_t)mm * nzp + 16];
+            // a mode that is left out adds nothing, also where its power overflowed
+            b[t][0] = wm == 0.0 ? 0.0 : wm * pz[(size_t)mm * nzp];
+            b[t][1] = wm == 0.0 ? 0.0 : wm * pz[(size_t)mm * nzp + 16];
         }
 #pragma unroll
         for (int t = 0; t < 8; ++t)

@@ -21,7 +21,7 @@ def _columns(pair, nv, v_length, nz, cols, pd13):
     k = np.arange(n // 2 + 1) * (2 * math.pi / length)
     R = synth.SPEED_OF_LIGHT / pair[0] / synth.ONE_SIGMA_2_FWHM
     w2 = synth.window_sq(k, pair[1], R)
-    keep = k * R < 9.5
+    keep = np.arange(k.size) <= math.ceil(9.6 / (R * k[1]))
     zc, width = BINS.zbin_centers()[0], BINS.z_bin_width
     out = []
     for iz in cols:
@@ -42,3 +42,26 @@ def test_more_than_2_31_modes_times_redshifts():
     cols = [0, 1, 31, 32, 32767, 32768, 65533, 65534]
     want = _columns(pair, nv, v_length, nz, cols, synth.PD13_DEFAULT)
     assert np.max(np.abs(s[0][:, cols] - want)) < 1e-11 * np.max(np.abs(want))
+
+
+def test_infinite_power_past_the_kept_modes():
+    """1 + lambda k^2 is zero at k = 1/8, nine modes past the last kept one: a
+    mode that is left out adds nothing, infinite or not."""
+    print("[case] infinite power past the kept modes", flush=True)
+    R_fwhm, nv, nz, mode = 1650, 1601, 3, 1975
+    R = synth.SPEED_OF_LIGHT / R_fwhm / synth.ONE_SIGMA_2_FWHM
+    n = 1 << (math.ceil(math.log2(4 * nv)) + 1)
+
+    def step(v_length):
+        return 2 * math.pi / (v_length / (nv - 1.0) / 2.0 * n)
+
+    v_length = 2 * math.pi / (0.125 / mode) / n * 2 * (nv - 1)
+    v_length = next(v for v in v_length + np.arange(-200, 200) * np.spacing(v_length) if mode * step(v) == 0.125)
+    last = math.ceil(9.6 / (R * step(v_length)))
+    assert last < mode < (last + 32) // 32 * 32     # in the last block of 32 modes
+    pd13 = (0.066, -2.7, -0.1, 3.6, 0.0, -64.0)
+    eng = QMLEngine(BINS)
+    _, s = eng.make_tables([(R_fwhm, 50.0)], nv, v_length, nz, pd13, deriv=False)
+    eng.close()
+    want = _columns((R_fwhm, 50.0), nv, v_length, nz, range(nz), pd13)
+    assert np.max(np.abs(s[0] - want)) < 1e-11 * np.max(np.abs(want))
