@@ -124,92 +124,109 @@ __global__ __launch_bounds__(256) void k_signal_window(const double *pairs, cons
     w2[(size_t)p * mpad + m] = w;
 }
 
-// part[s][p][iv][iz] = the sum over range s of pair p's modes of
-// cos(k_m v_iv) w2(m) pk(m, iz).  A wave takes 64 velocities and 32 redshifts,
-// four modes a step on v_mfma_f64_16x16x4f64: lane l's A values are the cosines
-// of its four velocities at mode l / 16 of the step, advanced by rotation by
-// four modes and re-seeded every 256 modes; its B values the weighted power at
-// that mode.  A cosine thus serves 32 redshifts and a loaded power 64
-// velocities; one thread per velocity and redshift advanced the same cosine for
-// each redshift (26.4 ms for 48 pairs at 4601 x 29 and 8000 to 20000 modes,
-// 3.8 ms here).  The phase k_m v_iv = 2 pi m iv / nhalf, nhalf a power of two, is
-// reduced exactly in integers.  The modes are cut into SIG_PARTS ranges whatever
-// the number of pairs, so that one pair fills the chip and its sums do not
-// depend on the others.
-constexpr int SIG_PARTS = 8, SIG_SEED = 256;
+// out[p][iv][iz] = inv_len times the sum over pair p's modes of
+// cos(k_m v_iv) w2(m) pk(m, iz), z contiguous.  A workgroup takes 32 velocities
+// and 16 Y redshifts, its eight waves an eighth of the modes each, four modes a
+// step on v_mfma_f64_16x16x4f64: lane l's A values are the cosines of its two
+// velocities at mode l / 16 of the step, advanced by rotation by four modes and
+// re-seeded every 256 modes; its B values the weighted power at that mode.  The
+// phase k_m v_iv = 2 pi m iv / nhalf, nhalf a power of two, is reduced exactly in
+// integers.  The modes are split whatever the number of pairs, so that one pair
+// fills the chip and its sums do not depend on the others; the eighths are added
+// in LDS.  Bound by the matrix cores with many pairs, by the steps' latency with
+// one.  Redshifts go 32 at a time, the rest with Y = 1 where it fits in 16: the
+// matrix work is for whole blocks of 16.  Whole calls for 48 pairs of 4601
+// velocities, 8000 to 20000 modes, with the copy out: 29 redshifts 28.3 -> 9.5
+// ms, 9 redshifts 8.5 -> 3.0, 2 redshifts 2.38 -> 2.24; one pair of 1601, 9
+// redshifts 187 -> 84 us (one thread per velocity and redshift before).  With
+// 64 velocities a workgroup one pair at 29 redshifts takes 390 us, not 259, and
+// 48 pairs 2 to 5 % less up to 16 redshifts; with 16, 48 pairs take 9 to 20 %
+// more.  Partial tables in memory, 32 columns whatever N_Z, took 12.0, 4.8 and
+// 3.3 ms and 233 us, and eight times the tables' memory.
+constexpr int SIG_PARTS = 8, SIG_SEED = 256, SIG_X = 2;   // SIG_X: 16-velocity blocks of a workgroup
 typedef double sd4 __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(256, 2) void k_signal_sum(const int *mend, const double *__restrict__ w2,
-                                                       const double *__restrict__ pk, int nhalf, int mpad, int nzp,
-                                                       int nv, int nz, double *part) {
-    const int p = blockIdx.z, s = blockIdx.y % SIG_PARTS, zb = 32 * (blockIdx.y / SIG_PARTS);
-    const int lane = threadIdx.x % 64, lr = lane % 16, lq = lane / 16;
-    const int v0 = (blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / 64)) * 64;
-    if (v0 >= nv) return;
+template <int Y>
+__global__ __launch_bounds__(64 * SIG_PARTS, 4) void k_signal_sum(
+    const int *mend, const double *__restrict__ w2, const double *__restrict__ pk, int nhalf, int mpad, int nzp,
+    int nv, int nz, int z0, double inv_len, double *out) {
+    constexpr int X = SIG_X, E = 4 * X * Y;   // accumulator elements of a lane
+    __shared__ double red[SIG_PARTS / 2][E][64];
+    const int p = blockIdx.z, zb = z0 + 16 * Y * blockIdx.y, v0 = blockIdx.x * 16 * X;
+    const int tid = threadIdx.x, lane = tid % 64, lr = lane % 16, lq = lane / 16;
+    const int s = __builtin_amdgcn_readfirstlane(tid / 64);
     const int modes = mend[p] + 1;
     const int len = ((modes + SIG_PARTS - 1) / SIG_PARTS + 31) / 32 * 32;   // modes of a range
     const int m0 = s * len, m1 = min(m0 + len, (modes + 31) / 32 * 32);
     const unsigned mask = nhalf - 1;
     const double unit = 2.0 / nhalf;
     const double *w = w2 + (size_t)p * mpad, *pz = pk + zb + lr;
-    unsigned iv[4];
-    double rc[4], rs[4], cc[4], ss[4];
+    unsigned iv[X];
+    double rc[X], rs[X], cc[X], ss[X];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
+    for (int x = 0; x < X; ++x) {
         iv[x] = v0 + 16 * x + lr;
         sincospi(unit * ((4u * iv[x]) & mask), &rs[x], &rc[x]);   // the rotation by four modes
         cc[x] = ss[x] = 0.0;
     }
-    sd4 acc[4][2];
+    sd4 acc[X][Y];
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
+    for (int x = 0; x < X; ++x)
 #pragma unroll
-        for (int y = 0; y < 2; ++y) acc[x][y] = sd4{0.0, 0.0, 0.0, 0.0};
+        for (int y = 0; y < Y; ++y) acc[x][y] = sd4{0.0, 0.0, 0.0, 0.0};
     for (int m = m0; m < m1; m += 32) {
         if ((m - m0) % SIG_SEED == 0) {
 #pragma unroll
-            for (int x = 0; x < 4; ++x) sincospi(unit * (((unsigned)(m + lq) * iv[x]) & mask), &ss[x], &cc[x]);
+            for (int x = 0; x < X; ++x) sincospi(unit * (((unsigned)(m + lq) * iv[x]) & mask), &ss[x], &cc[x]);
         }
-        double b[8][2];
+        double b[8][Y];
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const int mm = m + 4 * t + lq;
             const double wm = w[mm];
-            // a mode that is left out adds nothing, also where its power overflowed
-            b[t][0] = wm == 0.0 ? 0.0 : wm * pz[(size_t)mm * nzp];
-            b[t][1] = wm == 0.0 ? 0.0 : wm * pz[(size_t)mm * nzp + 16];
+#pragma unroll
+            for (int y = 0; y < Y; ++y) {
+                // a mode that is left out adds nothing, also where its power overflowed
+                const double pw = pz[(size_t)mm * nzp + 16 * y];
+                b[t][y] = wm == 0.0 ? 0.0 : wm * pw;
+            }
         }
 #pragma unroll
         for (int t = 0; t < 8; ++t)
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
+            for (int x = 0; x < X; ++x) {
 #pragma unroll
-                for (int y = 0; y < 2; ++y)
+                for (int y = 0; y < Y; ++y)
                     acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(cc[x], b[t][y], acc[x][y], 0, 0, 0);
                 const double c = cc[x] * rc[x] - ss[x] * rs[x];
                 ss[x] = ss[x] * rc[x] + cc[x] * rs[x];
                 cc[x] = c;
             }
     }
-    double *o = part + ((size_t)s * gridDim.z + p) * nv * nz;
+    // the eighths in pairs: 4 + 4, 2 + 2, then the last two as they are written out
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
+    for (int h = SIG_PARTS / 2; h >= 1; h /= 2) {
+        if (s >= h && s < 2 * h) {
 #pragma unroll
-        for (int y = 0; y < 2; ++y)
+            for (int e = 0; e < E; ++e) red[s - h][e][lane] = acc[e / (4 * Y)][e / 4 % Y][e % 4];
+        }
+        __syncthreads();
+        if (s < h) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int i = v0 + 16 * x + 4 * u + lq, iz = zb + 16 * y + lr;
-                if (i < nv && iz < nz) o[(size_t)i * nz + iz] = acc[x][y][u];
-            }
-}
-
-// out (npairs x nv x nz, z contiguous) = the ranges' sums times inv_len
-__global__ __launch_bounds__(256) void k_signal_table(const double *part, size_t total, double inv_len, double *out) {
-    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= total) return;
-    double s = 0.0;
+            for (int e = 0; e < E; ++e) acc[e / (4 * Y)][e / 4 % Y][e % 4] += red[s][e][lane];
+        }
+        __syncthreads();
+    }
+    if (s == 0) {
 #pragma unroll
-    for (int k = 0; k < SIG_PARTS; ++k) s += part[(size_t)k * total + e];
-    out[e] = s * inv_len;
+        for (int e = 0; e < E; ++e) red[0][e][lane] = acc[e / (4 * Y)][e / 4 % Y][e % 4];
+    }
+    __syncthreads();
+    // element e = (x Y + y) 4 + u of a lane: velocity 16 x + 4 u + lane / 16, redshift 16 y + lane % 16
+    for (int o = tid; o < 64 * E; o += 64 * SIG_PARTS) {
+        const int iz = o % (16 * Y), i = o / (16 * Y), e = (i / 16 * Y + iz / 16) * 4 + i % 16 / 4;
+        if (v0 + i < nv && zb + iz < nz)
+            out[((size_t)p * nv + v0 + i) * nz + zb + iz] = inv_len * red[0][e][i % 4 * 16 + iz % 16];
+    }
 }
 
 }  // namespace
@@ -225,8 +242,7 @@ SignalGrid signal_grid(int nhalf, int nz) {
     SignalGrid g;
     g.nhalf = nhalf;
     g.mpad = (nhalf + 1 + 31) / 32 * 32;
-    g.nzp = (nz + 31) / 32 * 32;
-    g.parts = SIG_PARTS;
+    g.nzp = (nz + 15) / 16 * 16;
     return g;
 }
 
@@ -236,14 +252,16 @@ void launch_pfid_grid(hipStream_t st, const SignalGrid &g, double dk, double z1,
 }
 
 void launch_signal_tables(hipStream_t st, const SignalGrid &g, const double *pairs, const int *mend, int npairs,
-                          const double *pk, double dk, double inv_len, int nv, int nz, double *w2, double *part,
-                          double *out) {
+                          const double *pk, double dk, double inv_len, int nv, int nz, double *w2, double *out) {
     if (npairs <= 0 || nv <= 0 || nz <= 0) return;
     k_signal_window<<<dim3((g.mpad + 255) / 256, npairs), 256, 0, st>>>(pairs, mend, g.nhalf, g.mpad, dk, w2);
-    k_signal_sum<<<dim3((nv + 255) / 256, SIG_PARTS * (g.nzp / 32), npairs), 256, 0, st>>>(mend, w2, pk, g.nhalf, g.mpad,
-                                                                                          g.nzp, nv, nz, part);
-    const size_t total = (size_t)npairs * nv * nz;
-    k_signal_table<<<(total + 255) / 256, 256, 0, st>>>(part, total, inv_len, out);
+    const int wide = g.nzp / 32, gx = (nv + 16 * SIG_X - 1) / (16 * SIG_X);
+    if (wide > 0)
+        k_signal_sum<2><<<dim3(gx, wide, npairs), 64 * SIG_PARTS, 0, st>>>(mend, w2, pk, g.nhalf, g.mpad, g.nzp, nv, nz, 0,
+                                                                          inv_len, out);
+    if (g.nzp % 32)
+        k_signal_sum<1><<<dim3(gx, 1, npairs), 64 * SIG_PARTS, 0, st>>>(mend, w2, pk, g.nhalf, g.mpad, g.nzp, nv, nz,
+                                                                       32 * wide, inv_len, out);
 }
 
 }  // namespace qml

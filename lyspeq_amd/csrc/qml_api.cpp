@@ -1957,32 +1957,28 @@ int qml_make_tables(qml_ctx *c, const qml_table_spec *s, int npairs, const int *
     const double z1 = c->zcenters[0] - c->bins.z_bin_width;
     const double dz = c->bins.z_bin_width * (c->bins.nz + 1) / (nz - 1.0);
     const PD13 pd{s->pd13[0], s->pd13[1], s->pd13[2], s->pd13[3], s->pd13[4], s->pd13[5]};
-    // pairs per pass: outputs and the signal's partial sums of up to 2 GiB on the device
-    const size_t per = (size_t)8 * ((deriv ? (size_t)nk * nv : 0) +
-                                    (signal ? (size_t)nv * nz * (1 + grid.parts) + grid.mpad : 0));
+    // pairs per pass: outputs of up to 2 GiB on the device
+    const size_t per = (size_t)8 * ((deriv ? (size_t)nk * nv : 0) + (signal ? (size_t)nv * nz : 0));
     const int nb = (int)std::max<size_t>(1, std::min<size_t>(npairs, ((size_t)2 << 30) / per));
-    struct Bufs {
-        std::vector<void *> p;
-        ~Bufs() { for (void *x : p) hipFree(x); }
-    } bufs;
-    auto dalloc = [&](void **ptr, size_t bytes) {
-        const hipError_t e = hipMalloc(ptr, std::max<size_t>(bytes, 8));
-        if (e == hipSuccess) bufs.p.push_back(*ptr);
-        return e;
+    // one allocation for all arrays: a small call's time is mostly theirs
+    size_t total = 0;
+    auto place = [&](size_t doubles) {
+        const size_t at = total;
+        total += align_up(std::max<size_t>(doubles, 1), 32);
+        return at;
     };
-    double *d_pairs = nullptr, *d_ke = nullptr, *d_pk = nullptr, *d_q = nullptr, *d_s = nullptr, *d_w2 = nullptr,
-           *d_part = nullptr;
-    int *d_mend = nullptr;
-    HIPCHK(dalloc((void **)&d_pairs, (size_t)2 * nb * sizeof(double)));
-    HIPCHK(dalloc((void **)&d_mend, (size_t)nb * sizeof(int)));
-    HIPCHK(dalloc((void **)&d_ke, (size_t)(nk + 1) * sizeof(double)));
-    if (deriv) HIPCHK(dalloc((void **)&d_q, (size_t)nb * nk * nv * sizeof(double)));
-    if (signal) {
-        HIPCHK(dalloc((void **)&d_pk, (size_t)grid.mpad * grid.nzp * sizeof(double)));
-        HIPCHK(dalloc((void **)&d_w2, (size_t)nb * grid.mpad * sizeof(double)));
-        HIPCHK(dalloc((void **)&d_part, (size_t)grid.parts * nb * nv * nz * sizeof(double)));
-        HIPCHK(dalloc((void **)&d_s, (size_t)nb * nv * nz * sizeof(double)));
-    }
+    const size_t o_pairs = place(2 * (size_t)nb), o_mend = place(nb), o_ke = place(nk + 1),
+                 o_q = place(deriv ? (size_t)nb * nk * nv : 0), o_s = place(signal ? (size_t)nb * nv * nz : 0),
+                 o_pk = place(signal ? (size_t)grid.mpad * grid.nzp : 0),
+                 o_w2 = place(signal ? (size_t)nb * grid.mpad : 0);
+    struct Buf {
+        double *p = nullptr;
+        ~Buf() { if (p) hipFree(p); }
+    } buf;
+    HIPCHK(hipMalloc(&buf.p, total * sizeof(double)));
+    double *d_pairs = buf.p + o_pairs, *d_ke = buf.p + o_ke, *d_q = buf.p + o_q, *d_s = buf.p + o_s, *d_pk = buf.p + o_pk,
+           *d_w2 = buf.p + o_w2;
+    int *d_mend = (int *)(buf.p + o_mend);
     HIPCHK(hipMemcpy(d_ke, c->kedges.data(), (nk + 1) * sizeof(double), hipMemcpyHostToDevice));
     if (signal) launch_pfid_grid(c->st, grid, dk, z1, dz, nz, pd, d_pk);
     std::vector<double> hp(2 * (size_t)nb);
@@ -2006,7 +2002,7 @@ int qml_make_tables(qml_ctx *c, const qml_table_spec *s, int npairs, const int *
             HIPCHK(hipStreamWaitEvent(c->st2, c->ev_fork, 0));
         }
         if (signal)
-            launch_signal_tables(c->st, grid, d_pairs, d_mend, n, d_pk, dk, 1.0 / length, nv, nz, d_w2, d_part, d_s);
+            launch_signal_tables(c->st, grid, d_pairs, d_mend, n, d_pk, dk, 1.0 / length, nv, nz, d_w2, d_s);
         HIPCHK(hipGetLastError());
         if (deriv)
             HIPCHK(hipMemcpyAsync(deriv + (size_t)p0 * nk * nv, d_q, (size_t)n * nk * nv * sizeof(double),

@@ -167,17 +167,16 @@ struct PD13 {
 void launch_deriv_tables(hipStream_t st, const double *pairs, int npairs, const double *kedges, int nk, int nv,
                          double dxv, int M, double *out);
 // Layout of the signal sums: the modes 0 .. nhalf padded to mpad rows and the
-// redshifts to nzp columns; parts partial tables per pair.
+// redshifts to nzp columns.
 struct SignalGrid {
-    int nhalf, mpad, nzp, parts;
+    int nhalf, mpad, nzp;
 };
 SignalGrid signal_grid(int nhalf, int nz);
 // pk: mpad x nzp
 void launch_pfid_grid(hipStream_t st, const SignalGrid &g, double dk, double z1, double dz, int nz, PD13 pd,
                       double *pk);
-// w2: npairs x mpad, part: parts x npairs x nv x nz (scratch)
+// w2: npairs x mpad (scratch); out: npairs x nv x nz
 void launch_signal_tables(hipStream_t st, const SignalGrid &g, const double *pairs, const int *mend, int npairs,
-                          const double *pk, double dk, double inv_len, int nv, int nz, double *w2, double *part,
-                          double *out);
+                          const double *pk, double dk, double inv_len, int nv, int nz, double *w2, double *out);
 
 }  // namespace qml

@@ -3,6 +3,7 @@ import math
 
 import numpy as np
 import pytest
+import torch
 
 from lyspeq_amd import synth
 from lyspeq_amd.qml import Binning, QMLEngine
@@ -65,3 +66,39 @@ def test_infinite_power_past_the_kept_modes():
     eng.close()
     want = _columns((R_fwhm, 50.0), nv, v_length, nz, range(nz), pd13)
     assert np.max(np.abs(s[0] - want)) < 1e-11 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("nv,nz", [(2, 2), (31, 15), (32, 16), (33, 17), (65, 31), (64, 32), (97, 33), (1601, 48),
+                                   (1600, 49)])
+def test_signal_blocks(nv, nz):
+    """Velocities around the blocks of 32 and redshifts around those of 16 and
+    32; a pair's table does not depend on the others of the call."""
+    print(f"[case] signal blocks {nv} x {nz}", flush=True)
+    pairs, v_length = [(2000, 50.0), (3100, 36.5), (4900, 65.9)], 10.0 * (nv - 1)
+    eng = QMLEngine(BINS)
+    _, s = eng.make_tables(pairs, nv, v_length, nz, synth.PD13_DEFAULT, deriv=False)
+    _, one = eng.make_tables(pairs[1:2], nv, v_length, nz, synth.PD13_DEFAULT, deriv=False)
+    eng.close()
+    assert np.array_equal(s[1], one[0])
+    for p, t in zip(pairs, s):
+        want = _columns(p, nv, v_length, nz, range(nz), synth.PD13_DEFAULT)
+        assert np.max(np.abs(t - want)) < 1e-11 * np.max(np.abs(want))
+
+
+def test_scratch_of_a_large_table():
+    """A signal table of 1.07 GB, whose P_fid grid takes 8.6 GB, is made with 14
+    GB of device memory left: the sums need no further copies of the table."""
+    print("[case] scratch of a large table", flush=True)
+    pair, nv, v_length, nz = (2000, 50.0), 4097, 40960.0, 32767
+    eng = QMLEngine(BINS)
+    eng.make_tables([pair], 65, 640.0, 9, synth.PD13_DEFAULT)      # the kernels are loaded
+    free = torch.cuda.mem_get_info()[0]
+    held = torch.empty(free - (14 << 30), dtype=torch.uint8, device="cuda")
+    try:
+        _, s = eng.make_tables([pair], nv, v_length, nz, synth.PD13_DEFAULT, deriv=False)
+    finally:
+        del held
+        torch.cuda.empty_cache()
+        eng.close()
+    want = _columns(pair, nv, v_length, nz, [0, nz - 1], synth.PD13_DEFAULT)
+    assert np.max(np.abs(s[0][:, [0, nz - 1]] - want)) < 1e-11 * np.max(np.abs(want))
