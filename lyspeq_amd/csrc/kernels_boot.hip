@@ -455,7 +455,8 @@ void launch_bootstrap(hipStream_t st, const ChunkOut *outs, const double *dbt, c
 // 13.3 GB that the pairs read from the L2s take about 1.3 ms, the barriers of the
 // counts the larger part of the rest.
 //
-// Longer columns, NaNs, and brackets that do not close (ties) take a radix
+// Longer columns (more than 8192 values), NaNs, and brackets that do not close
+// (ties) take a radix
 // select over order-preserving 64-bit keys of the FP64 values: eight passes of 8
 // bits, most significant first, each a 256-bin LDS histogram of the values
 // still matching the selected prefix and a block scan that picks the digit
@@ -487,7 +488,7 @@ __device__ __forceinline__ unsigned long long median_term(const double *a, const
 }
 
 constexpr int MED_CAP = 4096;   // keys of the median's 16-bit bin kept in LDS
-constexpr int MED_REGS = 80;    // values per thread held in registers, at most
+constexpr int MED_REGS = 32;    // values per thread held in registers, at most
 
 struct SelectLds {
     unsigned int hist[256];
@@ -796,12 +797,13 @@ static void launch_medians(hipStream_t st, int nboots, int T, double *X, double 
 void launch_boot_median(hipStream_t st, const double *R, int nboots, int T, double *X, double *median,
                         double *mad) {
     k_boot_transpose<<<dim3((T + 63) / 64, (nboots + 63) / 64), 256, 0, st>>>(R, nboots, T, X);
-    // values per thread, by the registers they take (two each): the fewer, the
-    // more workgroups run on a CU
+    // Values per thread, by the registers they take (two each): the fewer, the
+    // more workgroups run on a CU.  455 bands with the copies: 2048 realisations
+    // 2.0 -> 1.6 ms against the radix select, 8192 5.8 -> 4.1.  With 80 values per
+    // thread, two waves run on a SIMD and the counts' masks spill: 8193 5.9 -> 8.0,
+    // 20000 13.9 -> 16.6, so longer columns take the radix select (13.3 at 20000).
     if (nboots <= 256 * 8)
         launch_medians<8>(st, nboots, T, X, median, mad);
-    else if (nboots <= 256 * 32)
-        launch_medians<32>(st, nboots, T, X, median, mad);
     else if (nboots <= 256 * MED_REGS)
         launch_medians<MED_REGS>(st, nboots, T, X, median, mad);
     else

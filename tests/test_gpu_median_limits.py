@@ -1,0 +1,50 @@
+"""The median bootstrap at the limits of its kernels (needs an MI355X): 64
+values are ranked as they are, up to 2048 and up to 8192 are counted in
+registers, longer columns take the radix select.  Bit for bit against a sort by
+order-preserving keys: -0 before +0, NaN past the infinity of its sign."""
+import numpy as np
+import pytest
+
+from lyspeq_amd import synth
+from lyspeq_amd.qml import QMLEngine
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(x):
+    return np.ascontiguousarray(x).view(np.int64)
+
+
+def _median(x):
+    """Of the values in key order: the middle one, or the half-sum of the two."""
+    u = _bits(x)
+    k = np.sort(np.where(u < 0, u ^ np.int64(2**63 - 1), u))
+    v = np.where(k < 0, k ^ np.int64(2**63 - 1), k).view(np.float64)
+    n = v.size
+    return v[n // 2] if n % 2 else (v[n // 2 - 1] + v[n // 2]) / 2
+
+
+def _check(R):
+    eng = QMLEngine(synth.cpu_reference_config(nchunks=1, with_tables=False).binning)
+    med, mad = eng.bootstrap_median(R)
+    eng.close()
+    want = np.array([_median(r) for r in R.T])
+    assert np.array_equal(_bits(med), _bits(want))
+    X = np.ascontiguousarray(R.T) - want[:, None]
+    for i in range(len(X)):
+        for j in range(i, len(X)):
+            w = _median(X[i] * X[j])
+            assert _bits(mad[i, j]) == _bits(w) == _bits(mad[j, i]), (i, j)
+
+
+@pytest.mark.parametrize("nboots", [63, 64, 65, 2047, 2048, 2049, 8191, 8192, 8193, 20480, 20481])
+def test_counts_of_realisations(nboots):
+    print(f"[case] median limits {nboots}", flush=True)
+    rng = np.random.default_rng(nboots)
+    R = rng.standard_normal((nboots, 6))
+    R[:, 1] = np.exp(8 * R[:, 1])                              # many decades
+    R[:, 2] = np.sort(R[:, 2])                                 # an order the sample follows
+    R[:, 3] = np.where(R[:, 3] > 1.5, np.nan, R[:, 3])         # NaN past the rank
+    R[:, 4] = np.where(np.arange(nboots) % 61 == 0, np.nan, R[:, 4] ** 3)
+    R[:, 5] += 0.7 * R[:, 0]
+    _check(R)
