@@ -48,3 +48,10 @@ def test_counts_of_realisations(nboots):
     R[:, 4] = np.where(np.arange(nboots) % 61 == 0, np.nan, R[:, 4] ** 3)
     R[:, 5] += 0.7 * R[:, 0]
     _check(R)
+
+
+@pytest.mark.parametrize("T", [1, 7, 8, 9, 15, 16, 17, 24, 25, 33])
+def test_band_pairs(T):
+    """Every pair of the folded triangle, at whole and partial eights of bands."""
+    print(f"[case] median of {T} bands", flush=True)
+    _check(np.random.default_rng(T).standard_normal((70, T)))
