@@ -23,6 +23,7 @@
 #include "qml_kernels.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <mutex>
 
 namespace qml {
@@ -448,15 +449,18 @@ void launch_bootstrap(hipStream_t st, const ChunkOut *outs, const double *dbt, c
 // wave, give the first pivots; a count is one compare and one population count
 // per 64 values and one barrier, and the next pivot follows from it, first among
 // the sorted sample, then by interpolation between the bracket's ends; what is
-// left at 64 values or fewer is ranked exactly.  Eight counts are typical.  The
-// values are read once; the radix select below reads them three times and its
-// waves queue on the few histogram bins that hold a band pair's exponents.  455
-// bands x 8000 realisations: 4.65 -> 2.77 ms for the 103740 pairs, of which the
-// 13.3 GB that the pairs read from the L2s take about 1.3 ms, the barriers of the
-// counts the larger part of the rest.
+// left at 64 values or fewer is ranked exactly.  Eight counts are typical.  Where
+// two pivots have nothing between them, the least value of the bracket and its
+// copies are counted: a median with many equal values ends there.  The values are
+// read once; the radix select below reads them three times and its waves queue on
+// the few histogram bins that hold a band pair's exponents.  Bound by the barriers
+// and compares of the counts.  Whole calls with the copies: 455 bands x 8000
+// realisations 5.7 -> 3.3 ms, x 500 1.29 -> 1.04; 200 bands of whole numbers x 8000
+// 2.3 -> 0.89, x 500 0.38 -> 0.23 (2.7 and 0.65 where counting gave up on equal
+// values and the radix select followed).
 //
-// Longer columns (more than 8192 values), NaNs, and brackets that do not close
-// (ties) take a radix
+// Longer columns (more than 8192 values), NaNs, and brackets with an end at
+// infinity or whose copies part the two ranks of an even count take a radix
 // select over order-preserving 64-bit keys of the FP64 values: eight passes of 8
 // bits, most significant first, each a 256-bin LDS histogram of the values
 // still matching the selected prefix and a block scan that picks the digit
@@ -579,6 +583,12 @@ __device__ __forceinline__ double lane_value(double x, int lane) {   // lane is 
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+// The next double above x < infinity.
+__device__ __forceinline__ double value_above(double x) {
+    const long long u = __double_as_longlong(x);
+    return x == 0.0 ? __longlong_as_double(1) : __longlong_as_double(x > 0.0 ? u + 1 : u - 1);
+}
+
 // The median of the n <= 256 R values by counting (see above); false where it
 // is left to the radix select.  Called by all 256 threads.
 template <bool PROD, int R>
@@ -588,11 +598,20 @@ __device__ bool count_median(const double *a, const double *b, int n, SelectLds 
     const int r0 = two ? n / 2 - 1 : n / 2, r1 = r0 + two;   // the ranks wanted
     double v[R];
     bool nan = false;
+    constexpr int G = R < 8 ? R : 8;
 #pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const int i = tid + 256 * k;
-        v[k] = i < n ? (PROD ? a[i] * b[i] : a[i]) : __builtin_inf();   // never below a pivot
-        nan |= v[k] != v[k];
+    for (int g = 0; g < R; g += G) {   // eight loads in flight, none behind a test of its own
+#pragma unroll
+        for (int k = g; k < g + G; ++k) v[k] = __builtin_inf();   // never below a pivot
+        if (R == G || 256 * g < n) {
+#pragma unroll
+            for (int k = g; k < g + G; ++k) {
+                const int i = tid + 256 * k, e = min(i, n - 1);
+                const double x = PROD ? a[e] * b[e] : a[e];
+                nan |= x != x;
+                v[k] = i < n ? x : __builtin_inf();
+            }
+        }
     }
     // the same sorted sample in every wave, one value a lane
     double smp;
@@ -610,10 +629,52 @@ __device__ bool count_median(const double *a, const double *b, int n, SelectLds 
     if (tid == 0) s.ncand = 0;
     if (lane == 0) s.wave_min[wave] = 0;
     if (__any(nan) && lane == 0) s.wave_min[wave] = 1;
+    int turn = 0;
+    auto total = [&](int c) {   // over the waves
+        unsigned int *tot = s.hist + 4 * (turn++ & 1);
+        if (lane == 0) tot[wave] = (unsigned int)c;
+        __syncthreads();
+        return __builtin_amdgcn_readfirstlane((int)(tot[0] + tot[1] + tot[2] + tot[3]));
+    };
     // values below pl: cl <= r0 of them; below ph: ch > r1
     int cl = 0, ch = n, L = -1, H = 64, m = (int)((long long)r0 * 64 / n);
     double pl = -__builtin_inf(), ph = __builtin_inf();
     bool open = true;   // no upper end yet
+    // The least value t not below pl: 1 if both ranks lie among its copies, else 0
+    // with the lower end past them, or 2 where the copies part the ranks.
+    auto settle = [&]() -> int {
+        double t = __builtin_inf();
+#pragma unroll
+        for (int k = 0; k < R; ++k) t = v[k] >= pl ? fmin(t, v[k]) : t;
+        for (int d = 1; d < 64; d *= 2) t = fmin(t, __shfl_xor(t, d, 64));
+        if (lane == 0) s.wave_min[wave] = (unsigned long long)__double_as_longlong(t);
+        __syncthreads();
+        t = fmin(fmin(__longlong_as_double((long long)s.wave_min[0]), __longlong_as_double((long long)s.wave_min[1])),
+                 fmin(__longlong_as_double((long long)s.wave_min[2]), __longlong_as_double((long long)s.wave_min[3])));
+        t = lane_value(t, 0);   // uniform, and so the next pivots
+        if (!(t < __builtin_inf())) return 2;
+        int c = 0, z = 0;
+#pragma unroll
+        for (int k = 0; k < R; ++k) c += __popcll(__ballot(v[k] <= t));
+        c = total(c);
+        if (c <= r0) {
+            cl = c;
+            pl = value_above(t);
+            return 0;
+        }
+        if (c <= r1) return 2;
+        if (t == 0.0) {   // -0 sorts before +0
+#pragma unroll 1
+            for (int i = tid; i < (n + 255) / 256 * 256; i += 256) {
+                const double x = i < n ? (PROD ? a[i] * b[i] : a[i]) : 0.0;
+                z += __popcll(__ballot(__double_as_longlong(x) == LLONG_MIN));
+            }
+            z = total(z) + cl;
+        }
+        const double lo = t == 0.0 ? (r0 < z ? -0.0 : 0.0) : t, hi = t == 0.0 ? (r1 < z ? -0.0 : 0.0) : t;
+        median = two ? (lo + hi) / 2 : lo;
+        return 1;
+    };
     for (int step = 0; ch - cl > 64; ++step) {
         if (step == 24) return false;
         double p;
@@ -626,13 +687,11 @@ __device__ bool count_median(const double *a, const double *b, int n, SelectLds 
         int c = 0;
 #pragma unroll
         for (int k = 0; k < R; ++k) c += __popcll(__ballot(v[k] < p));
-        unsigned int *tot = s.hist + 4 * (step & 1);
-        if (lane == 0) tot[wave] = (unsigned int)c;
-        __syncthreads();
-        c = __builtin_amdgcn_readfirstlane((int)(tot[0] + tot[1] + tot[2] + tot[3]));
+        c = total(c);
         if (step == 0 && (s.wave_min[0] | s.wave_min[1] | s.wave_min[2] | s.wave_min[3])) return false;
         const bool below = c <= r0, above = c > r1;
         if (!below && !above) return false;   // the pivot parts the two ranks
+        const bool still = c == (below ? cl : ch);
         if (below) {
             cl = c;
             pl = p;
@@ -641,6 +700,7 @@ __device__ bool count_median(const double *a, const double *b, int n, SelectLds 
             ph = p;
             open = false;
         }
+        bool stuck = false;
         if (H - L > 1) {
             // the sample's own spacing to the rank, then one further, so that the
             // next count closes the bracket from the other side
@@ -649,7 +709,14 @@ __device__ bool count_median(const double *a, const double *b, int n, SelectLds 
             const int d = (int)((long long)(r0 - c) * 64 / n);
             m = m + d + (below ? 1 : -1);
             m = max(L + 1, min(H - 1, m));
-            if (H - L <= 1 && (open || L < 0 || !(ph - pl < __builtin_inf()))) return false;
+            stuck = (below && still) || (H - L <= 1 && (open || L < 0 || !(ph - pl < __builtin_inf())));
+        } else {
+            stuck = still;   // nothing between the last two pivots
+        }
+        if (stuck) {   // many equal values, or an end at infinity
+            const int r = settle();
+            if (r == 1) return true;
+            if (r == 2 || (H - L <= 1 && (open || !(ph - pl < __builtin_inf())))) return false;
         }
     }
     __syncthreads();
@@ -763,7 +830,7 @@ __global__ __launch_bounds__(256) void k_boot_transpose(const double *R, int nbo
 // One block per band: median[i], then X[i][:] -= median[i] (_calcuateMedian,
 // and the subtraction at the start of _calcuateMadCovariance).
 template <int R>
-__global__ __launch_bounds__(256) void k_boot_median(double *X, int nboots, double *median) {
+__global__ __launch_bounds__(256, 4) void k_boot_median(double *X, int nboots, double *median) {
     __shared__ SelectLds s;
     double *x = X + (size_t)blockIdx.x * nboots;
     const double m = block_median<false, R>(x, x, nboots, s);
@@ -781,7 +848,7 @@ __global__ __launch_bounds__(256) void k_boot_median(double *X, int nboots, doub
 // 12.8 -> 12.7; 200 bands of 20000 3.2 -> 2.8, 257 of 12000 3.0 -> 2.4 (folded
 // with a width of T + 1, where a band is read on every XCD).
 template <int R>
-__global__ __launch_bounds__(256) void k_boot_mad(const double *X, int nboots, int T, double *mad) {
+__global__ __launch_bounds__(256, 4) void k_boot_mad(const double *X, int nboots, int T, double *mad) {
     const int x = blockIdx.x, y = blockIdx.y, up = (int)gridDim.x - y / 8 * 8;
     const bool left = x < y / 8 * 8;
     const int i = left ? up + y % 8 : y, j = left ? x + up : x;
@@ -804,12 +871,15 @@ static void launch_medians(hipStream_t st, int nboots, int T, double *X, double 
 void launch_boot_median(hipStream_t st, const double *R, int nboots, int T, double *X, double *median,
                         double *mad) {
     k_boot_transpose<<<dim3((T + 63) / 64, (nboots + 63) / 64), 256, 0, st>>>(R, nboots, T, X);
-    // Values per thread, by the registers they take (two each): the fewer, the
-    // more workgroups run on a CU.  455 bands with the copies: 2048 realisations
-    // 2.0 -> 1.6 ms against the radix select, 8192 5.8 -> 4.1.  With 80 values per
-    // thread, two waves run on a SIMD and the counts' masks spill: 8193 5.9 -> 8.0,
-    // 20000 13.9 -> 16.6, so longer columns take the radix select (13.3 at 20000).
-    if (nboots <= 256 * 8)
+    // Values per thread, by the registers they take (two each) and the loads and
+    // compares past the column's end: 455 bands with the copies, 500 realisations
+    // 1.04 ms with 2, 1.13 with 8 (radix select 1.29), 2048 1.50 with 8 (2.0), 8000
+    // 3.3 with 32 (5.7).  With 80, two waves run on a SIMD and the counts' masks
+    // spill: 8193 5.9 -> 8.0, 20000 13.9 -> 16.6, so longer columns take the radix
+    // select (12.7 at 20000).
+    if (nboots <= 256 * 2)
+        launch_medians<2>(st, nboots, T, X, median, mad);
+    else if (nboots <= 256 * 8)
         launch_medians<8>(st, nboots, T, X, median, mad);
     else if (nboots <= 256 * MED_REGS)
         launch_medians<MED_REGS>(st, nboots, T, X, median, mad);

@@ -1,5 +1,5 @@
 """The median bootstrap at the limits of its kernels (needs an MI355X): 64
-values are ranked as they are, up to 2048 and up to 8192 are counted in
+values are ranked as they are, up to 512, 2048 and 8192 are counted in
 registers, longer columns take the radix select.  Bit for bit against a sort by
 order-preserving keys: -0 before +0, NaN past the infinity of its sign."""
 import numpy as np
@@ -24,10 +24,15 @@ def _median(x):
     return v[n // 2] if n % 2 else (v[n // 2 - 1] + v[n // 2]) / 2
 
 
-def _check(R):
+def _run(R):
     eng = QMLEngine(synth.cpu_reference_config(nchunks=1, with_tables=False).binning)
     med, mad = eng.bootstrap_median(R)
     eng.close()
+    return med, mad
+
+
+def _check(R):
+    med, mad = _run(R)
     want = np.array([_median(r) for r in R.T])
     assert np.array_equal(_bits(med), _bits(want))
     X = np.ascontiguousarray(R.T) - want[:, None]
@@ -37,7 +42,7 @@ def _check(R):
             assert _bits(mad[i, j]) == _bits(w) == _bits(mad[j, i]), (i, j)
 
 
-@pytest.mark.parametrize("nboots", [63, 64, 65, 2047, 2048, 2049, 8191, 8192, 8193, 20480, 20481])
+@pytest.mark.parametrize("nboots", [63, 64, 65, 511, 512, 513, 2047, 2048, 2049, 8191, 8192, 8193, 20480, 20481])
 def test_counts_of_realisations(nboots):
     print(f"[case] median limits {nboots}", flush=True)
     rng = np.random.default_rng(nboots)
@@ -55,3 +60,47 @@ def test_band_pairs(T):
     """Every pair of the folded triangle, at whole and partial eights of bands."""
     print(f"[case] median of {T} bands", flush=True)
     _check(np.random.default_rng(T).standard_normal((70, T)))
+
+
+@pytest.mark.parametrize("nboots", [66, 101, 512, 513, 2000, 2049, 8000, 8191, 8194])
+def test_equal_values(nboots):
+    """Columns whose median has many copies: whole and tenth values, one value,
+    zeros of both signs, two values that part the two ranks or nearly so, a value
+    repeated at few places, infinities on both sides and on the median."""
+    print(f"[case] median of equal values {nboots}", flush=True)
+    rng = np.random.default_rng(nboots + 1)
+    g = rng.standard_normal((nboots, 12))
+    n = np.arange(nboots)
+    R = g.copy()
+    R[:, 0] = np.round(g[:, 0])
+    R[:, 1] = np.round(g[:, 1], 1)
+    R[:, 2] = 3.25
+    R[:, 3] = np.copysign(0.0, g[:, 3])
+    R[:, 4] = np.where(np.abs(g[:, 4]) < 0.5, np.copysign(0.0, g[:, 5]), g[:, 4])
+    R[:, 5] = np.where(n < nboots // 2, -1.0, 2.0)             # one value for each rank where nboots is even
+    R[:, 6] = np.where(n < nboots // 2 + 1, -1.0, 2.0)
+    R[:, 7] = np.where(n % 50 == 3, np.median(g[:, 7]), g[:, 7])
+    R[:, 8] = rng.poisson(1.0, nboots)
+    R[:, 9] = np.where(np.abs(g[:, 9]) > 1.2, np.copysign(np.inf, g[:, 9]), np.abs(g[:, 9]) + 1.0)
+    R[:, 10] = np.round(g[:, 10], 2)
+    R[:, 11] = np.exp(6 * np.round(g[:, 11], 1))
+    med, mad = _run(R)
+    want = np.array([_median(r) for r in R.T])
+    assert np.array_equal(_bits(med), _bits(want))
+    X = np.ascontiguousarray(R.T) - want[:, None]
+    for i in range(12):
+        for j in range(i, 12):
+            p = X[i] * X[j]
+            if np.isnan(p).any():      # infinity times zero: the sign of that NaN is the machine's
+                continue
+            assert _bits(mad[i, j]) == _bits(_median(p)) == _bits(mad[j, i]), (i, j)
+
+
+def test_infinite_medians():
+    """A median among equal infinities, on its own."""
+    print("[case] infinite medians", flush=True)
+    for nboots in (100, 3000):
+        n = np.arange(nboots)
+        R = np.stack([np.where(n % 3 == 0, 1.0 + n, np.inf), np.where(n % 3 == 0, 1.0 + n, -np.inf)], axis=1)
+        med, _ = _run(R)
+        assert np.array_equal(med, [np.inf, -np.inf])
