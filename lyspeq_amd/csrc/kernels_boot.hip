@@ -90,9 +90,10 @@ __global__ __launch_bounds__(256) void k_boot_realize(const int *P, const double
         }
 }
 
-// Sums over a range of realisations, blockIdx.y of gridDim.y: part[y][i].  One
-// thread per band ran down all realisations (968 us at 4000 x 455).
-__global__ __launch_bounds__(256) void k_boot_mean_part(const double *R, int nboots, int T, double *part) {
+// Sums over a range of realisations, blockIdx.y of gridDim.y: part[y][i], or the
+// mean itself where there is one range.  One thread per band ran down all
+// realisations (968 us at 4000 x 455).
+__global__ __launch_bounds__(256) void k_boot_mean_part(const double *R, int nboots, int T, double *part, double *mean) {
     __shared__ double red[4][64];
     const int l = threadIdx.x % 64, w = threadIdx.x / 64, i = blockIdx.x * 64 + l;
     const int b0 = (int)((long long)nboots * blockIdx.y / gridDim.y);
@@ -103,7 +104,10 @@ __global__ __launch_bounds__(256) void k_boot_mean_part(const double *R, int nbo
         for (int b = b0 + w; b < b1; b += 4) s += R[(size_t)b * T + i];
     red[w][l] = s;
     __syncthreads();
-    if (w == 0 && i < T) part[(size_t)blockIdx.y * T + i] = (red[0][l] + red[1][l]) + (red[2][l] + red[3][l]);
+    if (w != 0 || i >= T) return;
+    s = (red[0][l] + red[1][l]) + (red[2][l] + red[3][l]);
+    if (gridDim.y == 1) mean[i] = s * (1.0 / nboots);
+    else part[(size_t)blockIdx.y * T + i] = s;
 }
 __global__ __launch_bounds__(256) void k_boot_mean(const double *part, int nparts, int nboots, int T, double *mean) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -118,10 +122,17 @@ __global__ __launch_bounds__(256) void k_boot_mean(const double *part, int npart
 // realisations, a quarter of it per wave, whose 16 blocks of 16 x 16 stay in
 // registers; a fragment is 16 consecutive bands of four realisations, loaded
 // one step ahead.  36 tiles at T = 455 would leave the chip empty without the
-// split over realisations (798 us at 4000 x 455 with one workgroup a tile).
+// split over realisations (798 us at 4000 x 455 with one workgroup a tile).  Where
+// there is one range (under 32 realisations) the covariance itself is written,
+// here and by k_boot_mean_part: a call of two realisations is a few launches.
+__device__ __forceinline__ void put_cov(double *cov, int T, int i, int j, double c) {
+    if (i >= T || j >= T || j < i) return;
+    cov[(size_t)i * T + j] = c;
+    cov[(size_t)j * T + i] = c;
+}
 typedef double bd4 __attribute__((ext_vector_type(4)));
 __global__ __launch_bounds__(256, 2) void k_boot_cov_part(const double *R, const double *mean, int nboots, int T,
-                                                          double *part) {
+                                                          double *part, double *cov) {
     __shared__ double red[2][4][256];
     int t = blockIdx.x, J = 0;   // tile t of the upper triangle by columns: I <= J
     while (t > J) { t -= J + 1; ++J; }
@@ -176,8 +187,10 @@ __global__ __launch_bounds__(256, 2) void k_boot_cov_part(const double *R, const
 #pragma unroll
             for (int u = 0; u < 4; ++u) red[flip][w][64 * u + lane] = acc[x][y][u];
             __syncthreads();
-            C[(16 * x + tid / 16) * BT + 16 * y + tid % 16] =
-                (red[flip][0][tid] + red[flip][1][tid]) + (red[flip][2][tid] + red[flip][3][tid]);
+            const double c = (red[flip][0][tid] + red[flip][1][tid]) + (red[flip][2][tid] + red[flip][3][tid]);
+            const int i = 16 * x + tid / 16, j = 16 * y + tid % 16;
+            if (gridDim.y > 1) C[i * BT + j] = c;
+            else put_cov(cov, T, 64 * I + i, 64 * J + j, c * (1.0 / (nboots - 1)));
             flip ^= 1;
         }
 }
@@ -189,12 +202,9 @@ __global__ __launch_bounds__(256) void k_boot_cov(const double *part, int nparts
     const double scale = 1.0 / (nboots - 1);
     for (int e = blockIdx.y * 256 + threadIdx.x; e < BT * BT; e += 256 * gridDim.y) {
         const int i = I * BT + e / BT, j = J * BT + e % BT;
-        if (i >= T || j >= T || j < i) continue;
         double s = 0.0;
         for (int p = 0; p < nparts; ++p) s += part[((size_t)p * gridDim.x + blockIdx.x) * BT * BT + e];
-        s *= scale;
-        cov[(size_t)i * T + j] = s;
-        cov[(size_t)j * T + i] = s;
+        put_cov(cov, T, i, j, s * scale);
     }
 }
 
@@ -420,10 +430,10 @@ size_t boot_meancov_scratch(int nboots, int T) {
 void launch_boot_meancov(hipStream_t st, const double *R, int nboots, int T, double *scratch, double *mean,
                          double *cov) {
     const int nt = (T + BT - 1) / BT, tiles = nt * (nt + 1) / 2, mp = mean_parts(nboots), cp = cov_parts(nboots, T);
-    k_boot_mean_part<<<dim3(nt, mp), 256, 0, st>>>(R, nboots, T, scratch);
-    k_boot_mean<<<(T + 255) / 256, 256, 0, st>>>(scratch, mp, nboots, T, mean);
-    k_boot_cov_part<<<dim3(tiles, cp), 256, 0, st>>>(R, mean, nboots, T, scratch);
-    k_boot_cov<<<dim3(tiles, 4), 256, 0, st>>>(scratch, cp, nboots, T, cov);
+    k_boot_mean_part<<<dim3(nt, mp), 256, 0, st>>>(R, nboots, T, scratch, mean);
+    if (mp > 1) k_boot_mean<<<(T + 255) / 256, 256, 0, st>>>(scratch, mp, nboots, T, mean);
+    k_boot_cov_part<<<dim3(tiles, cp), 256, 0, st>>>(R, mean, nboots, T, scratch, cov);
+    if (cp > 1) k_boot_cov<<<dim3(tiles, 4), 256, 0, st>>>(scratch, cp, nboots, T, cov);
 }
 
 void launch_bootstrap(hipStream_t st, const ChunkOut *outs, const double *dbt, const int *qptr, const int *qchunk,

@@ -1960,7 +1960,7 @@ int qml_make_tables(qml_ctx *c, const qml_table_spec *s, int npairs, const int *
     // pairs per pass: outputs of up to 2 GiB on the device
     const size_t per = (size_t)8 * ((deriv ? (size_t)nk * nv : 0) + (signal ? (size_t)nv * nz : 0));
     const int nb = (int)std::max<size_t>(1, std::min<size_t>(npairs, ((size_t)2 << 30) / per));
-    // one allocation for all arrays: a small call's time is mostly theirs
+    // one allocation for all arrays
     size_t total = 0;
     auto place = [&](size_t doubles) {
         const size_t at = total;
