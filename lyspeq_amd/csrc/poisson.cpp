@@ -14,6 +14,7 @@
 // exp(-1), which never rise); the draws then hop from start to start.
 #include "poisson.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 
@@ -39,9 +40,9 @@ inline uint64_t twist(uint64_t cur, uint64_t next, uint64_t far) {
     return far ^ (x >> 1) ^ ((0 - (x & 1)) & MT_A);
 }
 
-// BLOCKS regenerations of the state into uniforms u[0 .. LEN).
-QML_CLONES void uniforms(uint64_t *mt, double *u) {
-    for (int b = 0; b < BLOCKS; ++b) {
+// `blocks` regenerations of the state into uniforms u[0 .. blocks MT_N).
+QML_CLONES void uniforms(uint64_t *mt, double *u, int blocks) {
+    for (int b = 0; b < blocks; ++b) {
         for (int i = 0; i < MT_M; ++i) mt[i] = twist(mt[i], mt[i + 1], mt[i + MT_M]);
         for (int i = MT_M; i < MT_N - 1; ++i) mt[i] = twist(mt[i], mt[i + 1], mt[i - MT_M]);
         mt[MT_N - 1] = twist(mt[MT_N - 1], mt[0], mt[MT_M - 1]);
@@ -85,17 +86,21 @@ void poisson_draws(uint64_t seed, long long count, int *out) {
     double u[TAIL + LEN];   // on the stack (60 KB): a C entry allocates nothing here
     int n[TAIL + LEN];
     int have = 0, at = 0, ready = 0;   // uniforms in the window, the next one, starts with a count
-    const auto refill = [&]() {
+    // left: draws still to make, two uniforms each on average.  The few of a short
+    // call come from one block: one draw through Python takes 6.9 us on a Xeon
+    // host, 13.0 with all 16 blocks (the library's generator 6.9).
+    const auto refill = [&](long long left) {
         const int keep = have - at;   // at most TAIL
         for (int i = 0; i < keep; ++i) u[i] = u[at + i];
-        uniforms(mt, u + keep);
-        have = keep + LEN;
+        const int blocks = left > LEN / 2 ? BLOCKS : (int)(2 * left + TAIL) / MT_N + 1;
+        uniforms(mt, u + keep, std::min(blocks, BLOCKS));
+        have = keep + std::min(blocks, BLOCKS) * MT_N;
         at = 0;
         ready = have - LOOK;
         counts(u, stop, ready, n);
     };
     for (long long i = 0; i < count; ++i) {
-        if (at >= ready) refill();
+        if (at >= ready) refill(count - i);
         int k = n[at];
         if (k <= LOOK) {
             at += k;
@@ -103,7 +108,7 @@ void poisson_draws(uint64_t seed, long long count, int *out) {
             double p = 1.0;
             k = 0;
             do {
-                if (at == have) refill();
+                if (at == have) refill(count - i);
                 p *= u[at++];
                 ++k;
             } while (p > stop);

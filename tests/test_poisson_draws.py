@@ -37,3 +37,11 @@ def test_draws_are_the_standard_librarys(std_draws, seed, n):
     assert np.array_equal(poisson_draws(seed, n), want)
     if n == 2000000:
         assert want.max() >= 8
+
+
+def test_short_calls_are_prefixes(std_draws):
+    """A call makes as many blocks of uniforms as its count needs: every count
+    up to three blocks and some around the full window gives the same draws."""
+    want = std_draws(11, 6000)
+    for n in list(range(1, 480)) + [2480, 2481, 2495, 2496, 2497, 2500, 2501, 4991, 4992, 5999]:
+        assert np.array_equal(poisson_draws(11, n), want[:n]), n
