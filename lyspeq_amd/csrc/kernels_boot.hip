@@ -266,7 +266,8 @@ __global__ __launch_bounds__(256) void k_boot_collapse_fisher(const ChunkOut *ou
 
 // The batch's weights as doubles, realisation contiguous: Wt[q][b], zero past nb.
 __global__ __launch_bounds__(256) void k_boot_weights(const int *W, int nqso, int b0, int nb, double *Wt) {
-    const int e = blockIdx.x * 256 + threadIdx.x, q = e / BOOT_BATCH, b = e % BOOT_BATCH;
+    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;   // nqso BOOT_BATCH may exceed 32 bits
+    const int q = (int)(e / BOOT_BATCH), b = (int)(e % BOOT_BATCH);
     if (q < nqso) Wt[e] = (b < nb) ? (double)W[(size_t)(b0 + b) * nqso + q] : 0.0;
 }
 
