@@ -49,3 +49,33 @@ def test_mean_and_covariance_ranges(run, nboots):
     mo, co = ob.mean_covariance(R)
     assert _rel(R, Ro) < 1e-12 and _rel(mean, mo) < 1e-12 and _rel(cov, co) < 1e-11
     assert np.array_equal(cov, cov.T)
+
+
+@pytest.mark.parametrize("nboots", [127, 128, 129, 160, 161, 256, 290])
+def test_complete_bootstrap_batches(run, nboots):
+    """Realisations are solved 128 at a time: full batches, a tail of one, tails
+    around a group of 32, with an empty realisation (every weight zero) and one
+    whose Fisher matrix is not positive definite in the first and in each later
+    batch.  The bar is that of two Cholesky solves, 20 n cond eps."""
+    print(f"[case] complete bootstrap of {nboots}", flush=True)
+    eng, qso, nqso, col, fis = run
+    rng = np.random.default_rng(nboots)
+    W = rng.integers(1, 4, (nboots, nqso)).astype(np.int32)
+    empty = [b for b in (5, 130, 260) if b < nboots]
+    bad = [b for b in (40, 128, 200, 289) if b < nboots]
+    W[empty] = 0
+    W[bad, rng.integers(0, nqso, len(bad))] = -3
+    X, valid, mean, cov = eng.bootstrap_complete(nboots, qso, nqso, weights=W)
+    Xo, vo, systems = ob.complete_realizations(W, col, fis, eng.T, return_systems=True)
+    assert np.array_equal(valid, vo) and X.shape == Xo.shape
+    assert not valid[bad].any() and valid[empty].all() and valid.sum() == nboots - len(bad)
+    at = np.cumsum(valid) - 1
+    assert not X[at[empty]].any()
+    eps = np.finfo(float).eps
+    for xb, xo, (S, _) in zip(X, Xo, systems):
+        d = np.sqrt(np.diag(S))
+        scale = np.max(np.abs(xo * d))
+        if scale > 0:
+            assert np.max(np.abs((xb - xo) * d)) / scale < 20 * eng.T * np.linalg.cond(S / np.outer(d, d)) * eps
+    mg, cg = ob.mean_covariance(X)
+    assert _rel(mean, mg) < 1e-12 and _rel(cov, cg) < 1e-11
