@@ -135,7 +135,8 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
 
     // 1/(pi v) of this thread's entries in every pass (v = u_b - u_a does not
     // depend on the edge); the entry on the shared grid point (v = 0, at most
-    // one per pass and column) gets 0 here and k_e/pi written after the rest
+    // one per pass and column) gets 0 here and k_e/pi written after the rest.
+    // Points past the grid, which stand on its last one, take no part
     const int elast = c.ngrp ? -1 : kbu;          // the bands of a chunk with groups come from k_rm_bands
     double inv[NPM][EM];
     int dsel[NPM];
@@ -146,7 +147,7 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
 #pragma unroll
         for (int s = 0; s < EM; ++s) {
             const double d = (ub - ush[ar0 + 8 * s]) * RM_PI;
-            const bool live = p < npass && ar0 + 8 * s < ra;
+            const bool live = p < npass && ar0 + 8 * s < ra && amin + ar0 + 8 * s < M && bmin + p * RM_BW + bb < M;
             inv[p][s] = (live && d != 0.0) ? 1.0 / d : 0.0;
             if (live && d == 0.0) dsel[p] = s;
         }
