@@ -42,15 +42,14 @@
 // matrix gets nelem/2 extrapolated grid points on each side, whose weights
 // are zero), so every tap loop below has the same trip count.
 //
-// S is formed by k_rm_signal, unless R's rows are too long for its LDS (more than
-// about 55 taps): then it is k_rm_sandwich's first pass, for every chunk.
+// S is formed by k_rm_signal, the Q_k of a chunk without groups by k_rm_sandwich:
+// each chunk by its own shape, whatever the others of its batch.
 //
 // k_rm_sandwich<TJ>: one 16 x TJ output tile (I0.., J0..) per block, tiles
 // touching the upper triangle only.  The fine rows of its 16 R rows (the a
 // range, 15 ros + rnb) and the fine columns of its TJ R columns (the b range,
-// (TJ-1) ros + rnb, in passes of 32) are fixed for the block.  Per edge e
-// (and first for S, where asked):
-//   per pass:  Qh (a x 32, LDS) <- P_e(a, b), or Shat
+// (TJ-1) ros + rnb, in passes of 32) are fixed for the block.  Per edge e:
+//   per pass:  Qh (a x 32, LDS) <- P_e(a, b)
 //              T  (16 x b, LDS) <- R_I Qh                  (rnb taps, FP64 FMA)
 //   Z[i][j] = sum_t T[i][j ros + t] R[j][t]                (rnb taps, registers)
 //   Q_e-1 = Z_e - Z_e-1 written to the upper triangle and mirrored, as
@@ -68,13 +67,13 @@ constexpr int RM_QP = 33;    // row pitch of Qh (doubles)
 }  // namespace
 
 template <int TJ, int EM, int NPM>
-__global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const double *rin, const TableDev *tabs,
-                                                     BinsDev bins, RmLayout lay, int signal, double *mat) {
+__global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const double *rin, BinsDev bins, RmLayout lay,
+                                                     double *mat) {
     constexpr int NO = TJ / 16;                   // outputs per thread
     // EM: Qh entries per thread (rows ar0 + 8 s, s < EM); 8 EM >= 15 ros + rnb.
     // NPM: passes at most ((TJ - 1) ros + rnb <= 32 NPM), their 1/(pi v) kept in registers
     const ChunkDev c = cs[blockIdx.z];
-    if (!c.rm || (c.ngrp && !signal)) return;
+    if (!c.rm || c.ngrp) return;   // the bands of a chunk with groups come from k_rm_bands
     const int Np = c.Np, N = c.N, M = c.rM, nb = c.rnb, os = c.ros, kbu = c.kbu;
     const int I0 = blockIdx.y * 16, J0 = blockIdx.x * TJ;
     if (I0 >= Np || J0 >= Np || J0 + TJ - 1 < I0) return;
@@ -86,7 +85,7 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
         for (int o = 0; o < NO; ++o) {
             const int j = J0 + tj + 16 * o;
             if (j < i) continue;
-            for (int k = c.ngrp ? kbu : 0; k < kbu + signal; ++k) {
+            for (int k = 0; k < kbu; ++k) {
                 Qb[k * NN + (size_t)i * Np + j] = 0.0;
                 Qb[k * NN + (size_t)j * Np + i] = 0.0;
             }
@@ -95,7 +94,6 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
     }
     const double *R = rin + c.rin_off;            // N x nb
     const double *grid = R + (size_t)N * nb;      // M wavelengths (units of lambda_Lya)
-    const TableDev t = tabs[c.table];
     const int amin = c.rcol0 + I0 * os, ra = 15 * os + nb;
     const int bmin = c.rcol0 + J0 * os, rb = (TJ - 1) * os + nb;
     const int npass = (rb + RM_BW - 1) / RM_BW;
@@ -137,7 +135,6 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
     // depend on the edge); the entry on the shared grid point (v = 0, at most
     // one per pass and column) gets 0 here and k_e/pi written after the rest.
     // Points past the grid, which stand on its last one, take no part
-    const int elast = c.ngrp ? -1 : kbu;          // the bands of a chunk with groups come from k_rm_bands
     double inv[NPM][EM];
     int dsel[NPM];
 #pragma unroll
@@ -153,50 +150,28 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
         }
     }
 
-    for (int e = signal ? -1 : 0; e <= elast; ++e) {
-        double kpi = 0.0;
-        if (e >= 0) {
-            const double ke = bins.ke[e];
-            kpi = ke / RM_PI;
-            for (int p = tid; p < npts; p += 256) {
-                double sv, cv;
-                sincos(ke * ush[p], &sv, &cv);
-                scs[p] = make_double2(sv, cv);
-            }
-            __syncthreads();
+    for (int e = 0; e <= kbu; ++e) {
+        const double ke = bins.ke[e], kpi = ke / RM_PI;
+        for (int p = tid; p < npts; p += 256) {
+            double sv, cv;
+            sincos(ke * ush[p], &sv, &cv);
+            scs[p] = make_double2(sv, cv);
         }
+        __syncthreads();
         // the a points' (sin, cos) at this edge: the same in every pass
         double2 sa[EM];
-        if (e >= 0) {
 #pragma unroll
-            for (int s = 0; s < EM; ++s) sa[s] = scs[ar0 + 8 * s];
-        }
+        for (int s = 0; s < EM; ++s) sa[s] = scs[ar0 + 8 * s];
 #pragma unroll
         for (int p = 0; p < NPM; ++p) {
             if (p >= npass) break;
             const int pc = p * RM_BW + bb;
-            if (e < 0) {
-                const int gb = min(M - 1, bmin + pc);
-                const double lb = grid[gb];
-#pragma unroll 4
-                for (int s = 0; s < EM; ++s) {
-                    const int a = ar0 + 8 * s, ga = min(M - 1, amin + a);
-                    double val = 0.0;
-                    if (!bins.turn_off_sfid) {
-                        double v, z;
-                        vz_pair(grid[ga], lb, ga, gb, v, z);
-                        val = signal_interp(t, z, v);
-                    }
-                    Qh[a * RM_QP + bb] = val;
-                }
-            } else {
-                // rows past the a range fill Qh rows that the T step never reads
-                const double2 sb = scs[ra + pc];
+            // rows past the a range fill Qh rows that the T step never reads
+            const double2 sb = scs[ra + pc];
 #pragma unroll
-                for (int s = 0; s < EM; ++s)
-                    Qh[(ar0 + 8 * s) * RM_QP + bb] = (sb.x * sa[s].y - sb.y * sa[s].x) * inv[p][s];
-                if (dsel[p] >= 0) Qh[(ar0 + 8 * dsel[p]) * RM_QP + bb] = kpi;
-            }
+            for (int s = 0; s < EM; ++s)
+                Qh[(ar0 + 8 * s) * RM_QP + bb] = (sb.x * sa[s].y - sb.y * sa[s].x) * inv[p][s];
+            if (dsel[p] >= 0) Qh[(ar0 + 8 * dsel[p]) * RM_QP + bb] = kpi;
             __syncthreads();
             double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0;
             int tt = 0;
@@ -254,22 +229,20 @@ __global__ __launch_bounds__(256) void k_rm_sandwich(const ChunkDev *cs, const d
             if (tt < nb) s0 += tr[tt] * rr[tt];
             z[o] = s0 + s1;
         }
-        if (e != 0) {
-            double *Q = Qb + (size_t)(e < 0 ? kbu : e - 1) * NN;
+        if (e > 0) {
+            double *Q = Qb + (size_t)(e - 1) * NN;
 #pragma unroll
             for (int o = 0; o < NO; ++o) {
                 const int j = J0 + tj + 16 * o;
                 if (j >= i) {
-                    const double val = (e < 0) ? z[o] : z[o] - zp[o];
+                    const double val = z[o] - zp[o];
                     Q[(size_t)i * Np + j] = val;
                     Q[(size_t)j * Np + i] = val;
                 }
             }
         }
-        if (e >= 0) {
 #pragma unroll
-            for (int o = 0; o < NO; ++o) zp[o] = z[o];
-        }
+        for (int o = 0; o < NO; ++o) zp[o] = z[o];
     }
 }
 
@@ -421,10 +394,13 @@ __global__ __launch_bounds__(256) void k_rm_bands(const ChunkDev *cs, const RmBa
 // operand of S^T += R_J T^T.  A quarter evaluates 31 ros + rnb points a side, 1.7
 // times its own.  u and sqrt(lambda), in units of the table's steps, are formed
 // once per point, so that v and z are a difference and a product.  Bound by the
-// gathers of the table, two 16-byte rows a point.  160 chunks of 100 to 1200
-// pixels oversampled three times: 12.7 -> 1.7 ms (as the first pass of
-// k_rm_sandwich, whose registers leave two waves per SIMD to hide them), error
-// against extended precision 4e-14 -> 1.3e-15 of S's peak.
+// gathers of the table, two 16-byte rows a point.  160 chunks of 100 to 1200 pixels
+// oversampled three times: 12.7 -> 1.7 ms (as a pass of k_rm_sandwich, whose
+// registers leave two waves per SIMD to hide them), error against extended
+// precision 4e-14 -> 1.3e-15 of S's peak.  More than 57 taps a row take over 64 KB
+// of LDS, one workgroup a CU from 81 KB on, and are faster all the same: 64 chunks
+// of 480 to 600 pixels with 81 taps, S and Q_k together 25.9 -> 3.2 ms (6.2 with
+// S by the sandwich).
 __global__ __launch_bounds__(256) void k_rm_signal(const ChunkDev *cs, const double *rin, const TableDev *tabs,
                                                    BinsDev bins, double *mat) {
     typedef const double __attribute__((ext_vector_type(2), aligned(8), address_space(1))) GlobalD2u;
@@ -514,6 +490,7 @@ __global__ __launch_bounds__(256) void k_rm_signal(const ChunkDev *cs, const dou
 }
 
 size_t rmat_signal_lds(int os, int nb) {
+    // at most 90 KB under 15 os + nb <= RM_ROWS (81 taps), of a CU's 160
     return 8 * (4 * ((size_t)(TILE - 1) * os + nb + 16) + 2 * TILE * signal_pitch(os, nb));
 }
 
@@ -555,21 +532,17 @@ bool rmat_layout_ok(const RmLayout &lay) {
 bool launch_rmat(const LaunchCtx &L) {
     if (L.rm_kbu < 0) return true;
     const RmLayout &lay = L.rm_lay;
-    const int nt = L.np_max / TILE, signal = L.rm_sig_lds == 0;   // S with the edges' kernel
-    if (!signal)
-        k_rm_signal<<<dim3(nt * (nt + 1) / 2, L.nchunks), 256, L.rm_sig_lds, L.stream>>>(L.chunks, L.rin, L.tables,
-                                                                                         L.bins, L.mat);
-    if (signal || L.rm_edges) {
+    const int nt = L.np_max / TILE;
+    k_rm_signal<<<dim3(nt * (nt + 1) / 2, L.nchunks), 256, L.rm_sig_lds, L.stream>>>(L.chunks, L.rin, L.tables, L.bins,
+                                                                                     L.mat);
+    if (L.rm_edges) {
         const dim3 g(L.np_max / lay.tj, L.np_max / 16, L.nchunks);
         if (lay.tj == 32 && lay.em == 10 && lay.npass <= 4)
-            k_rm_sandwich<32, 10, 4><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.tables, L.bins, lay, signal,
-                                                                      L.mat);
+            k_rm_sandwich<32, 10, 4><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.bins, lay, L.mat);
         else if (lay.tj == 16 && lay.em == 10 && lay.npass <= 3)
-            k_rm_sandwich<16, 10, 3><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.tables, L.bins, lay, signal,
-                                                                      L.mat);
+            k_rm_sandwich<16, 10, 3><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.bins, lay, L.mat);
         else if (lay.tj == 16 && lay.em == RM_ROWS / 8 && lay.npass <= 3)
-            k_rm_sandwich<16, RM_ROWS / 8, 3><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.tables, L.bins, lay,
-                                                                               signal, L.mat);
+            k_rm_sandwich<16, RM_ROWS / 8, 3><<<g, 256, lay.bytes, L.stream>>>(L.chunks, L.rin, L.bins, lay, L.mat);
         else
             return false;
     }

@@ -75,7 +75,7 @@ struct Batch {
     int rm_kbu = -1;   // resolution-matrix chunks: largest KBIN_UPP
     RmLayout rm_lay;   // and the LDS layout of their sandwich launch
     int rm_edges = 0;         // whether one of them takes its Q_k from the band edges
-    size_t rm_sig_lds = 0;    // LDS of the signal launch, 0 if it is too large
+    size_t rm_sig_lds = 0;    // LDS of the signal launch
     int rm_groups = 0;        // quadrature: most band groups
     size_t rm_lds = 0;        // and the LDS of the node launch
     hipEvent_t evA[7]{};   // stage A (assembly .. solves) on stream st
@@ -912,7 +912,6 @@ int plan_batches(qml_ctx *c) {
         }
         xg.flush(wg);
         if (B.rm_kbu >= 0) {
-            if (B.rm_sig_lds > 65536) B.rm_sig_lds = 0;   // rows of more than about 55 taps
             // 16 x 32 output tiles where their LDS fits in 64 KB, their a range
             // in 80 rows and their b range in 4 passes; else 16 x 16 (which
             // always fits under the registration limit on 15 ros + rnb)

@@ -47,7 +47,7 @@ struct LaunchCtx {
     int rm_kbu;               // largest KBIN_UPP of the batch's resolution-matrix chunks; -1 if none
     RmLayout rm_lay;          // LDS layout of the batch's sandwich launch
     int rm_edges;             // whether one of them has its Q_k by the band edges
-    size_t rm_sig_lds;        // LDS of the signal launch, 0 if it is too large for it
+    size_t rm_sig_lds;        // LDS of the batch's signal launch
     int rm_groups;            // most band groups of a chunk in the batch
     size_t rm_lds;            // LDS of the batch's node launch
     const RmBand *rm_bands;

@@ -61,3 +61,36 @@ def test_band_matrices_of_few_taps(bins, n, shape):
             assert np.max(np.abs(got - want)) < 1e-11 * np.max(np.abs(want)), kn
     finally:
         eng.close()
+
+
+LONG = [("dia", 1, 11), ("dia", 1, 57), ("dia", 1, 59), ("dia", 1, 81), ("oversampled", 2, 65), ("oversampled", 3, 51),
+        ("oversampled", 5, 21)]
+
+
+@pytest.mark.parametrize("n", [64, 130])
+def test_signal_of_long_rows(n):
+    """R rows up to the most taps that are taken, in one batch: S against the
+    oracle's extended-precision run (the bar of the rounding of v), and each
+    chunk's S, F and d, b, t the same, bit for bit, alone and with the others."""
+    print(f"[case] long rows {n}", flush=True)
+    w = _workload((6, 0.004), n, LONG)
+    T = w.binning.total_kz_bins
+
+    def run(chunks):
+        eng = QMLEngine(w.binning, precision="fp64")
+        got = synth.load_engine(eng, w, chunks)
+        eng.commit()
+        eng.iterate(np.full(T, 0.1), np.zeros((T, T)), np.zeros((3, T)))
+        res = {i: (*eng.chunk_result(cid)[:2], eng.chunk_matrix(cid, qml.CMAT_SFID)) for i, cid in got}
+        eng.close()
+        return res
+
+    together = run(list(range(len(LONG))))
+    assert len(together) == len(LONG)
+    for i, c in enumerate(w.chunks):
+        ch = _oracle(w, c)
+        want, got = ch.signal_matrix(*ch.vz_matrices()), together[i][2]
+        assert np.array_equal(got, got.T)
+        assert np.max(np.abs(got - want)) < 1e-11 * np.max(np.abs(want)), LONG[i]
+        for a, b in zip(together[i], run([i])[i]):
+            assert np.array_equal(a, b), LONG[i]
