@@ -213,15 +213,16 @@ __global__ __launch_bounds__(256) void k_gemm(const ChunkDev *cs, const Work *wo
     }
 }
 
+// offdiag: whether Gram items lie off the diagonal (more than 128 members)
 void launch_bf3(hipStream_t st, int mode, int nprod, int nst, const ChunkDev *chunks, const Work *work, int nwork,
-                const void *A, const void *B, void *C, int jlo);
+                const void *A, const void *B, void *C, int jlo, bool offdiag);
 
 template <int MODE>
 static void launch_mode(hipStream_t st, int prec, int nst, const ChunkDev *chunks, const Work *work, int nwork,
-                        const void *A, const void *B, void *C, int jlo) {
+                        const void *A, const void *B, void *C, int jlo, bool offdiag = false) {
     if (nwork <= 0) return;
     if (prec >= 2) {   // split BF16: three products, or four with lo * lo
-        launch_bf3(st, MODE, prec == 3 ? 4 : 3, nst, chunks, work, nwork, A, B, C, jlo);
+        launch_bf3(st, MODE, prec == 3 ? 4 : 3, nst, chunks, work, nwork, A, B, C, jlo, offdiag);
         return;
     }
     const int grid = 8 * ((nwork + 7) / 8);
@@ -250,7 +251,7 @@ void launch_gemm_gram(hipStream_t st, int prec, int nst, const ChunkDev *chunks,
         if (nwork > 0) launch_gram64(st, chunks, work, nwork, (const double *)G, gram);
         return;
     }
-    launch_mode<MODE_GRAM>(st, prec, nst, chunks, work, nwork, G, G, gram, offdiag);   // jlo is not the Gram's
+    launch_mode<MODE_GRAM>(st, prec, nst, chunks, work, nwork, G, G, gram, 0, offdiag);
 }
 
 }  // namespace qml
@@ -957,7 +958,7 @@ __global__ __launch_bounds__(256, 3) void k_gram_bf3(const ChunkDev *cs, const W
 
 template <int NPROD>
 static void launch_bf3_np(hipStream_t st, int mode, int nst, const ChunkDev *chunks, const Work *work, int nwork,
-                          const __bf16 *a, const __bf16 *b, void *C, int jlo) {
+                          const __bf16 *a, const __bf16 *b, void *C, int jlo, bool offdiag) {
     const int grid = 8 * ((nwork + 7) / 8);
     // nst, the staging of the operands: 1 one LDS stage (three workgroups
     // per CU, the next stage in registers); 2 two LDS stages (two workgroups
@@ -980,7 +981,7 @@ static void launch_bf3_np(hipStream_t st, int mode, int nst, const ChunkDev *chu
         else QML_BF3_LAUNCH(MODE_RIGHT, 1);
     } else {
         if (nst == 4) QML_BF3D_LAUNCH(MODE_GRAM, 3, 3);
-        else if (nst == 3 && !jlo) k_gram_bf3<NPROD><<<grid, 256, 0, st>>>(chunks, work, nwork, a, (double *)C);
+        else if (nst == 3 && !offdiag) k_gram_bf3<NPROD><<<grid, 256, 0, st>>>(chunks, work, nwork, a, (double *)C);
         else if (nst == 3) QML_BF3D_LAUNCH(MODE_GRAM, 2, 2);
         else if (nst == 1) QML_BF3_LAUNCH(MODE_GRAM, 1);
         else QML_BF3_LAUNCH(MODE_GRAM, 2);
@@ -990,13 +991,13 @@ static void launch_bf3_np(hipStream_t st, int mode, int nst, const ChunkDev *chu
 }
 
 void launch_bf3(hipStream_t st, int mode, int nprod, int nst, const ChunkDev *chunks, const Work *work, int nwork,
-                const void *A, const void *B, void *C, int jlo) {
+                const void *A, const void *B, void *C, int jlo, bool offdiag) {
     if (nwork <= 0) return;
     const __bf16 *a = (const __bf16 *)A, *b = (const __bf16 *)B;
     if (nprod == 4)
-        launch_bf3_np<4>(st, mode, nst, chunks, work, nwork, a, b, C, jlo);
+        launch_bf3_np<4>(st, mode, nst, chunks, work, nwork, a, b, C, jlo, offdiag);
     else
-        launch_bf3_np<3>(st, mode, nst, chunks, work, nwork, a, b, C, jlo);
+        launch_bf3_np<3>(st, mode, nst, chunks, work, nwork, a, b, C, jlo, offdiag);
 }
 
 }  // namespace qml
