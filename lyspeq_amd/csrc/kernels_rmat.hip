@@ -57,6 +57,9 @@
 #include "qml_common.hpp"
 #include "qml_kernels.hpp"
 
+#include <algorithm>
+#include <cmath>
+
 namespace qml {
 
 namespace {
@@ -501,12 +504,18 @@ size_t rmat_node_lds(int os, int nb) {
 
 int rmat_nodes(double dk, double vmax) {
     // n nodes integrate cos(x t) over [-1, 1] to 1e-17 up to x = 2 (n - 8.75 n^(1/3) + 9.6)
-    // (found from n = 8 to 256); beyond 256 nodes the edges cost no more
-    const double x = 0.5 * dk * vmax;
+    // (found from n = 8 to 256); beyond 256 nodes the edges cost no more.  The
+    // limits are formed once: a plan asks for every band of every chunk
+    struct Limits {
+        double x[32];
+        Limits() {
+            for (int k = 0; k < 32; ++k) x[k] = 2.0 * (8.0 * (k + 1) - 8.75 * std::cbrt(8.0 * (k + 1)) + 9.6);
+        }
+    };
+    static const Limits lim;
     if (!(dk > 0 && vmax >= 0)) return 0;
-    for (int n = 8; n <= 256; n += 8)
-        if (x <= 2.0 * (n - 8.75 * std::cbrt((double)n) + 9.6)) return n;
-    return 0;
+    const int k = (int)(std::lower_bound(lim.x, lim.x + 32, 0.5 * dk * vmax) - lim.x);
+    return k < 32 ? 8 * (k + 1) : 0;
 }
 
 RmLayout rmat_layout(int tj, int ra_max, int rb_max, int nb_max) {

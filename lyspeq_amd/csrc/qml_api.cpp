@@ -206,7 +206,7 @@ struct qml_ctx {
     double *d_theta = nullptr, *d_F = nullptr, *d_dbtsum = nullptr;
     double *d_rin = nullptr;   // resolution-matrix rows and fine grids
     RmBand *d_rmb = nullptr;   // their bands' quadrature in k
-    RmNode *d_rmn = nullptr;
+    const RmNode *d_rmn = nullptr;   // in d_rmb's allocation
     std::vector<Batch> batches;
     hipEvent_t ev_begin{}, ev_end{}, ev_acc{};
     hipEvent_t ev_fork{}, ev_join{};   // order stage B's stream inside one iteration
@@ -286,7 +286,7 @@ int qml_destroy(qml_ctx *c) {
     for (auto &t : c->tables) { hipFree(t.d_qt); hipFree(t.d_q2); hipFree(t.d_s); }
     release_plan(c);
     void *ptrs[] = {c->d_tables, c->d_in, c->d_outs, c->d_fc, c->d_dbt, c->d_status, c->d_skip,
-                    c->d_theta, c->d_F, c->d_dbtsum, c->d_rin, c->d_rmb, c->d_rmn};
+                    c->d_theta, c->d_F, c->d_dbtsum, c->d_rin, c->d_rmb};
     for (void *p : ptrs) if (p) hipFree(p);
     if (c->ev_begin) hipEventDestroy(c->ev_begin);
     if (c->ev_end) hipEventDestroy(c->ev_end);
@@ -699,7 +699,8 @@ void gauss_legendre(int n, std::vector<long double> &x, std::vector<long double>
 int plan_quadrature(qml_ctx *c) {
     std::vector<RmBand> bands;
     std::vector<RmNode> nodes;
-    std::map<std::pair<int, int>, int> at;   // (band, n) -> nodes
+    constexpr int RULES = 33;   // node counts 0, 8 .. 256
+    std::vector<int> at(c->kedges.size() * RULES, -1);   // (band, n / 8) -> nodes
     std::map<int, std::pair<std::vector<long double>, std::vector<long double>>> rule;
     for (auto &ch : c->chunks) {
         ch.ngrp = 0;
@@ -721,9 +722,12 @@ int plan_quadrature(qml_ctx *c) {
         }
         if ((int)bs.size() < ch.kbu) continue;
         for (int k = 0; k < ch.kbu; ++k) {
-            const auto f = at.emplace(std::make_pair(k, bs[k].n), (int)nodes.size());
-            bs[k].node = f.first->second;
-            if (!f.second) continue;
+            int &place = at[k * RULES + bs[k].n / 8];
+            if (place >= 0) {
+                bs[k].node = place;
+                continue;
+            }
+            bs[k].node = place = (int)nodes.size();
             auto &r = rule[bs[k].n];
             if (r.first.empty()) gauss_legendre(bs[k].n, r.first, r.second);
             const long double k0 = c->kedges[k], k1 = c->kedges[k + 1];
@@ -741,10 +745,14 @@ int plan_quadrature(qml_ctx *c) {
         bands.insert(bands.end(), bs.begin(), bs.end());
     }
     if (bands.empty()) return QML_OK;
-    HIPCHK(hipMalloc(&c->d_rmb, bands.size() * sizeof(RmBand)));
-    HIPCHK(hipMemcpy(c->d_rmb, bands.data(), bands.size() * sizeof(RmBand), hipMemcpyHostToDevice));
-    HIPCHK(hipMalloc(&c->d_rmn, nodes.size() * sizeof(RmNode)));
-    HIPCHK(hipMemcpy(c->d_rmn, nodes.data(), nodes.size() * sizeof(RmNode), hipMemcpyHostToDevice));
+    // one allocation and one copy: the bands, then the nodes
+    const size_t nb = align_up(bands.size() * sizeof(RmBand), 256), nn = nodes.size() * sizeof(RmNode);
+    std::vector<char> both(nb + nn);
+    std::memcpy(both.data(), bands.data(), bands.size() * sizeof(RmBand));
+    std::memcpy(both.data() + nb, nodes.data(), nn);
+    HIPCHK(hipMalloc(&c->d_rmb, both.size()));
+    HIPCHK(hipMemcpy(c->d_rmb, both.data(), both.size(), hipMemcpyHostToDevice));
+    c->d_rmn = (const RmNode *)((const char *)c->d_rmb + nb);
     return QML_OK;
 }
 
@@ -874,12 +882,13 @@ int plan_batches(qml_ctx *c) {
         if (c->d_G) HIPCHK(hipMemset(c->d_G, 0xff, std::max<size_t>(mx.g, 1) * es));
     }
 
+    std::vector<Work> wl, wr, wg;   // these keep their memory from batch to batch
+    XcdLists xl, xr, xg;
     for (size_t bi = 0; bi < groups.size(); ++bi) {
         Batch B;
         B.ids = groups[bi];
         const auto &cd = devs[bi];
-        std::vector<Work> wl, wr, wg;
-        XcdLists xl, xr, xg;
+        for (auto *w : {&wl, &wr, &wg}) w->clear();
         int ra_max = 0, rb_max = 0, nb_max = 0;
         for (int li = 0; li < (int)cd.size(); ++li) {
             const ChunkDev &d = cd[li];
