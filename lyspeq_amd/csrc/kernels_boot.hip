@@ -658,10 +658,11 @@ __device__ bool count_median(const double *a, const double *b, int n, SelectLds 
 #pragma unroll
         for (int k = 0; k < R; ++k) t = v[k] >= pl ? fmin(t, v[k]) : t;
         for (int d = 1; d < 64; d *= 2) t = fmin(t, __shfl_xor(t, d, 64));
-        if (lane == 0) s.wave_min[wave] = (unsigned long long)__double_as_longlong(t);
+        // past total's places: a wave may still be reading the NaN flags in wave_min
+        double *mins = reinterpret_cast<double *>(s.hist + 8);
+        if (lane == 0) mins[wave] = t;
         __syncthreads();
-        t = fmin(fmin(__longlong_as_double((long long)s.wave_min[0]), __longlong_as_double((long long)s.wave_min[1])),
-                 fmin(__longlong_as_double((long long)s.wave_min[2]), __longlong_as_double((long long)s.wave_min[3])));
+        t = fmin(fmin(mins[0], mins[1]), fmin(mins[2], mins[3]));
         t = lane_value(t, 0);   // uniform, and so the next pivots
         if (!(t < __builtin_inf())) return 2;
         int c = 0, z = 0;
