@@ -194,26 +194,51 @@ def copy_calibration(mb: int):
 TRAFFIC_DIR = os.path.join(ROOT, "profiles")
 
 
-def measured_traffic(kernel: str, precision: str, workload: str):
+def product_kernel(kernel: str, precision: str, schedule: dict) -> str:
+    """The kernels that a dense product launches, as the profiler names them
+    (launch_gemm_whiten_left, _right and launch_gemm_gram): counters recorded of
+    other kernels say nothing about this run."""
+    if precision == "fp64":
+        return {"whiten_left": "k_gemm64<false>", "whiten_right": "k_gemm64<true>", "gram": "k_gram64"}[kernel]
+    mode = {"whiten_left": 0, "whiten_right": 1, "gram": 2}[kernel]
+    if precision == "fp32":
+        return f"k_gemm<{mode}>"
+    nprod = 4 if precision == "bf16x4" else 3
+    stages = schedule[{"whiten_left": "stages_left", "whiten_right": "stages_right", "gram": "stages_gram"}[kernel]]
+    if stages == 4:
+        return f"k_gemm_bf3d<{mode}, 3, 3, {nprod}>"
+    if stages == 3:
+        if kernel == "gram":    # by batch: over 128 members, and up to 128
+            return f"k_gemm_bf3d<2, 2, 2, {nprod}>, k_gram_bf3<{nprod}>"
+        return f"k_gemm_bf3d<{mode}, 3, 2, {nprod}>"
+    return f"k_gemm_bf3<{mode}, {stages}, {nprod}>"
+
+
+def measured_traffic(kernel: str, precision: str, workload: str, name: str):
     """HBM bytes per launch of the dominant kernel from the committed PMC
     summary (profiles/traffic_<kernel>_<precision>_<workload>.json), if one
-    was recorded for this configuration."""
+    was recorded for this configuration with the kernels of this name."""
     path = os.path.join(TRAFFIC_DIR, f"traffic_{kernel}_{precision}_{workload}.json")
     if not os.path.exists(path):
         return None, None
     with open(path) as f:
         t = json.load(f)
+    if t.get("kernel_name") != name:
+        return None, None
     return float(t["hbm_bytes_per_launch"]), os.path.relpath(path, ROOT)
 
 
-def measured_mfma_busy(kernel: str, precision: str):
+def measured_mfma_busy(kernel: str, precision: str, name: str):
     """MFMA-busy fraction of a dense product from the committed counter
-    summary (profiles/mfma_util_products_desi-4096.json), if recorded."""
+    summary (profiles/mfma_util_products_desi-4096.json), if recorded with the
+    kernels of this name."""
     path = os.path.join(TRAFFIC_DIR, "mfma_util_products_desi-4096.json")
     if not os.path.exists(path):
         return None, None
     with open(path) as f:
         t = json.load(f)
+    if t.get("kernel_name", {}).get(precision, {}).get(kernel) != name:
+        return None, None
     v = t.get("mfma_busy", {}).get(precision, {}).get(kernel)
     return v, (os.path.relpath(path, ROOT) if v is not None else None)
 
@@ -481,19 +506,20 @@ def main():
     work = kernel_work(resm["shapes"], args.precision)
     if dom in ("whiten_left", "whiten_right", "gram"):
         ach = work[dom] / (km[dom] / 1e3)
-        traffic, tsrc = measured_traffic(dom, args.precision, w.name) if not args.nchunks else (None, None)
+        name = product_kernel(dom, args.precision, resm["schedule"])
+        traffic, tsrc = measured_traffic(dom, args.precision, w.name, name) if not args.nchunks else (None, None)
         roof = {"kernel": dom, "bound": "mfma", "achieved": ach / 1e12, "peak": PEAK[args.precision] / 1e12,
                 "unit": "TFLOP/s", "frac": ach / PEAK[args.precision], "traffic": traffic,
                 "launches": nb, "avg_launch_ms": km[dom] / nb}
-        busy, bsrc = measured_mfma_busy(dom, args.precision)
+        busy, bsrc = measured_mfma_busy(dom, args.precision, name)
         if bsrc:
             # issued MFMA-pipe occupancy from counters (three MFMAs per split product)
             roof["mfma_busy_issued"] = busy
             roof["mfma_busy_source"] = bsrc
         if tsrc:
             roof["traffic_source"] = tsrc
-            # the same launches against the HBM roof: at split-BF16 operand
-            # planes (4 bytes per element) the whitening products are close to it
+            # the same launches against the HBM roof: the split-BF16 operand
+            # planes have 4 bytes per element
             roof["hbm_achieved_GBps"] = traffic / (roof["avg_launch_ms"] / 1e3) / 1e9
             roof["hbm_frac"] = roof["hbm_achieved_GBps"] * 1e9 / HBM_PEAK
     else:
