@@ -228,11 +228,11 @@ def measured_traffic(kernel: str, precision: str, workload: str, name: str):
     return float(t["hbm_bytes_per_launch"]), os.path.relpath(path, ROOT)
 
 
-def measured_mfma_busy(kernel: str, precision: str, name: str):
-    """MFMA-busy fraction of a dense product from the committed counter
-    summary (profiles/mfma_util_products_desi-4096.json), if recorded with the
-    kernels of this name."""
-    path = os.path.join(TRAFFIC_DIR, "mfma_util_products_desi-4096.json")
+def measured_mfma_busy(kernel: str, precision: str, workload: str, name: str):
+    """MFMA-busy fraction of a dense product from the committed counter summary
+    (profiles/mfma_util_products_<workload>.json), if recorded for this workload
+    with the kernels of this name."""
+    path = os.path.join(TRAFFIC_DIR, f"mfma_util_products_{workload}.json")
     if not os.path.exists(path):
         return None, None
     with open(path) as f:
@@ -511,7 +511,7 @@ def main():
         roof = {"kernel": dom, "bound": "mfma", "achieved": ach / 1e12, "peak": PEAK[args.precision] / 1e12,
                 "unit": "TFLOP/s", "frac": ach / PEAK[args.precision], "traffic": traffic,
                 "launches": nb, "avg_launch_ms": km[dom] / nb}
-        busy, bsrc = measured_mfma_busy(dom, args.precision, name)
+        busy, bsrc = measured_mfma_busy(dom, args.precision, w.name, name) if not args.nchunks else (None, None)
         if bsrc:
             # issued MFMA-pipe occupancy from counters (three MFMAs per split product)
             roof["mfma_busy_issued"] = busy
