@@ -465,8 +465,8 @@ void launch_bootstrap(hipStream_t st, const ChunkOut *outs, const double *dbt, c
 // copies are counted: a median with many equal values ends there.  The values are
 // read once; the radix select below reads them three times and its waves queue on
 // the few histogram bins that hold a band pair's exponents.  Bound by the barriers
-// and compares of the counts.  Whole calls with the copies: 455 bands x 8000
-// realisations 5.7 -> 3.3 ms, x 500 1.29 -> 1.04; 200 bands of whole numbers x 8000
+// and compares of the counts.  455 bands x 8000 realisations: 4.65 -> 2.31 ms for
+// the 103740 pairs.  Whole calls with the copies: 5.7 -> 3.3 ms, x 500 1.29 -> 1.04; 200 bands of whole numbers x 8000
 // 2.3 -> 0.89, x 500 0.38 -> 0.23 (2.7 and 0.65 where counting gave up on equal
 // values and the radix select followed).
 //

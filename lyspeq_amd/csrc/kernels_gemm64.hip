@@ -180,7 +180,7 @@ __global__ __launch_bounds__(256, 4) void k_gemm64(const ChunkDev *cs, const Wor
 // flight while this one is multiplied (32 terms a step where I = J, whose steps
 // are short, 8 else).  The partial sums of the waves meet in LDS, block by
 // block.  (64 x 64 tiles of padded members took 537 us for 64 chunks with
-// m = 21, this 134 us; the survey sample with m up to 175 took 8.9 ms, now 6.9.)
+// m = 21, this 134 us; the survey sample with m up to 175 took 8.9 ms, now 5.8.)
 constexpr int GW = 8;   // waves
 __global__ __launch_bounds__(64 * GW, 2) void k_gram64(const ChunkDev *cs, const Work *work, int nwork, const double *G,
                                                     double *gram) {
