@@ -470,8 +470,8 @@ void launch_bootstrap(hipStream_t st, const ChunkOut *outs, const double *dbt, c
 // 2.3 -> 0.89, x 500 0.38 -> 0.23 (2.7 and 0.65 where counting gave up on equal
 // values and the radix select followed).
 //
-// Longer columns (more than 8192 values), NaNs, and brackets with an end at
-// infinity or whose copies part the two ranks of an even count take a radix
+// Few bands, longer columns (more than 8192 values), NaNs, and brackets with an
+// end at infinity or whose copies part the two ranks of an even count take a radix
 // select over order-preserving 64-bit keys of the FP64 values: eight passes of 8
 // bits, most significant first, each a 256-bin LDS histogram of the values
 // still matching the selected prefix and a block scan that picks the digit
@@ -888,8 +888,13 @@ void launch_boot_median(hipStream_t st, const double *R, int nboots, int T, doub
     // 1.04 ms with 2, 1.13 with 8 (radix select 1.29), 2048 1.50 with 8 (2.0), 8000
     // 3.3 with 32 (5.7).  With 80, two waves run on a SIMD and the counts' masks
     // spill: 8193 5.9 -> 8.0, 20000 13.9 -> 16.6, so longer columns take the radix
-    // select (12.7 at 20000).
-    if (nboots <= 256 * 2)
+    // select (12.7 at 20000).  Where the pairs fit the chip at once (256 CUs, four
+    // workgroups each), a pair's own latency counts, and the radix select's is the
+    // shorter: 32 bands, 500 realisations 91 us (97 by counting), 8000 243 (253); 64
+    // bands 111 (112) and 386 (351).
+    if (T * (T + 1LL) / 2 <= 1024)
+        launch_medians<0>(st, nboots, T, X, median, mad);
+    else if (nboots <= 256 * 2)
         launch_medians<2>(st, nboots, T, X, median, mad);
     else if (nboots <= 256 * 8)
         launch_medians<8>(st, nboots, T, X, median, mad);
